@@ -1713,17 +1713,36 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
     sum = sum >= 2.0 * q ? sum - 2.0 * q : sum;
     return sum >= q ? sum - q : sum;
   };
+  // floor(X / P) mod q plus the base on a row whose prime is at or above the
+  // binary64 limit 2^42: (X_P R) mod q by the reference basis-extension
+  // formula, then ((x R) - (X_P R)) * P^{-1} with REDC = (x - X_P) P^{-1} mod q.
+  auto moddown_integer = [&](int64_t grow, int64_t xval, int64_t bval) -> int64_t {
+    const Mont m = load_mont(a.params, grow);
+    int64_t xp = mont_mul(dg[0], m.r2, m);
+#pragma unroll
+    for (int r = 1; r < P; ++r)
+      xp = add_lazy(xp, mont_mul(dg[r], global(a.pdig.basis)[(r - 1) * a.pdig.basis_stride + grow], m), m.twice_q);
+    const int64_t xr = mont_mul(xval, m.r2, m);
+    return with_base(bval, mont_mul(sub_lazy(xr, xp, m.twice_q), a.p_inverse[grow], m), m.twice_q);
+  };
   // Fused rescale: every thread needs the final row-0 value of its
-  // coefficient (row 0 is a binary64 row: the dropped prime is a scale prime).
+  // coefficient.  Row 0 is a binary64 row, or, when the scale primes are at
+  // or above 2^42, an integer row as every other row then is.
   const bool rescale = a.rescale_inv != nullptr;
   double c0 = 0.0;
-  double round_up = 0.0;
+  int64_t c0_int = 0;
+  int64_t round_up = 0;
   if (rescale) {
     Global<double>* rec0 = global(a.pdig.f64_table) + a.level * pitch;
     const int64_t x0 = row_begin == 0 ? xv[0] : acc_row(0);
     const int64_t b0 = row_begin == 0 ? bv[0] : (has_base ? base.at(b, 0, i) : 0);
-    c0 = add_base_f64(moddown_f64(rec0, x0), b0, rec0[14]);
-    round_up = c0 > static_cast<double>(a.half_drop) ? 1.0 : 0.0;
+    if (rec0[14] != 0.0) {
+      c0 = add_base_f64(moddown_f64(rec0, x0), b0, rec0[14]);
+      c0_int = static_cast<int64_t>(f64_to_u64(c0));
+    } else {
+      c0_int = moddown_integer(a.level, x0, b0);
+    }
+    round_up = c0_int > a.half_drop ? 1 : 0;
   }
 #pragma unroll
   for (int rr = 0; rr < kRows; ++rr) {
@@ -1738,26 +1757,19 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
       if (rescale && row > 0) {
         // ((v - c0) q0^{-1} + round_up) mod q, |v - c0| < 2^47 exact
         double r = f64_mulmod_signed(static_cast<double>(a.rescale_inv[row - 1]), v - c0, q, rec[15]);
-        r += round_up;
+        r += static_cast<double>(round_up);
         v = r < 0.0 ? r + q : (r >= q ? r - q : r);
       }
       value = static_cast<int64_t>(f64_to_u64(v));
     } else {
-      // A prime at or above the binary64 limit 2^42 (the base prime): the
-      // integer formula.
-      const Mont m = load_mont(a.params, grow);
-      // (X_P R) mod q by the reference basis-extension formula, then
-      // ((x R) - (X_P R)) * P^{-1} with REDC = (x - X_P) P^{-1} mod q.
-      int64_t xp = mont_mul(dg[0], m.r2, m);
-#pragma unroll
-      for (int r = 1; r < P; ++r)
-        xp = add_lazy(xp, mont_mul(dg[r], global(a.pdig.basis)[(r - 1) * a.pdig.basis_stride + grow], m),
-                      m.twice_q);
-      const int64_t xr = mont_mul(xv[rr], m.r2, m);
-      value = with_base(bv[rr], mont_mul(sub_lazy(xr, xp, m.twice_q), a.p_inverse[grow], m), m.twice_q);
+      value = moddown_integer(grow, xv[rr], bv[rr]);
       if (rescale && row > 0) {
-        const uint64_t qq = m.q;
-        int64_t d = value - static_cast<int64_t>(c0);
+        // the dropped prime may exceed this one: c0 mod q first (c0 >= q is
+        // rare, so the division hardly ever runs)
+        const uint64_t qq = a.rows[grow].q;
+        uint64_t c0_q = static_cast<uint64_t>(c0_int);
+        if (c0_q >= qq) c0_q %= qq;
+        int64_t d = value - static_cast<int64_t>(c0_q);
         if (d < 0) d += static_cast<int64_t>(qq);
         uint64_t r = shoup_mulmod(static_cast<uint64_t>(a.rescale_inv[row - 1]),
                                   static_cast<uint64_t>(a.rescale_inv_shoup[row - 1]), static_cast<uint64_t>(d), qq);

@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 import torch
 
+from fhelium_amd.config import CkksConfig
 from fhelium_amd.engine import CkksEngine
 from tests import helpers as H
 
@@ -98,3 +99,20 @@ def test_seeded_keyswitch_matches_bases(eng, level, rescale):
     # plain residues are not seeds, and seeds carry their level
     with pytest.raises(TypeError):
         ks.key_switch_fused(d2, key, level, rescale=rescale, seeds=d[:2])
+
+
+@pytest.mark.parametrize("preset,level", [("slots8192-scale50-levels5-int64", 0),
+                                          ("slots16384-scale50-levels12-int64", 3),
+                                          ("slots32768-scale50-levels27-int64", 25)])
+def test_fused_rescale_by_a_50_bit_prime(preset, level):
+    """The dropped prime of a 50-bit parameter set is no binary64 row: the
+    fused product still equals the method composition."""
+
+    e = CkksEngine(CkksConfig.from_preset(preset).with_ring_log(12), rng_seed=7)
+    rng = np.random.default_rng(level)
+    x = rng.uniform(-1, 1, (2, e.config.slots))
+    y = rng.uniform(-1, 1, (2, e.config.slots))
+    a, b = e.encrypt(x, level=level), e.encrypt(y, level=level)
+    fused = e.hmult(a, b)
+    assert torch.equal(fused.data, e.rescale_to_next_level(e.relinearize(composed(e, a, b))).data)
+    assert np.abs(e.decrypt(fused).real - x * y).max() < 2e-5
