@@ -177,6 +177,18 @@ __device__ __forceinline__ int64_t canonical_operand(int64_t v, uint64_t q) {
   return r;
 }
 
+// canonical_operand with 1/q at hand (|v / q| < 2^51): a binary64
+// multiplication in place of the division, the same corrections.
+__device__ __forceinline__ int64_t canonical_operand(int64_t v, uint64_t q, double qinv) {
+  const int64_t qs = static_cast<int64_t>(q);
+  const double est = __builtin_floor(static_cast<double>(v) * qinv);
+  int64_t r = static_cast<int64_t>(static_cast<uint64_t>(v) -
+                                   static_cast<uint64_t>(static_cast<int64_t>(est)) * q);
+  r = r < 0 ? r + qs : r;
+  r = r >= qs ? r - qs : r;
+  return r;
+}
+
 __device__ __forceinline__ int64_t mont_mul_split(int64_t a, int64_t b,
                                                   const Mont& m) {
   return mont_mul(canonical_operand(a, m.q), canonical_operand(b, m.q), m);
@@ -241,6 +253,42 @@ __device__ __forceinline__ double f64_mulmod_signed(double w, double x, double q
   const double l = __builtin_fma(w, x, -h);
   const double t = __builtin_fma(h, qinv, kRoundMagic) - kRoundMagic;
   return __builtin_fma(-t, q, h) + l;
+}
+
+// Exact sum of products w_i x_i of integers held in binary64, reduced modulo
+// q once at the end: 4 operations per product (3 for the first) and 5 for the
+// reduction, where a product reduced by itself and added costs 7.
+// `hi` starts at 1.5 2^52 g for a power of two g, so every fma below rounds
+// the running sum to a multiple of g; the step it took (d) is exact, and
+// w x - d is an integer of magnitude at most g / 2, which `lo` collects
+// exactly.  Conditions: |sum| < 2^51 g (f64_sum_start picks g from a bound on
+// the sum), terms * g / 2 < 2^53 and |sum| / q < 2^51.  The reduced value is
+// within q (1/2 + |sum| / q 2^-52) + terms g / 2 of zero.
+struct F64Sum {
+  double hi, lo;
+};
+
+// 1.5 2^(e+2) for 2^e <= bound < 2^(e+1): g = 2^(e-50), 2^51 g > bound.
+__device__ __forceinline__ double f64_sum_start(double bound) {
+  const uint64_t bits = static_cast<uint64_t>(__double_as_longlong(bound));
+  return __longlong_as_double(static_cast<int64_t>((bits & 0x7ff0000000000000ull) + 0x0028000000000000ull));
+}
+
+__device__ __forceinline__ void f64_sum_first(F64Sum& s, double start, double w, double x) {
+  s.hi = __builtin_fma(w, x, start);
+  s.lo = __builtin_fma(w, x, start - s.hi);
+}
+
+__device__ __forceinline__ void f64_sum_add(F64Sum& s, double w, double x) {
+  const double h = __builtin_fma(w, x, s.hi);
+  s.lo += __builtin_fma(w, x, s.hi - h);
+  s.hi = h;
+}
+
+__device__ __forceinline__ double f64_sum_reduce(const F64Sum& s, double start, double q, double qinv) {
+  const double v = s.hi - start;
+  const double t = __builtin_fma(v, qinv, kRoundMagic) - kRoundMagic;
+  return __builtin_fma(-t, q, v) + s.lo;
 }
 
 __device__ __forceinline__ uint64_t shoup_mulmod(uint64_t w, uint64_t wp,

@@ -205,6 +205,30 @@ __device__ __forceinline__ void garner_fixed(const KsDigit& d, int64_t* dg) {
   }
 }
 
+// garner_fixed for the P residues of ModDown: canonical residues (the
+// inverse NTT's output), so a difference is within R + 1 primes of zero and
+// its canonical residue follows from the row's reciprocal instead of a
+// division.  rows: NTT records of the P primes.
+template <int R>
+__device__ __forceinline__ void garner_p(const KsDigit& d, const NttRow* rows, int64_t* dg) {
+  const int64_t first = dg[0];
+  int64_t src[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    src[r] = dg[r];
+    dg[r] = first;
+  }
+#pragma unroll
+  for (int row = 1; row < R; ++row) {
+    const Mont mr = digit_mont(d, row);
+    const int64_t digit = mont_mul(canonical_operand(src[row] - dg[row], mr.q, rows[row].qinv),
+                                   global(d.normalizers)[row - 1], mr);
+    dg[row] = digit;
+#pragma unroll
+    for (int t = row + 1; t < R; ++t) dg[t] += mont_mul(digit, global(d.propagation)[(row - 1) * R + t], digit_mont(d, t));
+  }
+}
+
 // The same recurrence in binary64 for a digit whose primes are all below
 // 2^45, from its Garner record (standard-form constants).  Each product is
 // f64_mulmod_signed, exact and within (-0.53q, 0.53q) (the operands stay
@@ -525,23 +549,60 @@ __device__ __forceinline__ void modup_columns_x2(const KsArgs& a, const KsDigit&
   if (d.f64_ok) {
     const double q0 = row0.qd, qi0 = row0.qinv, q1 = row1.qd, qi1 = row1.qinv;
     const double c00 = static_cast<double>(row0.to_mont), c10 = static_cast<double>(row1.to_mont);
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const double x = __longlong_as_double(dig0[at(k)]);
-      v0[k] = f64_mulmod_signed(c00, x, q0, qi0);
-      v1[k] = f64_mulmod_signed(c10, x, q1, qi1);
-    }
-#pragma unroll
-    for (int r = 1; r < kMaxR; ++r) {
-      if (r >= rows) break;
-      const double cr0 = static_cast<double>(global(d.basis_std)[(r - 1) * d.basis_stride + grow0]);
-      const double cr1 = static_cast<double>(global(d.basis_std)[(r - 1) * d.basis_stride + grow1]);
-      const int64_t* src = dig0 + r * n;
+    if constexpr (kRows < 3) {
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
-        const double x = __longlong_as_double(src[at(k)]);
-        v0[k] += f64_mulmod_signed(cr0, x, q0, qi0);
-        v1[k] += f64_mulmod_signed(cr1, x, q1, qi1);
+        const double x = __longlong_as_double(dig0[at(k)]);
+        v0[k] = f64_mulmod_signed(c00, x, q0, qi0);
+        v1[k] = f64_mulmod_signed(c10, x, q1, qi1);
+      }
+#pragma unroll
+      for (int r = 1; r < kMaxR; ++r) {
+        if (r >= rows) break;
+        const double cr0 = static_cast<double>(global(d.basis_std)[(r - 1) * d.basis_stride + grow0]);
+        const double cr1 = static_cast<double>(global(d.basis_std)[(r - 1) * d.basis_stride + grow1]);
+        const int64_t* src = dig0 + r * n;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+          const double x = __longlong_as_double(src[at(k)]);
+          v0[k] += f64_mulmod_signed(cr0, x, q0, qi0);
+          v1[k] += f64_mulmod_signed(cr1, x, q1, qi1);
+        }
+      }
+    } else {
+      // Digits of 3 and 4 rows: one reduction per sum (F64Sum).  Digits are
+      // below 2^45, so the sum is below 2^47 q; its reduced value stays
+      // within q (0.54 + rows^2 / 64) < 0.8q.  Four coefficients at a time
+      // keep both parts of the sums in registers.
+      constexpr int kGroup = 4;
+      const double start0 = f64_sum_start(0x1.0p45 * kRows * q0), start1 = f64_sum_start(0x1.0p45 * kRows * q1);
+#pragma unroll
+      for (int h = 0; h < 16; h += kGroup) {
+        __builtin_amdgcn_sched_barrier(0);  // one group's loads and sums in registers at a time
+        F64Sum s0[kGroup], s1[kGroup];
+#pragma unroll
+        for (int k = 0; k < kGroup; ++k) {
+          const double x = __longlong_as_double(dig0[at(h + k)]);
+          f64_sum_first(s0[k], start0, c00, x);
+          f64_sum_first(s1[k], start1, c10, x);
+        }
+#pragma unroll
+        for (int r = 1; r < kRows; ++r) {
+          const double cr0 = static_cast<double>(global(d.basis_std)[(r - 1) * d.basis_stride + grow0]);
+          const double cr1 = static_cast<double>(global(d.basis_std)[(r - 1) * d.basis_stride + grow1]);
+          const int64_t* src = dig0 + r * n;
+#pragma unroll
+          for (int k = 0; k < kGroup; ++k) {
+            const double x = __longlong_as_double(src[at(h + k)]);
+            f64_sum_add(s0[k], cr0, x);
+            f64_sum_add(s1[k], cr1, x);
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < kGroup; ++k) {
+          v0[h + k] = f64_sum_reduce(s0[k], start0, q0, qi0);
+          v1[h + k] = f64_sum_reduce(s1[k], start1, q1, qi1);
+        }
       }
     }
   } else {
@@ -561,7 +622,7 @@ __device__ __forceinline__ void modup_columns_x2(const KsArgs& a, const KsDigit&
 
 // One launch per arithmetic path, as for the tile pass below.
 template <int S1, int MODE, bool kSmall>
-__global__ __launch_bounds__(kBlock) void k_ks_modup_columns(KsArgs a, int64_t j_begin, int64_t j_count) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSmall && MODE == 1 ? 4 : 2))) void k_ks_modup_columns(KsArgs a, int64_t j_begin, int64_t j_count) {
   // (+1 column of padding: the packed store's transpose pitch)
   __shared__ int64_t lds[(1 << S1) * (kBlock / ((1 << S1) / 16) + 1)];
   // Work items (column group fastest, then destination row, then (entry,
@@ -587,6 +648,7 @@ __global__ __launch_bounds__(kBlock) void k_ks_modup_columns(KsArgs a, int64_t j
     switch (static_cast<int>(d.rows)) {
       case 1: modup_columns_x2<S1, 1>(a, d, di, b, j, two, cg, lds); break;
       case 2: modup_columns_x2<S1, 2>(a, d, di, b, j, two, cg, lds); break;
+      case 3: modup_columns_x2<S1, 3>(a, d, di, b, j, two, cg, lds); break;
       case 4: modup_columns_x2<S1, 4>(a, d, di, b, j, two, cg, lds); break;
       default: modup_columns_x2<S1, 0>(a, d, di, b, j, two, cg, lds); break;
     }
@@ -782,7 +844,7 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e3(t, k));
-        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], kF64 ? 0 : twp[slot]));
+        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
       }
     }
 #pragma unroll
@@ -798,7 +860,7 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e2(t, k));
-        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], kF64 ? 0 : twp[slot]));
+        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
       }
     }
 #pragma unroll
@@ -814,7 +876,7 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e1(t, k));
-        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], kF64 ? 0 : twp[slot]));
+        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
       }
     }
 #pragma unroll
@@ -1512,7 +1574,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e3(t, k));
-        p.inv(v[k], v[k + half], p.tw_make(tww[slot], kF64 ? 0 : twp[slot]));
+        p.inv(v[k], v[k + half], p.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
       }
     }
 #pragma unroll
@@ -1527,7 +1589,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e2(t, k));
-        p.inv(v[k], v[k + half], p.tw_make(tww[slot], kF64 ? 0 : twp[slot]));
+        p.inv(v[k], v[k + half], p.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
       }
     }
 #pragma unroll
@@ -1542,7 +1604,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e1(t, k));
-        p.inv(v[k], v[k + half], p.tw_make(tww[slot], kF64 ? 0 : twp[slot]));
+        p.inv(v[k], v[k + half], p.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
       }
     }
 #pragma unroll
@@ -1630,6 +1692,11 @@ __global__ __launch_bounds__(kBlock) void k_ks_gather_base(View3 base, const int
   out[(b * lq + row) * n + i] = read_maybe_galois(base, gal_idx, gal_sign, b, row, i, twice_q);
 }
 
+// Bound by load latency, then by the binary64 arithmetic: all of a thread's
+// loads issue before any of its work, and each row is one F64Sum (2P + 1
+// products, one reduction).  logN = 16, four P primes: 186 -> 141 us at 7
+// entries of 29 Q rows (3.9 TB/s of accumulators, base and output), 520 ->
+// 385 us at 16 entries of 33 rows with the fused rescale.
 template <int P>
 __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   constexpr int kRows = kModDownRowsPerThread;
@@ -1660,20 +1727,48 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   const bool has_base = (c == 0 ? a.has_base0 : a.has_base1) != 0;
   const View3& out = c == 0 ? a.out0 : a.out1;
   const int64_t row_begin = group * kRows;
-  // Issue every load of the thread first: P rows, Q rows, base rows.
+  const int64_t row_end = row_begin + kRows < a.lq ? row_begin + kRows : a.lq;
+  const int64_t f64_rows = a.small_rows < a.lq ? a.small_rows : a.lq;
+  // Issue every load of the thread's binary64 rows first, with no branch
+  // between them (a row past the end reads the last one): joined branches
+  // made the compiler wait for each row's load in turn, which cost more than
+  // the arithmetic.  The halves of a packed value stay apart until used.
   int64_t dg[P];
+  if (a.small_rows <= a.lq) {
 #pragma unroll
-  for (int r = 0; r < P; ++r) dg[r] = acc_row(a.lq + r);
-  int64_t xv[kRows], bv[kRows];
+    for (int r = 0; r < P; ++r) dg[r] = slab[static_cast<uint32_t>((a.lq + r) * n + i)];
+  } else {
 #pragma unroll
-  for (int rr = 0; rr < kRows; ++rr) {
-    const int64_t row = row_begin + rr;
-    xv[rr] = row < a.lq ? acc_row(row) : 0;
-    bv[rr] = (has_base && row < a.lq) ? base.at(b, row, i) : 0;
+    for (int r = 0; r < P; ++r) dg[r] = acc_row(a.lq + r);
   }
+  uint32_t xlo[kRows], xlo0 = 0;
+  uint16_t xhi[kRows], xhi0 = 0;
+  int64_t bv[kRows], bv0 = 0;
+  if (f64_rows > 0) {
+#pragma unroll
+    for (int rr = 0; rr < kRows; ++rr) {
+      const int64_t row = row_begin + rr < f64_rows ? row_begin + rr : f64_rows - 1;
+      const uint32_t idx = static_cast<uint32_t>(row * n + pidx);
+      xlo[rr] = pk.lo[idx];
+      xhi[rr] = pk.hi[idx];
+    }
+    xlo0 = pk.lo[static_cast<uint32_t>(pidx)];  // row 0, for the fused rescale
+    xhi0 = pk.hi[static_cast<uint32_t>(pidx)];
+    if (has_base) {
+#pragma unroll
+      for (int rr = 0; rr < kRows; ++rr) {
+        const int64_t row = row_begin + rr < f64_rows ? row_begin + rr : f64_rows - 1;
+        bv[rr] = base.at(b, row, i);
+      }
+      bv0 = base.at(b, 0, i);
+    }
+  }
+  auto packed_f64 = [](uint32_t lo, uint16_t hi) -> double {
+    return u64_to_f64(static_cast<uint64_t>(lo) | static_cast<uint64_t>(hi) << 32);
+  };
   // Mixed-radix digits of X mod P (X_P = sum_r c_r prod_{t<r} p_t), each
   // split as c_hi 2^30 + c_lo (both exact in binary64).
-  garner_fixed<P>(a.pdig, dg);
+  garner_p<P>(a.pdig, a.rows + a.level + a.lq, dg);
   double dlo[P], dhi[P];
 #pragma unroll
   for (int r = 0; r < P; ++r) {
@@ -1688,22 +1783,24 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
     if (sum >= twice_q) sum -= twice_q;
     return canonicalize(sum, twice_q);
   };
-  // floor(X / P) mod q of a binary64 row from its 16-word record (M_r,
-  // 2^30 M_r, P^{-1}, ..., q, 1/q): (x - X_P) P^{-1} mod q with
-  // X_P mod q = sum_r c_lo M_r + c_hi 2^30 M_r, all in signed binary64
-  // (|sum| < 4.2q), canonicalised once.
-  // The result of a binary64 row stays in binary64 (exact integers below
-  // 2^47) through the base addition and the fused rescale.
-  auto moddown_f64 = [&](Global<double>* rec, int64_t xval) -> double {
+  // floor(X / P) mod q of a binary64 row from its 16-word record: one sum of
+  // 2P + 1 products (x P^{-1}, and the digit halves of X_P times their
+  // negated constants), reduced once.  x and the constants are below q, the
+  // halves below 2^30, so the sum is below q (q + 2P 2^30) and its reduced
+  // value within 0.52q.  The result of a binary64 row stays in binary64
+  // (exact integers below 2^47) through the base addition and the fused
+  // rescale.
+  auto moddown_f64 = [&](Global<double>* rec, double x) -> double {
     const double q = rec[14], qinv = rec[15];
-    double xp = 0.0;
+    const double start = f64_sum_start(q * (q + 2.0 * P * 0x1.0p30));
+    F64Sum sum;
+    f64_sum_first(sum, start, rec[2 * P], x);
 #pragma unroll
     for (int r = 0; r < P; ++r) {
-      xp += f64_mulmod_signed(rec[r], dlo[r], q, qinv);
-      xp += f64_mulmod_signed(rec[P + r], dhi[r], q, qinv);
+      f64_sum_add(sum, rec[r], dlo[r]);
+      f64_sum_add(sum, rec[P + r], dhi[r]);
     }
-    const double diff = u64_to_f64(static_cast<uint64_t>(xval)) - xp;
-    double res = f64_mulmod_signed(rec[2 * P], diff, q, qinv);
+    const double res = f64_sum_reduce(sum, start, q, qinv);
     return res < 0.0 ? res + q : res;
   };
   // add_canonical of a canonical value and a base below 2q
@@ -1733,50 +1830,54 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   int64_t c0_int = 0;
   int64_t round_up = 0;
   if (rescale) {
-    Global<double>* rec0 = global(a.pdig.f64_table) + a.level * pitch;
-    const int64_t x0 = row_begin == 0 ? xv[0] : acc_row(0);
-    const int64_t b0 = row_begin == 0 ? bv[0] : (has_base ? base.at(b, 0, i) : 0);
-    if (rec0[14] != 0.0) {
-      c0 = add_base_f64(moddown_f64(rec0, x0), b0, rec0[14]);
+    if (f64_rows > 0) {
+      Global<double>* rec0 = global(a.pdig.f64_table) + a.level * pitch;
+      c0 = add_base_f64(moddown_f64(rec0, packed_f64(xlo0, xhi0)), bv0, rec0[14]);
       c0_int = static_cast<int64_t>(f64_to_u64(c0));
     } else {
-      c0_int = moddown_integer(a.level, x0, b0);
+      c0_int = moddown_integer(a.level, acc_row(0), has_base ? base.at(b, 0, i) : 0);
     }
     round_up = c0_int > a.half_drop ? 1 : 0;
   }
 #pragma unroll
   for (int rr = 0; rr < kRows; ++rr) {
     const int64_t row = row_begin + rr;
-    if (row >= a.lq) break;
-    const int64_t grow = a.level + row;
-    Global<double>* rec = global(a.pdig.f64_table) + grow * pitch;
+    if (row >= f64_rows) break;
+    Global<double>* rec = global(a.pdig.f64_table) + (a.level + row) * pitch;
     const double q = rec[14];
-    int64_t value;
-    if (q != 0.0) {
-      double v = add_base_f64(moddown_f64(rec, xv[rr]), bv[rr], q);
-      if (rescale && row > 0) {
-        // ((v - c0) q0^{-1} + round_up) mod q, |v - c0| < 2^47 exact
-        double r = f64_mulmod_signed(static_cast<double>(a.rescale_inv[row - 1]), v - c0, q, rec[15]);
-        r += static_cast<double>(round_up);
-        v = r < 0.0 ? r + q : (r >= q ? r - q : r);
-      }
-      value = static_cast<int64_t>(f64_to_u64(v));
-    } else {
-      value = moddown_integer(grow, xv[rr], bv[rr]);
-      if (rescale && row > 0) {
-        // the dropped prime may exceed this one: c0 mod q first (c0 >= q is
-        // rare, so the division hardly ever runs)
-        const uint64_t qq = a.rows[grow].q;
-        uint64_t c0_q = static_cast<uint64_t>(c0_int);
-        if (c0_q >= qq) c0_q %= qq;
-        int64_t d = value - static_cast<int64_t>(c0_q);
-        if (d < 0) d += static_cast<int64_t>(qq);
-        uint64_t r = shoup_mulmod(static_cast<uint64_t>(a.rescale_inv[row - 1]),
-                                  static_cast<uint64_t>(a.rescale_inv_shoup[row - 1]), static_cast<uint64_t>(d), qq);
-        r += static_cast<uint64_t>(round_up);
-        if (r >= qq) r -= qq;
-        value = static_cast<int64_t>(r);
-      }
+    double v = add_base_f64(moddown_f64(rec, packed_f64(xlo[rr], xhi[rr])), bv[rr], q);
+    if (rescale && row > 0) {
+      // ((v - c0) q0^{-1} + round_up) mod q, |v - c0| < 2^47 exact
+      const double inv = u64_to_f64(static_cast<uint64_t>(global(a.rescale_inv)[row - 1]));
+      double r = f64_mulmod_signed(inv, v - c0, q, rec[15]);
+      r += static_cast<double>(round_up);
+      v = r < 0.0 ? r + q : (r >= q ? r - q : r);
+    }
+    const int64_t value = static_cast<int64_t>(f64_to_u64(v));
+    if (!rescale) {
+      out.at(b, row, i) = value;
+    } else if (row > 0) {
+      out.at(b, row - 1, i) = value;
+    }
+  }
+  // Integer rows (the base prime), one body outside the unrolled loop.
+#pragma nounroll
+  for (int64_t row = row_begin > f64_rows ? row_begin : f64_rows; row < row_end; ++row) {
+    const int64_t grow = a.level + row;
+    int64_t value = moddown_integer(grow, acc_row(row), has_base ? base.at(b, row, i) : 0);
+    if (rescale && row > 0) {
+      // the dropped prime may exceed this one: c0 mod q first (c0 >= q is
+      // rare, so the division hardly ever runs)
+      const uint64_t qq = a.rows[grow].q;
+      uint64_t c0_q = static_cast<uint64_t>(c0_int);
+      if (c0_q >= qq) c0_q %= qq;
+      int64_t d = value - static_cast<int64_t>(c0_q);
+      if (d < 0) d += static_cast<int64_t>(qq);
+      uint64_t r = shoup_mulmod(static_cast<uint64_t>(a.rescale_inv[row - 1]),
+                                static_cast<uint64_t>(a.rescale_inv_shoup[row - 1]), static_cast<uint64_t>(d), qq);
+      r += static_cast<uint64_t>(round_up);
+      if (r >= qq) r -= qq;
+      value = static_cast<int64_t>(r);
     }
     if (!rescale) {
       out.at(b, row, i) = value;

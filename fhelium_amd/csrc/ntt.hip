@@ -182,7 +182,7 @@ __device__ __forceinline__ void inv_tiles(const P& p, int log_n, int g, int64_t*
     for (int k = 0; k < 16; ++k) {
       if (k & half) continue;
       p.inv(v[k], v[k + half],
-            p.tw(tw, twp, (n >> (a + 1)) + (r << (7 - a)) + (t << (3 - a)) + (k >> (a + 1))));
+            p.tw(tw, twp, (n >> (a + 1)) + (r << (7 - a)) + (t << (3 - a)) + (k >> (a + 1))), a);
     }
   }
 #pragma unroll
@@ -197,7 +197,7 @@ __device__ __forceinline__ void inv_tiles(const P& p, int log_n, int g, int64_t*
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & half) continue;
-      p.inv(v[k], v[k + half], p.tw(tw, twp, (n >> (a + 5)) + (r << (3 - a)) + (k >> (a + 1))));
+      p.inv(v[k], v[k + half], p.tw(tw, twp, (n >> (a + 5)) + (r << (3 - a)) + (k >> (a + 1))), a + 4);
     }
   }
 #pragma unroll
@@ -230,7 +230,7 @@ __device__ __forceinline__ void inv_columns(const P& p, Load load, Store store, 
     for (int k = 0; k < 16; ++k) {
       if (k & half) continue;
       p.inv(v[k], v[k + half],
-            p.tw(tw, twp, ((1 << L) >> (kTileLog + a + 1)) + ((16 * t + k) >> (a + 1))));
+            p.tw(tw, twp, ((1 << L) >> (kTileLog + a + 1)) + ((16 * t + k) >> (a + 1))), a);
     }
   }
   if constexpr (S1 > 4) {
@@ -247,7 +247,7 @@ __device__ __forceinline__ void inv_columns(const P& p, Load load, Store store, 
       for (int k = 0; k < 16; ++k) {
         if (k & half) continue;
         p.inv(v[k], v[k + half],
-              p.tw(tw, twp, ((1 << L) >> (kTileLog + b + 1)) + ((t + T * k) >> (b + 1))));
+              p.tw(tw, twp, ((1 << L) >> (kTileLog + b + 1)) + ((t + T * k) >> (b + 1))), b);
       }
     }
 #pragma unroll
@@ -427,7 +427,7 @@ __device__ __forceinline__ void stage_body(const P& p, int64_t* base, const int6
   if (forward) {
     p.fwd(u, l, p.tw(tw, twp, idx));
   } else {
-    p.inv(u, l, p.tw(tw, twp, idx));
+    p.inv(u, l, p.tw(tw, twp, idx), 0);
   }
   base[j] = p.out_fwd(u);
   base[j + half] = p.out_fwd(l);

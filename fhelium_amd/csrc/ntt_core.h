@@ -58,7 +58,9 @@ __device__ __forceinline__ int64_t center_canonical(int64_t r, uint64_t q) {
 //   mid/unmid        working value <-> 64-bit intermediate between passes
 //   out_fwd(v)       final forward value -> int64 residue
 //   out_inv(v, f)    N^{-1} scaling and representation f -> int64 residue
-//   fwd/inv          butterflies; mul_const for to-Montgomery scaling.
+//   fwd/inv          butterflies (inv is told its stage within the pass, a
+//                    compile-time constant after unrolling); mul_const for
+//                    to-Montgomery scaling.
 // ---------------------------------------------------------------------------
 
 // Exact binary64 path (q < 2^42): reference lazy semantics, see fh_common.h.
@@ -97,7 +99,7 @@ struct F64Exact {
     l = sub(u, v);
     u = e;
   }
-  __device__ __forceinline__ void inv(V& u, V& l, Tw w) const {
+  __device__ __forceinline__ void inv(V& u, V& l, Tw w, int) const {
     const V d = sub(u, l);
     u = add(u, l);
     l = mul(w, d);
@@ -149,9 +151,14 @@ struct F64Fast {
     l = u - v;
     u = u + v;
   }
-  __device__ __forceinline__ void inv(V& u, V& l, Tw w) const {
+  // `stage` counts the stages of one pass (0..7).  Sums are reduced at
+  // stages 0 and 4 only: from |x| <= 10q at the start of a pass they grow to
+  // 0.51q, 1.1q, 2.2q, 4.3q over stages 0..3 and again over 4..7, so the
+  // differences stay below 20q (stage 0) and 8.6q, inside the exactness
+  // bound |w x| / q < 2^46.4 for q < 2^42, and a pass ends below 4.3q.
+  __device__ __forceinline__ void inv(V& u, V& l, Tw w, int stage) const {
     const V d = u - l;
-    u = reduce(u + l);
+    u = (stage & 3) == 0 ? reduce(u + l) : u + l;
     l = mul(w, d);
   }
   __device__ __forceinline__ V to_mont(V x) const { return mul(konst(row->to_mont, 0), x); }
@@ -196,7 +203,7 @@ struct U64Path {
     l = sub(u, v);
     u = e;
   }
-  __device__ __forceinline__ void inv(V& u, V& l, Tw w) const {
+  __device__ __forceinline__ void inv(V& u, V& l, Tw w, int) const {
     const V d = sub(u, l);
     u = add(u, l);
     l = mul(w, d);
@@ -251,7 +258,7 @@ struct U64Fast {
     u = a + v;
     l = a + (twoq + 1u) + ~v;  // a - v + 2q without a borrow chain
   }
-  __device__ __forceinline__ void inv(V& u, V& l, Tw w) const {
+  __device__ __forceinline__ void inv(V& u, V& l, Tw w, int) const {
     const V d = u + (twoq + 1u) + ~l;
     u = half(u + l);
     l = mul_lazy(w, d);

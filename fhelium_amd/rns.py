@@ -202,11 +202,13 @@ MODDOWN_RECORD_WORDS = 16
 def moddown_binary64_table(moduli: tuple[int, ...], p_ids: tuple[int, ...],
                            q_ids: tuple[int, ...]) -> torch.Tensor:
     """[Q0, 16] float64 ModDown records, one per Q row whose prime is below
-    BINARY64_PRIME_LIMIT: words 0..P-1 hold M_r mod q, words P..2P-1 hold 2^30 M_r mod q
-    (M_r = prod_{t<r} p_t), word 2P holds P^{-1} mod q, word 14 holds q and
-    word 15 holds 1/q.  Rows of larger primes are all zero (they take the
-    integer path).  One 128-byte record per row lets a wave fetch a row's
-    constants with two scalar loads."""
+    BINARY64_PRIME_LIMIT.  With M_r = prod_{t<r} p_t, words 0..P-1 hold
+    -M_r P^{-1} mod q, words P..2P-1 hold -2^30 M_r P^{-1} mod q, word 2P
+    holds P^{-1} mod q, word 14 holds q and word 15 holds 1/q, so that
+    floor(X / P) = (x - X_P) P^{-1} mod q is one sum of 2P + 1 products (the
+    digits of X_P split at 30 bits).  Rows of larger primes are all zero
+    (they take the integer path).  One 128-byte record per row lets a wave
+    fetch a row's constants with two scalar loads."""
 
     p = [moduli[i] for i in p_ids]
     if 2 * len(p) + 1 > 14:
@@ -220,10 +222,11 @@ def moddown_binary64_table(moduli: tuple[int, ...], p_ids: tuple[int, ...],
         q = moduli[qi]
         if q >= BINARY64_PRIME_LIMIT:
             continue
+        p_inverse = pow(p_product, -1, q)
         for r, m in enumerate(prefix):
-            out[j, r] = float(m % q)
-            out[j, len(p) + r] = float((m << MODDOWN_SPLIT_BITS) % q)
-        out[j, 2 * len(p)] = float(pow(p_product, -1, q))
+            out[j, r] = float(-m * p_inverse % q)
+            out[j, len(p) + r] = float(-(m << MODDOWN_SPLIT_BITS) * p_inverse % q)
+        out[j, 2 * len(p)] = float(p_inverse)
         out[j, 14] = float(q)
         out[j, 15] = 1.0 / q
     return out
