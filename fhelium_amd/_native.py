@@ -114,6 +114,15 @@ SIGNATURES: dict[str, list] = {
     "fh_sample_gaussian": [_ptr, _ptr, ctypes.c_uint32, _i64, ctypes.c_double, _ptr, _ptr],
     "fh_ckks_encode": [_ptr, _i64, _i64, _ptr, ctypes.c_double, _ptr, _i64, _ptr, _ptr, _ptr],
     "fh_ckks_decode": [_ptr, _ptr, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, ctypes.c_double, _ptr, _ptr, _ptr],
+    "fh_codec_tables": [_i64, _ptr, _ptr, _ptr, _ptr],
+    "fh_ckks_encode_coefficients": [_ptr, _i64, _i64, _ptr, _ptr, ctypes.c_double, _ptr, _ptr, _ptr],
+    "fh_ckks_lift_montgomery": [_ptr, _i64, _i64, _i64, _ptr, _i64, fh_table2, _ptr, _ptr],
+    "fh_ckks_decode_rows": [_ptr, _ptr, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, ctypes.c_double, _ptr, _ptr,
+                            _ptr],
+    "fh_ckks_decrypt_decode": [fh_view3, fh_view3, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64,
+                               _i64, _i64, _ptr, _ptr, ctypes.c_double, _ptr, _ptr, _ptr, _ptr],
+    "fh_ntt_forward_lifted": [_ptr, _ptr, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _i32, _i32,
+                              _ptr],
     "fh_ckks_hmult_tensor_coefficient": [_ptr, _ptr, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                          _i64, _i64, fh_table2, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
                                          _i32, _ptr],

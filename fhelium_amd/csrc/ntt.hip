@@ -36,6 +36,8 @@
 // host may split a call into chunks of entries on several streams (a launch
 // schedule chosen per call).  Rings with logN < 12 (tests) use one launch
 // per stage.
+#include <type_traits>
+
 #include "fh_common.h"
 
 #include "ntt_core.h"
@@ -51,9 +53,10 @@ using namespace ::fh::ntt;
 
 // Forward column pass: stages 0 .. S1-1 over rows i of columns c
 // (element 256*i + c).  Block: C = 256/T columns x T = 2^{S1-4} threads.
-// Reads input residues, writes intermediates.
-template <int S1, class P>
-__device__ __forceinline__ void fwd_columns(const P& p, int64_t* base, const int64_t* src,
+// Reads input words, turned into working values by convert(words, values),
+// and writes intermediates.
+template <int S1, class P, class Convert>
+__device__ __forceinline__ void fwd_columns(const P& p, int64_t* base, const int64_t* src, Convert convert,
                                             const int64_t* tw, const int64_t* twp, bool to_mont,
                                             int64_t* lds) {
   constexpr int R1 = 1 << S1;
@@ -63,9 +66,11 @@ __device__ __forceinline__ void fwd_columns(const P& p, int64_t* base, const int
   const int c = threadIdx.x % C;
   const int t = threadIdx.x / C;
   const int col = blockIdx.x * C + c;
-  V v[16];
+  int64_t words[16];
 #pragma unroll
-  for (int k = 0; k < 16; ++k) v[k] = p.in(src[static_cast<int64_t>(t + T * k) * kTile + col]);
+  for (int k = 0; k < 16; ++k) words[k] = src[static_cast<int64_t>(t + T * k) * kTile + col];
+  V v[16];
+  convert(words, v);
   if (to_mont) {
 #pragma unroll
     for (int k = 0; k < 16; ++k) v[k] = p.to_mont(v[k]);
@@ -153,6 +158,95 @@ __device__ __forceinline__ void fwd_tiles(const P& p, int log_n, int g, int64_t*
 }
 
 static_assert(64 % (kBlock / kTilesPerBlock) == 0, "a tile's threads must lie in one wave");
+
+// One product of an NTT-domain value in the working format (Montgomery,
+// unreduced forward output) with a Montgomery word below 2q, in the format
+// and scaling kOutStdMac undoes: a b R^2 on binary64 rows, a b R on others.
+__device__ __forceinline__ double ntt_product(const F64Fast& p, double x, int64_t w) {
+  return f64_mulmod_signed(u64_to_f64(static_cast<uint64_t>(w)), p.reduce(x), p.q, p.qinv);
+}
+__device__ __forceinline__ uint64_t ntt_product(const U64Fast& p, uint64_t x, int64_t w) {
+  // x < 4q, w < 2q: the REDC value is below 2q, inside wide_redc62's range
+  WideAcc acc{0, 0, 0};
+  wide_mac(acc, x, static_cast<uint64_t>(w));
+  return wide_redc62(acc, p.q, p.row->neg_qinv64);
+}
+
+// Tile passes of a product with one NTT-domain polynomial: the last eight
+// forward stages, the product with `words` (the row's NTT-domain Montgomery
+// words) and the first eight inverse stages of each 256-element tile, in
+// place.  The value after the forward stages is owned as the inverse's first
+// round needs it, so the product costs no exchange and no pass over memory.
+template <class P>
+__device__ __forceinline__ void product_tiles(const P& p, int log_n, int g, int64_t* base, const int64_t* tw,
+                                              const int64_t* twp, const int64_t* itw, const int64_t* itwp,
+                                              const int64_t* words, int64_t* lds) {
+  using V = typename P::V;
+  const int m = threadIdx.x / 16;
+  const int t = threadIdx.x % 16;
+  const int r = g * kTilesPerBlock + m;
+  int64_t* tile = base + static_cast<int64_t>(r) * kTile;
+  const int64_t* word = words + static_cast<int64_t>(r) * kTile;
+  int64_t* sh = lds + m * kTilePitch;
+  const int s0 = log_n - kTileLog;
+  const int n = 1 << log_n;
+  V v[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = p.unmid(tile[t + 16 * k]);
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int half = 8 >> a;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      if (k & half) continue;
+      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << (s0 + a)) + (r << a) + (k >> (4 - a))));
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) sh[tile_pad(t + 16 * k)] = p.mid(v[k]);
+  tile_sync();
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = p.unmid(sh[17 * t + k]);
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int half = 8 >> a;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      if (k & half) continue;
+      p.fwd(v[k], v[k + half],
+            p.tw(tw, twp, (1 << (s0 + 4 + a)) + (r << (4 + a)) + (t << a) + (k >> (4 - a))));
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = ntt_product(p, v[k], word[16 * t + k]);
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int half = 1 << a;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      if (k & half) continue;
+      p.inv(v[k], v[k + half],
+            p.tw(itw, itwp, (n >> (a + 1)) + (r << (7 - a)) + (t << (3 - a)) + (k >> (a + 1))), a);
+    }
+  }
+  // each thread rewrites the words it read
+#pragma unroll
+  for (int k = 0; k < 16; ++k) sh[17 * t + k] = p.mid(v[k]);
+  tile_sync();
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = p.unmid(sh[tile_pad(t + 16 * k)]);
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int half = 1 << a;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      if (k & half) continue;
+      p.inv(v[k], v[k + half], p.tw(itw, itwp, (n >> (a + 5)) + (r << (3 - a)) + (k >> (a + 1))), a + 4);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) tile[t + 16 * k] = p.mid(v[k]);
+}
 
 // Inverse tile pass: stages 0..7 inside 256-element tiles.  Reads input
 // residues, writes intermediates.
@@ -281,6 +375,7 @@ struct NttArgs {
   // entry count (the launch covers all entries' rows).  0: 2-D grid of
   // (tile group, flat row from row_offset).
   int64_t tile_batch;
+  int lift;             // forward: src holds signed coefficients (k_fwd_columns_lifted)
 };
 
 struct RowRef {
@@ -352,11 +447,54 @@ enum Mode : int { kExact = 0, kFast = 1 };
     }                                                      \
   } while (0)
 
+template <class P>
+__device__ __forceinline__ void words_in(const P& p, const int64_t (&words)[16], typename P::V (&v)[16]) {
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = p.in(words[k]);
+}
+
+// Working values of signed coefficients' residues: canonical, except that
+// the fast binary64 path takes any small signed representative.  One test
+// over a thread's 16 words picks the short form (a branch per word would
+// make each wait for its own load).
+template <class P>
+__device__ __forceinline__ void words_lift(const P& p, const int64_t (&words)[16], typename P::V (&v)[16]) {
+  if constexpr (std::is_same<P, F64Fast>::value) {
+    uint64_t any = 0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) any |= static_cast<uint64_t>(words[k] ^ (words[k] >> 63));
+    if (any < (uint64_t{1} << 50)) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        // 1.5 2^52 + x for |x| < 2^50
+        v[k] = p.reduce(__longlong_as_double(words[k] + 0x4338000000000000ll) - kRoundMagic);
+      }
+      return;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = p.in(canonical_operand(words[k], p.row->q, p.row->qinv));
+}
+
 template <int S1, int MODE>
 __global__ __launch_bounds__(kBlock) void k_fwd_columns(NttArgs a) {
   __shared__ int64_t lds[(1 << S1) * (kBlock / ((1 << S1) / 16))];
   const RowRef rr = row_ref(a);
-  FH_DISPATCH_PATH(MODE, *rr.row, (fwd_columns<S1>(p, rr.base, rr.src, rr.tw, rr.twp, a.form != 0, lds)));
+  FH_DISPATCH_PATH(MODE, *rr.row,
+                   (fwd_columns<S1>(p, rr.base, rr.src, [&](auto& w, auto& v) { words_in(p, w, v); }, rr.tw, rr.twp,
+                                    a.form != 0, lds)));
+}
+
+// Forward column pass of signed coefficients [batch, N] (src_limb_stride 0)
+// onto every limb: the residues are formed as they are read, so encoding
+// never writes or reads them in the coefficient domain.
+template <int S1, int MODE>
+__global__ __launch_bounds__(kBlock) void k_fwd_columns_lifted(NttArgs a) {
+  __shared__ int64_t lds[(1 << S1) * (kBlock / ((1 << S1) / 16))];
+  const RowRef rr = row_ref(a);
+  FH_DISPATCH_PATH(MODE, *rr.row,
+                   (fwd_columns<S1>(p, rr.base, rr.src, [&](auto& w, auto& v) { words_lift(p, w, v); }, rr.tw, rr.twp,
+                                    a.form != 0, lds)));
 }
 
 template <int MODE>
@@ -396,6 +534,21 @@ __global__ __launch_bounds__(kBlock) void k_inv_columns(NttArgs a) {
   auto load = [&](int i, int c) -> int64_t { return base[static_cast<int64_t>(i) * kTile + c]; };
   auto store = [&](int i, int c, int64_t v) { base[static_cast<int64_t>(i) * kTile + c] = v; };
   FH_DISPATCH_PATH(MODE, *rr.row, (inv_columns<S1>(p, load, store, rr.tw, rr.twp, a.form, lds)));
+}
+
+// Grid (tile groups, flat rows); `words` [limbs, N].
+__global__ __launch_bounds__(kBlock) void k_product_tiles(NttArgs a, const int64_t* itw, const int64_t* itwp,
+                                                         const int64_t* words, int64_t words_stride) {
+  __shared__ int64_t lds[kTilesPerBlock * kTilePitch];
+  const RowRef rr = row_ref(a);
+  const int64_t off = (a.row_start + rr.limb) << a.log_n;
+  const int64_t* w = words + rr.limb * words_stride;
+  const int g = static_cast<int>(blockIdx.x);
+  if (rr.row->small) {
+    product_tiles(F64Fast(*rr.row), a.log_n, g, rr.base, rr.tw, rr.twp, itw + off, itwp + off, w, lds);
+  } else {
+    product_tiles(U64Fast(*rr.row), a.log_n, g, rr.base, rr.tw, rr.twp, itw + off, itwp + off, w, lds);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -475,7 +628,9 @@ template <int MODE>
 void launch_columns(bool forward, int s1, dim3 grid, hipStream_t stream, const NttArgs& a) {
 #define FH_COLUMNS_CASE(S)                                                           \
   case S:                                                                            \
-    if (forward) {                                                                   \
+    if (forward && a.lift) {                                                         \
+      hipLaunchKernelGGL((k_fwd_columns_lifted<S, MODE>), grid, dim3(kBlock), 0, stream, a); \
+    } else if (forward) {                                                            \
       hipLaunchKernelGGL((k_fwd_columns<S, MODE>), grid, dim3(kBlock), 0, stream, a); \
     } else {                                                                         \
       hipLaunchKernelGGL((k_inv_columns<S, MODE>), grid, dim3(kBlock), 0, stream, a); \
@@ -711,6 +866,24 @@ int forward_columns_internal(int64_t* dst, const int64_t* src, int64_t batch, in
   return kOk;
 }
 
+int product_internal(int64_t* dst, const int64_t* src, int64_t batch, int64_t limbs, int log_n,
+                     int64_t src_batch_stride, int64_t src_limb_stride, const NttRow* rows, const int64_t* tw,
+                     const int64_t* twp, const int64_t* itw, const int64_t* itwp, int64_t row_start,
+                     const int64_t* words, int64_t words_stride, hipStream_t stream) {
+  const int64_t n = int64_t{1} << log_n;
+  FH_CHECK_ARG(batch * limbs <= kMaxGridY, "product with one polynomial: %lld rows exceed the launch grid",
+               (long long)(batch * limbs));
+  int st = forward_columns_internal(dst, src, batch, limbs, log_n, limbs * n, n, src_batch_stride, src_limb_stride,
+                                    rows, tw, twp, row_start, true, stream);
+  if (st != kOk) return st;
+  NttArgs a{dst, limbs * n, n, limbs, 0, rows, tw, twp, row_start, log_n, 0, 1};
+  const dim3 grid(static_cast<uint32_t>(n / (kTile * kTilesPerBlock)), static_cast<uint32_t>(batch * limbs));
+  hipLaunchKernelGGL(k_product_tiles, grid, dim3(kBlock), 0, stream, a, itw, itwp, words, words_stride);
+  FH_CHECK_LAUNCH("product with one polynomial");
+  return inverse_columns_internal(dst, batch, limbs, log_n, limbs * n, n, rows, itw, itwp, row_start, kOutStdMac, 0,
+                                  stream);
+}
+
 int inverse_columns_internal(int64_t* data, int64_t batch, int64_t limbs, int log_n,
                              int64_t batch_stride, int64_t limb_stride, const NttRow* rows,
                              const int64_t* tw, const int64_t* twp, int64_t row_start,
@@ -781,6 +954,24 @@ FH_API int fh_ntt_forward_from(int64_t* residues, const int64_t* source, int64_t
   NttArgs a{residues, batch_stride, limb_stride, limbs, 0, static_cast<const NttRow*>(ntt_rows),
             twiddles, twiddles_shoup, row_start, static_cast<int>(log_n), to_montgomery ? 1 : 0, 0,
             source, source_batch_stride, source_limb_stride};
+  return launch(a, batch * limbs, true, mode, static_cast<hipStream_t>(stream));
+}
+
+// Signed coefficients [batch, N] onto `limbs` rows and forward.
+FH_API int fh_ntt_forward_lifted(int64_t* residues, const int64_t* coefficients, int64_t batch, int64_t limbs,
+                                 int64_t log_n, int64_t batch_stride, int64_t limb_stride,
+                                 int64_t coefficient_batch_stride, const void* ntt_rows, const int64_t* twiddles,
+                                 const int64_t* twiddles_shoup, int64_t row_start, int32_t to_montgomery,
+                                 int32_t mode, void* stream) {
+  int st = check_ntt_common(batch, limbs, log_n, ntt_rows, twiddles, twiddles_shoup, row_start, mode);
+  if (st != kOk) return st;
+  FH_CHECK_ARG(log_n >= 12, "lifted forward NTT supports logN 12..16");
+  if (batch == 0 || limbs == 0) return kOk;
+  FH_CHECK_ARG(residues != nullptr && coefficients != nullptr, "NTT operands must be non-null");
+  NttArgs a{residues, batch_stride, limb_stride, limbs, 0, static_cast<const NttRow*>(ntt_rows),
+            twiddles, twiddles_shoup, row_start, static_cast<int>(log_n), to_montgomery ? 1 : 0, 0,
+            coefficients, coefficient_batch_stride, 0};
+  a.lift = 1;
   return launch(a, batch * limbs, true, mode, static_cast<hipStream_t>(stream));
 }
 

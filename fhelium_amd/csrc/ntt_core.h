@@ -324,6 +324,14 @@ int forward_columns_internal(int64_t* dst, const int64_t* src, int64_t batch, in
                              int64_t dst_batch_stride, int64_t dst_limb_stride, int64_t src_batch_stride,
                              int64_t src_limb_stride, const NttRow* rows, const int64_t* tw,
                              const int64_t* twp, int64_t row_start, bool to_montgomery, hipStream_t stream);
+// src [batch, limbs, N] (standard residues) times one NTT-domain polynomial
+// (words [limbs, N], Montgomery, below 2q) back in the coefficient domain,
+// canonical standard, into dst [batch, limbs, N] contiguous (logN 12..16,
+// fast arithmetic, three launches).
+int product_internal(int64_t* dst, const int64_t* src, int64_t batch, int64_t limbs, int log_n,
+                     int64_t src_batch_stride, int64_t src_limb_stride, const NttRow* rows, const int64_t* tw,
+                     const int64_t* twp, const int64_t* itw, const int64_t* itwp, int64_t row_start,
+                     const int64_t* words, int64_t words_stride, hipStream_t stream);
 // Only the column pass of that inverse (logN 12..16): for rows whose tile
 // stages were already applied, holding working-format values.
 // packed_rows > 0: limbs [0, packed_rows) of each batch entry are binary64

@@ -245,14 +245,20 @@ class CkksEngine:
     def decrypt_residues(self, ct: Ciphertext) -> torch.Tensor:
         """Canonical standard residues of <c, (1, s, s^2, ...)> over the ct's Q rows."""
 
+        return self._decrypt_rows(ct, 0)
+
+    def _decrypt_rows(self, ct: Ciphertext, skip: int) -> torch.Tensor:
+        """decrypt_residues of the rows after the ciphertext's first ``skip``."""
+
         cfg = self.config
         sk = self._require_secret()
         rt = self.runtime
-        params = rt.params(ct.level)
-        s = sk.data[ct.level: cfg.num_q_primes]
-        comps = ct.data.clone()
+        start = ct.level + skip
+        params = rt.params_rows(start, cfg.num_q_primes)
+        s = sk.data[start: cfg.num_q_primes]
+        comps = ct.data[..., skip:, :].clone()
         if ct.polynomial_domain == "coefficient":
-            rt.ntt.forward_to_montgomery_(comps, ct.level)
+            rt.ntt.forward_to_montgomery_(comps, start)
         elif ct.residue_representation != "montgomery":
             raise CkksStateError("NTT-domain values must be Montgomery")
         acc = comps[0]
@@ -261,7 +267,7 @@ class CkksEngine:
             power = s if power is None else K.montgomery_mul(power, s, params)
             acc = K.add_lazy(acc, K.montgomery_mul(comps[i], power, params), params)
         acc = acc.contiguous()
-        rt.ntt.inverse_to_standard_(acc, ct.level)
+        rt.ntt.inverse_to_standard_(acc, start)
         return acc
 
     def decrypt(self, ct: Ciphertext, crt_primes: int = 3) -> np.ndarray:
@@ -322,11 +328,32 @@ class CkksEngine:
         if v.dim() < 1 or v.size(-1) > cfg.slots:
             raise ValueError(f"at most {cfg.slots} slots per plaintext")
         batch_shape = tuple(v.shape[:-1])
-        flat = torch.zeros((int(np.prod(batch_shape)) if batch_shape else 1, cfg.slots), dtype=torch.complex128,
-                           device=self.device)
-        flat[:, : v.size(-1)] = v.reshape(-1, v.size(-1)).to(torch.complex128)
+        if v.size(-1) == cfg.slots and v.dtype == torch.complex128 and v.numel():
+            flat = v.reshape(-1, cfg.slots).resolve_conj().contiguous()
+        else:
+            flat = torch.zeros((int(np.prod(batch_shape)) if batch_shape else 1, cfg.slots), dtype=torch.complex128,
+                               device=self.device)
+            flat[:, : v.size(-1)] = v.reshape(-1, v.size(-1)).to(torch.complex128)
         ws = torch.empty((flat.size(0), cfg.N, 2), dtype=torch.float64, device=self.device)
         rows = self.layout.prime_ids(level)
+        start = self.runtime.row_start(level)
+        if 12 <= cfg.logN <= 16:
+            # rounded coefficients once, then straight onto every row in the
+            # requested domain
+            twiddles, slot_map = self._codec_tables()
+            coeffs = torch.empty((flat.size(0), cfg.N), dtype=torch.int64, device=self.device)
+            nat.call("fh_ckks_encode_coefficients", torch.view_as_real(flat).data_ptr(), flat.size(0), cfg.logN,
+                     slot_map.data_ptr(), twiddles.data_ptr(), scale, ws.data_ptr(), coeffs.data_ptr(),
+                     nat.stream_ptr(self.device))
+            if polynomial_domain == "ntt":
+                data = self.runtime.ntt.forward_lifted_to_montgomery(coeffs, len(rows), start)
+            else:
+                data = torch.empty((flat.size(0), len(rows), cfg.N), dtype=torch.int64, device=self.device)
+                nat.call("fh_ckks_lift_montgomery", coeffs.data_ptr(), flat.size(0), len(rows), cfg.N,
+                         self.runtime.ntt_tables.rows.data_ptr(), start, nat.t2(self.runtime.params(level)),
+                         data.data_ptr(), nat.stream_ptr(self.device))
+            return Plaintext(data=data.reshape(*batch_shape, len(rows), cfg.N), level=level, scale=scale,
+                             polynomial_domain=polynomial_domain)
         moduli = self._moduli_cache.get(rows)
         if moduli is None:
             moduli = torch.tensor([cfg.moduli[i] for i in rows], dtype=torch.int64, device=self.device)
@@ -345,23 +372,73 @@ class CkksEngine:
     def decrypt_on_device(self, ct: Ciphertext) -> torch.Tensor:
         """Slots [*batch, S] complex128 on the device: decryption, then the
         centered CRT over the last two Q rows and the embedding on the
-        device (fh_ckks_decode)."""
+        device.  Only those two rows are decrypted: the others do not enter
+        the result."""
 
         from fhelium_amd import _native as nat
 
         cfg = self.config
-        res = self.decrypt_residues(ct)
-        lq = res.size(-2)
-        if lq < 2:
-            raise ValueError("device decode needs at least two Q rows")
-        flat = res.reshape(-1, lq, cfg.N)
-        qa, qb = cfg.moduli[ct.level + lq - 1], cfg.moduli[ct.level + lq - 2]
-        ws = torch.empty((flat.size(0), cfg.N, 2), dtype=torch.float64, device=self.device)
-        out = torch.empty((flat.size(0), cfg.slots), dtype=torch.complex128, device=self.device)
-        nat.call("fh_ckks_decode", flat[:, lq - 1].data_ptr(), flat[:, lq - 2].data_ptr(), flat.stride(0),
-                 flat.size(0), cfg.logN, qa, qb, pow(qa, -1, qb), self._slot_positions().data_ptr(), float(ct.scale),
-                 ws.data_ptr(), torch.view_as_real(out).data_ptr(), nat.stream_ptr(self.device))
-        return out.reshape(*res.shape[:-2], cfg.slots)
+        lq = ct.data.size(-2)
+        if ct.includes_p or lq != cfg.num_q_primes - ct.level or ct.data.size(-1) != cfg.N or lq < 2:
+            lq = self.decrypt_residues(ct).size(-2)  # raises for a payload its level does not describe
+            raise ValueError("device decode needs at least two Q rows" if lq < 2 else
+                             "device decode needs a Q-basis ciphertext of its level's rows")
+        start = ct.level + lq - 2
+        qa, qb = cfg.moduli[start + 1], cfg.moduli[start]
+        batch_shape = ct.batch_shape
+        b = math.prod(batch_shape)
+        ws = torch.empty((b, cfg.N, 2), dtype=torch.float64, device=self.device)
+        out = torch.empty((b, cfg.slots), dtype=torch.complex128, device=self.device)
+        two_pass = 12 <= cfg.logN <= 16
+        if two_pass and b <= 32767 and ct.component_count == 2 and ct.polynomial_domain == "coefficient":
+            sk = self._require_secret()
+            rows = ct.data[..., lq - 2:, :]
+            if rows.stride(-1) != 1:
+                rows = rows.contiguous()
+            nat.require_device(rows, sk.data)
+            if rows.dtype != torch.int64 or rows.device != sk.data.device:
+                raise TypeError("decryption needs int64 residues on the secret key's device")
+            c0, c1 = rows[0].reshape(b, 2, cfg.N), rows[1].reshape(b, 2, cfg.N)
+            s = sk.data[start: start + 2]
+            product = torch.empty((b, 2, cfg.N), dtype=torch.int64, device=self.device)
+            nt = self.runtime.ntt_tables
+            twiddles, slot_map = self._codec_tables()
+            nat.call("fh_ckks_decrypt_decode", nat.v3(c0), nat.v3(c1), b, cfg.logN, start, nt.rows.data_ptr(),
+                     nt.fwd.data_ptr(), nt.fwd_shoup.data_ptr(), nt.inv.data_ptr(), nt.inv_shoup.data_ptr(),
+                     s.data_ptr(), s.stride(0), qa, qb, pow(qa, -1, qb), slot_map.data_ptr(), twiddles.data_ptr(),
+                     float(ct.scale), product.data_ptr(), ws.data_ptr(), torch.view_as_real(out).data_ptr(),
+                     nat.stream_ptr(self.device))
+            return out.reshape(*batch_shape, cfg.slots)
+        flat = self._decrypt_rows(ct, lq - 2).reshape(-1, 2, cfg.N)
+        args = (flat[:, 1].data_ptr(), flat[:, 0].data_ptr(), flat.stride(0), flat.size(0), cfg.logN, qa, qb,
+                pow(qa, -1, qb))
+        if two_pass:
+            twiddles, slot_map = self._codec_tables()
+            nat.call("fh_ckks_decode_rows", *args, slot_map.data_ptr(), twiddles.data_ptr(), float(ct.scale),
+                     ws.data_ptr(), torch.view_as_real(out).data_ptr(), nat.stream_ptr(self.device))
+        else:
+            nat.call("fh_ckks_decode", *args, self._slot_positions().data_ptr(), float(ct.scale), ws.data_ptr(),
+                     torch.view_as_real(out).data_ptr(), nat.stream_ptr(self.device))
+        return out.reshape(*batch_shape, cfg.slots)
+
+    def _codec_tables(self) -> tuple[torch.Tensor, torch.Tensor]:
+        """(twiddles [2N] complex128, slot map [N] int32) of the two-pass
+        codec, built on first use; the build is waited for once, so that any
+        stream may use them."""
+
+        from fhelium_amd import _native as nat
+
+        hit = self.__dict__.get("_codec_tables_dev")
+        if hit is None:
+            n = self.config.N
+            twiddles = torch.empty(2 * n, dtype=torch.complex128, device=self.device)
+            slot_map = torch.empty(n, dtype=torch.int32, device=self.device)
+            nat.call("fh_codec_tables", self.config.logN, self._slot_positions().data_ptr(),
+                     torch.view_as_real(twiddles).data_ptr(), slot_map.data_ptr(), nat.stream_ptr(self.device))
+            torch.cuda.current_stream(self.device).synchronize()
+            hit = (twiddles, slot_map)
+            self._codec_tables_dev = hit
+        return hit
 
     def _check_plaintext(self, ct: Ciphertext, pt: Plaintext, domain: str) -> None:
         if pt.level != ct.level:

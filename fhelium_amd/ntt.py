@@ -210,6 +210,35 @@ class Gfx950NttBackend:
             rec.append((start, end, 2 * src.size(0) * src.size(1) * src.size(2) * 8))
         return out
 
+    def forward_lifted_to_montgomery(self, coefficients: torch.Tensor, rows: int,
+                                     parameter_row_start: int) -> torch.Tensor:
+        """Signed int64 coefficients [*batch, N] (contiguous, logN 12..16) ->
+        NTT/Montgomery residues [*batch, rows, N] of rows parameter_row_start
+        onwards: the reduction modulo each prime and the forward transform in
+        one pass pair (fh_ntt_forward_lifted)."""
+
+        t = self.tables
+        n = 1 << t.log_n
+        nat.require_device(coefficients)
+        if coefficients.dtype != torch.int64 or coefficients.size(-1) != n or not coefficients.is_contiguous():
+            raise ValueError(f"lifted transform takes contiguous int64 coefficients [*, {n}]")
+        if parameter_row_start < 0 or rows < 1 or parameter_row_start + rows > t.rows.size(0):
+            raise ValueError("lifted transform rows exceed the prepared canonical parameter range")
+        flat = coefficients.view(-1, n)
+        out = torch.empty((*coefficients.shape[:-1], rows, n), dtype=torch.int64, device=coefficients.device)
+        rec = self.recorder
+        if rec is not None:
+            start = torch.cuda.Event(enable_timing=True)
+            end = torch.cuda.Event(enable_timing=True)
+            start.record()
+        nat.call("fh_ntt_forward_lifted", out.data_ptr(), flat.data_ptr(), flat.size(0), rows, t.log_n, rows * n, n,
+                 n, t.rows.data_ptr(), t.fwd.data_ptr(), t.fwd_shoup.data_ptr(), parameter_row_start, 1, self._mode,
+                 nat.stream_ptr(out.device))
+        if rec is not None:
+            end.record()
+            rec.append((start, end, (flat.numel() + out.numel()) * 8))
+        return out
+
     def inverse_to_standard(self, operand: torch.Tensor, parameter_row_start: int) -> torch.Tensor:
         """Out-of-place inverse to canonical standard residues."""
 

@@ -117,6 +117,14 @@ int fh_ntt_forward_from(int64_t* residues, const int64_t* source, int64_t batch,
                         const void* ntt_rows, const int64_t* twiddles,
                         const int64_t* twiddles_shoup, int64_t row_start, int32_t to_montgomery,
                         int32_t mode, void* stream);
+/* fh_ntt_forward of signed integer coefficients [batch, N] onto `limbs` rows
+ * (logN 12..16): the residues mod each row's prime are formed as the first
+ * pass reads them. */
+int fh_ntt_forward_lifted(int64_t* residues, const int64_t* coefficients, int64_t batch, int64_t limbs,
+                          int64_t log_n, int64_t batch_stride, int64_t limb_stride,
+                          int64_t coefficient_batch_stride, const void* ntt_rows, const int64_t* twiddles,
+                          const int64_t* twiddles_shoup, int64_t row_start, int32_t to_montgomery,
+                          int32_t mode, void* stream);
 /* fh_ntt_inverse reading `source` (same [batch, limb, N] shape, its own
  * strides) and writing `residues`; `source` is left unchanged.  Replaces the
  * clone + in-place inverse of relinearize (ckks_engine.py:1608-1675). */
@@ -402,6 +410,41 @@ int fh_ckks_decode(const int64_t* residues_a, const int64_t* residues_b, int64_t
                    int64_t log_n, int64_t modulus_a, int64_t modulus_b, int64_t modulus_a_inverse_mod_b,
                    const int32_t* slot_positions, double scale, double* workspace, double* slots,
                    void* stream);
+/* Tables of the two-pass codec (logN 12..16): twiddles [2N] complex,
+ * twiddles[h + k] = e^{i pi k / h} for every power of two h <= N, k < h;
+ * slot_map int32 [N], j where slot_positions[j] = p and ~j where
+ * N - 1 - slot_positions[j] = p. */
+int fh_codec_tables(int64_t log_n, const int32_t* slot_positions, double* twiddles, int32_t* slot_map,
+                    void* stream);
+/* fh_ckks_encode up to the rounding (two launches, the same rounded values):
+ * out [batch, N] = rint(scale * coefficient). */
+int fh_ckks_encode_coefficients(const double* slots, int64_t batch, int64_t log_n, const int32_t* slot_map,
+                                const double* twiddles, double scale, double* workspace, int64_t* out,
+                                void* stream);
+/* Signed coefficients [batch, n] -> canonical Montgomery residues
+ * [batch, limbs, n] of rows row_start .. row_start + limbs (ntt_rows: every
+ * row's record; rns_params: the limbs' columns). */
+int fh_ckks_lift_montgomery(const int64_t* coefficients, int64_t batch, int64_t limbs, int64_t n,
+                            const void* ntt_rows, int64_t row_start, fh_table2 rns_params, int64_t* out,
+                            void* stream);
+/* fh_ckks_decode in two launches with the codec tables. */
+int fh_ckks_decode_rows(const int64_t* residues_a, const int64_t* residues_b, int64_t batch_stride, int64_t batch,
+                        int64_t log_n, int64_t modulus_a, int64_t modulus_b, int64_t modulus_a_inverse_mod_b,
+                        const int32_t* slot_map, const double* twiddles, double scale, double* workspace,
+                        double* slots, void* stream);
+/* Decryption and decode of two-component coefficient-domain ciphertexts in
+ * five launches: c0 + c1 s on the last two Q rows (c0, c1 [batch, 2, N] views
+ * of them, prime b then prime a, parameter rows row_start and row_start + 1),
+ * then fh_ckks_decode_rows.  The remaining rows do not enter the result.
+ * secret: NTT-domain Montgomery words of those two rows.  product: batch * 2N
+ * words; workspace: batch * N complex. */
+int fh_ckks_decrypt_decode(fh_view3 c0, fh_view3 c1, int64_t batch, int64_t log_n, int64_t row_start,
+                           const void* ntt_rows, const int64_t* forward_twiddles,
+                           const int64_t* forward_twiddles_shoup, const int64_t* inverse_twiddles,
+                           const int64_t* inverse_twiddles_shoup, const int64_t* secret,
+                           int64_t secret_row_stride, int64_t modulus_a, int64_t modulus_b,
+                           int64_t modulus_a_inverse_mod_b, const int32_t* slot_map, const double* twiddles,
+                           double scale, int64_t* product, double* workspace, double* slots, void* stream);
 /* keyswitch_moddown_qp_to_q */
 int fh_ckks_moddown(fh_view3 out, fh_view3 q_residues, fh_view3 p_residues,
                     fh_table2 p_drop_inverses, fh_table2 rns_params, int64_t batch,
