@@ -410,6 +410,31 @@ __device__ __forceinline__ void modup_columns(const P& p, const KsArgs& a, const
         v[k] = u64_to_f64(extend_integer(d, row, grow, dig0, n, pos));
       }
     }
+  } else if constexpr (std::is_same<P, U64Pm>::value) {
+    // Integer rows of a prime 2^60 - delta: the exact sum of the digit
+    // products (digits and constants below 2^60, at most 8 terms), reduced
+    // once: 4 multiplies per product and 3 per coefficient, against 10 per
+    // Shoup product.  Eight coefficients at a time keep the wide sums in
+    // registers, each digit row's loads issued together.
+#pragma unroll
+    for (int h = 0; h < 16; h += 8) {
+      WideAcc s[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        s[k] = WideAcc{0, 0, 0};
+        wide_mac(s[k], digit_u64(d, dig0[at(h + k)]), row.to_mont);
+      }
+#pragma unroll
+      for (int r = 1; r < kMaxR; ++r) {
+        if (r >= rows) break;
+        const uint64_t cr = static_cast<uint64_t>(global(d.basis_std)[(r - 1) * d.basis_stride + grow]);
+        const int64_t* src = dig0 + r * n;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) wide_mac(s[k], digit_u64(d, src[at(h + k)]), cr);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[h + k] = p.reduce(s[k]);
+    }
   } else {
     // Integer rows (fast path): each term d_r (M_r R mod q) is a Shoup
     // product left in [0, 2q); the sum (below 2 rows q <= 16q < 2^64) is
@@ -466,7 +491,7 @@ __device__ __forceinline__ void modup_tail(const P& p, const KsArgs& a, int64_t 
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & half) continue;
-      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << s) + (k >> (4 - s))));
+      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << s) + (k >> (4 - s))), s);
     }
   }
   int64_t* out = a.inter + ((b * a.dnum + di) * a.lqp + j) * n;
@@ -481,7 +506,7 @@ __device__ __forceinline__ void modup_tail(const P& p, const KsArgs& a, int64_t 
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & half) continue;
-      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << s) + ((16 * t + k) >> (S1 - s))));
+      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << s) + ((16 * t + k) >> (S1 - s))), s);
     }
   }
   if constexpr (std::is_same<P, F64Fast>::value) {
@@ -622,7 +647,7 @@ __device__ __forceinline__ void modup_columns_x2(const KsArgs& a, const KsDigit&
 
 // One launch per arithmetic path, as for the tile pass below.
 template <int S1, int MODE, bool kSmall>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSmall && MODE == 1 ? 4 : 2))) void k_ks_modup_columns(KsArgs a, int64_t j_begin, int64_t j_count) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSmall && MODE == 0 ? 2 : 4))) void k_ks_modup_columns(KsArgs a, int64_t j_begin, int64_t j_count) {
   // (+1 column of padding: the packed store's transpose pitch)
   __shared__ int64_t lds[(1 << S1) * (kBlock / ((1 << S1) / 16) + 1)];
   // Work items (column group fastest, then destination row, then (entry,
@@ -665,6 +690,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSmall &
   if constexpr (kSmall) {
     modup_columns<S1, 0>(F64Exact(row), a, d, di, b, j, cg, lds);
   } else {
+    if (row.delta60) {
+      switch (static_cast<int>(d.rows)) {
+        case 1: modup_columns<S1, 1>(U64Pm(row), a, d, di, b, j, cg, lds); break;
+        case 2: modup_columns<S1, 2>(U64Pm(row), a, d, di, b, j, cg, lds); break;
+        case 3: modup_columns<S1, 3>(U64Pm(row), a, d, di, b, j, cg, lds); break;
+        case 4: modup_columns<S1, 4>(U64Pm(row), a, d, di, b, j, cg, lds); break;
+        default: modup_columns<S1, 0>(U64Pm(row), a, d, di, b, j, cg, lds); break;
+      }
+      return;
+    }
     switch (static_cast<int>(d.rows)) {
       case 1: modup_columns<S1, 1>(U64Fast(row), a, d, di, b, j, cg, lds); break;
       case 2: modup_columns<S1, 2>(U64Fast(row), a, d, di, b, j, cg, lds); break;
@@ -792,7 +827,7 @@ __device__ __forceinline__ MacDest hoisted_dest(const KsArgs& a, int r, int t, i
 // the rest of the inverse), then the working-format store the inverse column
 // pass reads.  With kHoist the sums arrive in source order and first move to
 // the destination layout through the exchange buffer.
-template <bool kHoist, class Acc>
+template <bool kHoist, class PI, class Acc>
 __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b, int t, const MacDest& dst,
                                            int64_t* sh, int64_t* tww, int64_t* twp, Acc (&acc0)[8],
                                            Acc (&acc1)[8]) {
@@ -830,12 +865,13 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
       const int g = idx - (kTile - (kTile >> st));
       const int64_t gi = (n >> (st + 1)) + (static_cast<int64_t>(r_dst) << (7 - st)) + g;
       tww[idx] = w_row[gi];
-      if constexpr (!kF64) twp[idx] = wp_row[gi];
+      if constexpr (PI::kCompanion) twp[idx] = wp_row[gi];
     }
   }
   tile_sync();
   auto inv_slot = [](int st, int e) { return (kTile - (kTile >> st)) + (e >> (st + 1)); };
-  auto inverse_tile = [&](const auto& pi, auto (&v)[8], auto store) {
+  const PI pi(row);
+  auto inverse_tile = [&](auto (&v)[8], auto store) {
     // Round 1 (slots = bits 2..0 of the element): inverse stages 0..2.
 #pragma unroll
     for (int st = 0; st < 3; ++st) {
@@ -844,7 +880,7 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e3(t, k));
-        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
+        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], PI::kCompanion ? twp[slot] : 0), st);
       }
     }
 #pragma unroll
@@ -860,7 +896,7 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e2(t, k));
-        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
+        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], PI::kCompanion ? twp[slot] : 0), st);
       }
     }
 #pragma unroll
@@ -876,7 +912,7 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e1(t, k));
-        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
+        pi.inv(v[k], v[k + half], pi.tw_make(tww[slot], PI::kCompanion ? twp[slot] : 0), st);
       }
     }
 #pragma unroll
@@ -886,22 +922,20 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
   };
   if constexpr (kF64) {
     // binary64 rows of the accumulators travel packed (canonical, 6 bytes)
-    const F64Fast pi(row);
     const PackedInter pk0 = packed_slab(a.acc + (0 * a.batch + b) * a.lqp * n, a.small_rows, n);
     const PackedInter pk1 = packed_slab(a.acc + (1 * a.batch + b) * a.lqp * n, a.small_rows, n);
     const int64_t row_off = j * n;
-    inverse_tile(pi, acc0, [&](int e, double x) {
+    inverse_tile(acc0, [&](int e, double x) {
       packed_store(pk0, row_off + packed_index(r_dst, e), f64_to_u64(pi.canon(x)));
     });
-    inverse_tile(pi, acc1, [&](int e, double x) {
+    inverse_tile(acc1, [&](int e, double x) {
       packed_store(pk1, row_off + packed_index(r_dst, e), f64_to_u64(pi.canon(x)));
     });
   } else {
-    const U64Fast pi(row);
     int64_t* out0 = a.acc + ((0 * a.batch + b) * a.lqp + j) * n + static_cast<int64_t>(r_dst) * kTile;
     int64_t* out1 = a.acc + ((1 * a.batch + b) * a.lqp + j) * n + static_cast<int64_t>(r_dst) * kTile;
-    inverse_tile(pi, acc0, [&](int e, uint64_t x) { out0[e] = static_cast<int64_t>(x); });
-    inverse_tile(pi, acc1, [&](int e, uint64_t x) { out1[e] = static_cast<int64_t>(x); });
+    inverse_tile(acc0, [&](int e, uint64_t x) { out0[e] = static_cast<int64_t>(x); });
+    inverse_tile(acc1, [&](int e, uint64_t x) { out1[e] = static_cast<int64_t>(x); });
   }
 }
 
@@ -928,14 +962,14 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
       const int st = 31 - __builtin_clz(idx + 1);
       const int64_t gi = (int64_t{1} << (s0 + st)) + (static_cast<int64_t>(r) << st) + (idx + 1 - (1 << st));
       tww[idx] = w_row[gi];
-      if constexpr (!kF64) twp[idx] = wp_row[gi];
+      if constexpr (P::kCompanion) twp[idx] = wp_row[gi];
     }
     if (threadIdx.x < a.dnum) key_digit[threadIdx.x] = a.dig[threadIdx.x].key_digit;
   }
   __syncthreads();
   auto tw_at = [&](int st, int e) {
     const int slot = mac_tw_slot(st, e);
-    return p.tw_make(tww[slot], kF64 ? 0 : twp[slot]);
+    return p.tw_make(tww[slot], P::kCompanion ? twp[slot] : 0);
   };
   Global<int64_t>* key = global(a.key_bases ? reinterpret_cast<const int64_t*>(a.key_bases[b]) : a.key);
   const int64_t tile_off = static_cast<int64_t>(r) * kTile;
@@ -1013,7 +1047,7 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
-        p.fwd(v[k], v[k + half], tw_at(st, mac_e1(t, k)));
+        p.fwd(v[k], v[k + half], tw_at(st, mac_e1(t, k)), st);
       }
     }
     // The previous digit's last reads of this buffer must be done.
@@ -1030,7 +1064,7 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
-        p.fwd(v[k], v[k + half], tw_at(st, mac_e2(t, k)));
+        p.fwd(v[k], v[k + half], tw_at(st, mac_e2(t, k)), st);
       }
     }
     // Each thread rewrites the words it just read: no barrier needed.
@@ -1046,7 +1080,7 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
-        p.fwd(v[k], v[k + half], tw_at(st, mac_e3(t, k)));
+        p.fwd(v[k], v[k + half], tw_at(st, mac_e3(t, k)), st);
       }
     }
 #pragma unroll
@@ -1057,8 +1091,9 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
       } else {
         w0[k] = k0[mac_e3(t, k)];
         w1[k] = k1[mac_e3(t, k)];
-        wide_mac(wacc0[k], v[k], static_cast<uint64_t>(w0[k]));
-        wide_mac(wacc1[k], v[k], static_cast<uint64_t>(w1[k]));
+        const V y = p.settle(v[k]);
+        wide_mac(wacc0[k], y, static_cast<uint64_t>(w0[k]));
+        wide_mac(wacc1[k], y, static_cast<uint64_t>(w1[k]));
       }
     }
   }
@@ -1099,9 +1134,9 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
     }
   }
   if constexpr (kF64) {
-    mac_finish<false>(a, j, b, t, MacDest{r, 8 * t, 0u}, sh, tww, twp, facc0, facc1);
+    mac_finish<false, F64Fast>(a, j, b, t, MacDest{r, 8 * t, 0u}, sh, tww, twp, facc0, facc1);
   } else {
-    mac_finish<false>(a, j, b, t, MacDest{r, 8 * t, 0u}, sh, tww, twp, uacc0, uacc1);
+    mac_finish<false, P>(a, j, b, t, MacDest{r, 8 * t, 0u}, sh, tww, twp, uacc0, uacc1);
   }
 }
 
@@ -1133,7 +1168,11 @@ __global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(kSmal
       tiles_mac(F64Exact(row), a, g, j, b, lds);
     }
   } else {
-    tiles_mac(U64Fast(row), a, g, j, b, lds);
+    if (row.delta60) {
+      tiles_mac(U64Pm(row), a, g, j, b, lds);
+    } else {
+      tiles_mac(U64Fast(row), a, g, j, b, lds);
+    }
   }
 }
 
@@ -1172,13 +1211,13 @@ __device__ __forceinline__ void tiles_forward_store(const P& p, const KsArgs& a,
       const int st = 31 - __builtin_clz(idx + 1);
       const int64_t gi = (int64_t{1} << (s0 + st)) + (static_cast<int64_t>(r) << st) + (idx + 1 - (1 << st));
       tww[idx] = w_row[gi];
-      if constexpr (!kF64) twp[idx] = wp_row[gi];
+      if constexpr (P::kCompanion) twp[idx] = wp_row[gi];
     }
   }
   tile_sync();
   auto tw_at = [&](int st, int e) {
     const int slot = mac_tw_slot(st, e);
-    return p.tw_make(tww[slot], kF64 ? 0 : twp[slot]);
+    return p.tw_make(tww[slot], P::kCompanion ? twp[slot] : 0);
   };
   int64_t* slab = a.inter + di * a.lqp * n;
   int64_t* tile = slab + j * n + static_cast<int64_t>(r) * kTile;
@@ -1209,7 +1248,7 @@ __device__ __forceinline__ void tiles_forward_store(const P& p, const KsArgs& a,
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       if (k & half) continue;
-      p.fwd(v[k], v[k + half], tw_at(st, mac_e1(t, k)));
+      p.fwd(v[k], v[k + half], tw_at(st, mac_e1(t, k)), st);
     }
   }
   tile_sync();
@@ -1224,7 +1263,7 @@ __device__ __forceinline__ void tiles_forward_store(const P& p, const KsArgs& a,
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       if (k & half) continue;
-      p.fwd(v[k], v[k + half], tw_at(st, mac_e2(t, k)));
+      p.fwd(v[k], v[k + half], tw_at(st, mac_e2(t, k)), st);
     }
   }
 #pragma unroll
@@ -1238,7 +1277,7 @@ __device__ __forceinline__ void tiles_forward_store(const P& p, const KsArgs& a,
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       if (k & half) continue;
-      p.fwd(v[k], v[k + half], tw_at(st, mac_e3(t, k)));
+      p.fwd(v[k], v[k + half], tw_at(st, mac_e3(t, k)), st);
     }
   }
   if constexpr (kPacked) {
@@ -1246,7 +1285,7 @@ __device__ __forceinline__ void tiles_forward_store(const P& p, const KsArgs& a,
     for (int k = 0; k < 8; ++k) packed_store(pk, pidx + k, f64_to_u64(p.canon(v[k])));
   } else {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) tile[mac_e3(t, k)] = p.mid(v[k]);
+    for (int k = 0; k < 8; ++k) tile[mac_e3(t, k)] = p.mid(p.settle(v[k]));
   }
 }
 
@@ -1268,7 +1307,11 @@ __global__ __launch_bounds__(kMacBlock) void k_ks_tiles_fwd(KsArgs a, int64_t gr
       tiles_forward_store(F64Exact(row), a, g, j, di, lds);
     }
   } else {
-    tiles_forward_store(U64Fast(row), a, g, j, di, lds);
+    if (row.delta60) {
+      tiles_forward_store(U64Pm(row), a, g, j, di, lds);
+    } else {
+      tiles_forward_store(U64Fast(row), a, g, j, di, lds);
+    }
   }
 }
 
@@ -1362,7 +1405,7 @@ __device__ __forceinline__ void tiles_mac_hoisted(const P& p, const KsArgs& a, i
     mac_digit(wb0, wb1, vb);
   }
   if constexpr (kF64) {
-    mac_finish<true>(a, j, b, t, dst, sh, tww, twp, facc0, facc1);
+    mac_finish<true, F64Fast>(a, j, b, t, dst, sh, tww, twp, facc0, facc1);
   } else {
     // at most 16 products y w with y < 4q, w < 2q: REDC value below 9q
 #pragma unroll
@@ -1370,7 +1413,7 @@ __device__ __forceinline__ void tiles_mac_hoisted(const P& p, const KsArgs& a, i
       uacc0[k] = wide_redc62(wacc0[k], row.q, row.neg_qinv64);
       uacc1[k] = wide_redc62(wacc1[k], row.q, row.neg_qinv64);
     }
-    mac_finish<true>(a, j, b, t, dst, sh, tww, twp, uacc0, uacc1);
+    mac_finish<true, P>(a, j, b, t, dst, sh, tww, twp, uacc0, uacc1);
   }
 }
 
@@ -1396,7 +1439,11 @@ __global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(2))) 
       tiles_mac_hoisted(F64Exact(row), a, g, j, b, lds);
     }
   } else {
-    tiles_mac_hoisted(U64Fast(row), a, g, j, b, lds);
+    if (row.delta60) {
+      tiles_mac_hoisted(U64Pm(row), a, g, j, b, lds);
+    } else {
+      tiles_mac_hoisted(U64Fast(row), a, g, j, b, lds);
+    }
   }
 }
 
@@ -1448,13 +1495,13 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
       const int st = 31 - __builtin_clz(idx + 1);
       const int64_t gi = (int64_t{1} << (s0 + st)) + (static_cast<int64_t>(r) << st) + (idx + 1 - (1 << st));
       tww[idx] = w_row[gi];
-      if constexpr (!kF64) twp[idx] = wp_row[gi];
+      if constexpr (P::kCompanion) twp[idx] = wp_row[gi];
     }
   }
   tile_sync();
   auto tw_at = [&](int st, int e) {
     const int slot = mac_tw_slot(st, e);
-    return p.tw_make(tww[slot], kF64 ? 0 : twp[slot]);
+    return p.tw_make(tww[slot], P::kCompanion ? twp[slot] : 0);
   };
   const int64_t tile_off = static_cast<int64_t>(r) * kTile;
   const int64_t comp_stride = a.batch * a.limbs * n;
@@ -1471,7 +1518,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
-        p.fwd(v[k], v[k + half], tw_at(st, mac_e1(t, k)));
+        p.fwd(v[k], v[k + half], tw_at(st, mac_e1(t, k)), st);
       }
     }
     tile_sync();  // earlier readers of the exchange buffer are done
@@ -1486,7 +1533,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
-        p.fwd(v[k], v[k + half], tw_at(st, mac_e2(t, k)));
+        p.fwd(v[k], v[k + half], tw_at(st, mac_e2(t, k)), st);
       }
     }
 #pragma unroll
@@ -1500,7 +1547,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
-        p.fwd(v[k], v[k + half], tw_at(st, mac_e3(t, k)));
+        p.fwd(v[k], v[k + half], tw_at(st, mac_e3(t, k)), st);
       }
     }
   };
@@ -1525,6 +1572,9 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
       // result (sums below 32 q^2: REDC value below 3q)
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
+        x0[k] = p.settle(x0[k]);
+        x1[k] = p.settle(x1[k]);
+        y[k] = p.settle(y[k]);
         WideAcc w0{0, 0, 0};
         wide_mac(w0, x0[k], y[k]);
         d0[k] = wide_redc62(w0, row.q, row.neg_qinv64);
@@ -1543,6 +1593,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
     } else {
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
+        y[k] = p.settle(y[k]);
         wide_mac(w1[k], x0[k], y[k]);
         d1[k] = wide_redc62(w1[k], row.q, row.neg_qinv64);
         WideAcc w2{0, 0, 0};
@@ -1561,7 +1612,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
       const int gg = idx - (kTile - (kTile >> st));
       const int64_t gi = (n >> (st + 1)) + (static_cast<int64_t>(r) << (7 - st)) + gg;
       tww[idx] = w_row[gi];
-      if constexpr (!kF64) twp[idx] = wp_row[gi];
+      if constexpr (P::kCompanion) twp[idx] = wp_row[gi];
     }
   }
   tile_sync();
@@ -1574,7 +1625,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e3(t, k));
-        p.inv(v[k], v[k + half], p.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
+        p.inv(v[k], v[k + half], p.tw_make(tww[slot], P::kCompanion ? twp[slot] : 0), st);
       }
     }
 #pragma unroll
@@ -1589,7 +1640,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e2(t, k));
-        p.inv(v[k], v[k + half], p.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
+        p.inv(v[k], v[k + half], p.tw_make(tww[slot], P::kCompanion ? twp[slot] : 0), st);
       }
     }
 #pragma unroll
@@ -1604,7 +1655,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
       for (int k = 0; k < 8; ++k) {
         if (k & half) continue;
         const int slot = inv_slot(st, mac_e1(t, k));
-        p.inv(v[k], v[k + half], p.tw_make(tww[slot], kF64 ? 0 : twp[slot]), st);
+        p.inv(v[k], v[k + half], p.tw_make(tww[slot], P::kCompanion ? twp[slot] : 0), st);
       }
     }
 #pragma unroll
@@ -1643,7 +1694,11 @@ __global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(kSmal
   if constexpr (kSmall) {
     tiles_hmult<kNttD01>(F64Fast(row), a, g, j, b, lds);
   } else {
-    tiles_hmult<kNttD01>(U64Fast(row), a, g, j, b, lds);
+    if (row.delta60) {
+      tiles_hmult<kNttD01>(U64Pm(row), a, g, j, b, lds);
+    } else {
+      tiles_hmult<kNttD01>(U64Fast(row), a, g, j, b, lds);
+    }
   }
 }
 

@@ -82,7 +82,7 @@ __device__ __forceinline__ void fwd_columns(const P& p, int64_t* base, const int
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & half) continue;
-      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << a) + (k >> (4 - a))));
+      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << a) + (k >> (4 - a))), a);
     }
   }
   if constexpr (S1 > 4) {
@@ -98,7 +98,7 @@ __device__ __forceinline__ void fwd_columns(const P& p, int64_t* base, const int
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
         if (k & half) continue;
-        p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << s) + ((16 * t + k) >> (S1 - s))));
+        p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << s) + ((16 * t + k) >> (S1 - s))), s);
       }
     }
 #pragma unroll
@@ -130,7 +130,7 @@ __device__ __forceinline__ void fwd_tiles(const P& p, int log_n, int g, int64_t*
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & half) continue;
-      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << (s0 + a)) + (r << a) + (k >> (4 - a))));
+      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << (s0 + a)) + (r << a) + (k >> (4 - a))), a);
     }
   }
 #pragma unroll
@@ -145,7 +145,7 @@ __device__ __forceinline__ void fwd_tiles(const P& p, int log_n, int g, int64_t*
     for (int k = 0; k < 16; ++k) {
       if (k & half) continue;
       p.fwd(v[k], v[k + half],
-            p.tw(tw, twp, (1 << (s0 + 4 + a)) + (r << (4 + a)) + (t << a) + (k >> (4 - a))));
+            p.tw(tw, twp, (1 << (s0 + 4 + a)) + (r << (4 + a)) + (t << a) + (k >> (4 - a))), a + 4);
     }
   }
   // Convert, then transpose back through LDS so the stores are coalesced.
@@ -169,6 +169,12 @@ __device__ __forceinline__ uint64_t ntt_product(const U64Fast& p, uint64_t x, in
   // x < 4q, w < 2q: the REDC value is below 2q, inside wide_redc62's range
   WideAcc acc{0, 0, 0};
   wide_mac(acc, x, static_cast<uint64_t>(w));
+  return wide_redc62(acc, p.q, p.row->neg_qinv64);
+}
+
+__device__ __forceinline__ uint64_t ntt_product(const U64Pm& p, uint64_t x, int64_t w) {
+  WideAcc acc{0, 0, 0};
+  wide_mac(acc, p.settle(x), static_cast<uint64_t>(w));
   return wide_redc62(acc, p.q, p.row->neg_qinv64);
 }
 
@@ -199,7 +205,7 @@ __device__ __forceinline__ void product_tiles(const P& p, int log_n, int g, int6
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & half) continue;
-      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << (s0 + a)) + (r << a) + (k >> (4 - a))));
+      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << (s0 + a)) + (r << a) + (k >> (4 - a))), a);
     }
   }
 #pragma unroll
@@ -214,7 +220,7 @@ __device__ __forceinline__ void product_tiles(const P& p, int log_n, int g, int6
     for (int k = 0; k < 16; ++k) {
       if (k & half) continue;
       p.fwd(v[k], v[k + half],
-            p.tw(tw, twp, (1 << (s0 + 4 + a)) + (r << (4 + a)) + (t << a) + (k >> (4 - a))));
+            p.tw(tw, twp, (1 << (s0 + 4 + a)) + (r << (4 + a)) + (t << a) + (k >> (4 - a))), a + 4);
     }
   }
 #pragma unroll
@@ -437,7 +443,10 @@ enum Mode : int { kExact = 0, kFast = 1 };
         CALL;                                              \
       }                                                    \
     } else {                                               \
-      if (MODE == kFast) {                                 \
+      if (MODE == kFast && (ROW).delta60) {                \
+        U64Pm p(ROW);                                      \
+        CALL;                                              \
+      } else if (MODE == kFast) {                          \
         U64Fast p(ROW);                                    \
         CALL;                                              \
       } else {                                             \
@@ -546,6 +555,8 @@ __global__ __launch_bounds__(kBlock) void k_product_tiles(NttArgs a, const int64
   const int g = static_cast<int>(blockIdx.x);
   if (rr.row->small) {
     product_tiles(F64Fast(*rr.row), a.log_n, g, rr.base, rr.tw, rr.twp, itw + off, itwp + off, w, lds);
+  } else if (rr.row->delta60) {
+    product_tiles(U64Pm(*rr.row), a.log_n, g, rr.base, rr.tw, rr.twp, itw + off, itwp + off, w, lds);
   } else {
     product_tiles(U64Fast(*rr.row), a.log_n, g, rr.base, rr.tw, rr.twp, itw + off, itwp + off, w, lds);
   }
@@ -578,7 +589,7 @@ __device__ __forceinline__ void stage_body(const P& p, int64_t* base, const int6
   V u = p.in(base[j]);
   V l = p.in(base[j + half]);
   if (forward) {
-    p.fwd(u, l, p.tw(tw, twp, idx));
+    p.fwd(u, l, p.tw(tw, twp, idx), 0);
   } else {
     p.inv(u, l, p.tw(tw, twp, idx), 0);
   }
@@ -803,6 +814,8 @@ __global__ void k_prepare_rows(ParamView params, int64_t limbs, NttRow* rows) {
   r.to_mont_p = shoup_companion(r.to_mont, m.q);
   r.ninv_mont_p = shoup_companion(r.ninv_mont, m.q);
   r.ninv_std_p = shoup_companion(r.ninv_std, m.q);
+  const uint64_t delta = (uint64_t{1} << 60) - m.q;
+  r.delta60 = m.q < (uint64_t{1} << 60) && delta < (uint64_t{1} << 26) ? delta : 0;
   // k = -q^{-1} mod 2^62 lifts by one Newton step: q k (2 + q k) = -1 mod 2^124
   r.neg_qinv64 = m.k * (2 + m.q * m.k);
   rows[l] = r;

@@ -58,13 +58,14 @@ __device__ __forceinline__ int64_t center_canonical(int64_t r, uint64_t q) {
 //   mid/unmid        working value <-> 64-bit intermediate between passes
 //   out_fwd(v)       final forward value -> int64 residue
 //   out_inv(v, f)    N^{-1} scaling and representation f -> int64 residue
-//   fwd/inv          butterflies (inv is told its stage within the pass, a
-//                    compile-time constant after unrolling); mul_const for
-//                    to-Montgomery scaling.
+//   settle(v)        forward output as an operand of the exact product sums
+//   fwd/inv          butterflies, told their stage within the pass (a
+//                    compile-time constant after unrolling).
 // ---------------------------------------------------------------------------
 
 // Exact binary64 path (q < 2^42): reference lazy semantics, see fh_common.h.
 struct F64Exact {
+  static constexpr bool kCompanion = false;  // twiddles carry a Shoup companion
   using V = double;
   struct Tw {
     double w;
@@ -84,6 +85,7 @@ struct F64Exact {
   __device__ __forceinline__ V in(int64_t raw) const { return u64_to_f64(static_cast<uint64_t>(raw)); }
   __device__ __forceinline__ int64_t mid(V v) const { return __double_as_longlong(v); }
   __device__ __forceinline__ V unmid(int64_t b) const { return __longlong_as_double(b); }
+  __device__ __forceinline__ V settle(V v) const { return v; }
   __device__ __forceinline__ V mul(Tw w, V x) const { return f64_mulmod(w.w, x, q, qinv); }
   __device__ __forceinline__ V add(V a, V b) const {
     const V s = a + b;
@@ -93,7 +95,7 @@ struct F64Exact {
     const V d = (a + twoq) - b;
     return d >= twoq ? d - twoq : d;
   }
-  __device__ __forceinline__ void fwd(V& u, V& l, Tw w) const {
+  __device__ __forceinline__ void fwd(V& u, V& l, Tw w, int) const {
     const V v = mul(w, l);
     const V e = add(u, v);
     l = sub(u, v);
@@ -120,6 +122,7 @@ struct F64Exact {
 // Fast binary64 path (q < 2^42): signed values, products reduced to
 // (-0.52q, 0.52q) without the final correction.
 struct F64Fast {
+  static constexpr bool kCompanion = false;  // twiddles carry a Shoup companion
   using V = double;
   using Tw = F64Exact::Tw;
   double q, qinv;
@@ -135,6 +138,7 @@ struct F64Fast {
   __device__ __forceinline__ V in(int64_t raw) const { return u64_to_f64(static_cast<uint64_t>(raw)); }
   __device__ __forceinline__ int64_t mid(V v) const { return __double_as_longlong(v); }
   __device__ __forceinline__ V unmid(int64_t b) const { return __longlong_as_double(b); }
+  __device__ __forceinline__ V settle(V v) const { return v; }
   // w*x - round(w*x/q) q, exact; |result| < 0.52 q for |x| < 2^45.
   __device__ __forceinline__ V mul(Tw w, V x) const { return f64_mulmod_signed(w.w, x, q, qinv); }
   // x - round(x/q) q, exact for |x| < 2^51; |result| <= q/2 (+ulp-level).
@@ -146,7 +150,7 @@ struct F64Fast {
     const V r = reduce(x);
     return r < 0.0 ? r + q : r;
   }
-  __device__ __forceinline__ void fwd(V& u, V& l, Tw w) const {
+  __device__ __forceinline__ void fwd(V& u, V& l, Tw w, int) const {
     const V v = mul(w, l);
     l = u - v;
     u = u + v;
@@ -176,6 +180,7 @@ struct F64Fast {
 
 // Integer Shoup path (any q < 2^62), reference lazy semantics (exact mode).
 struct U64Path {
+  static constexpr bool kCompanion = true;  // twiddles carry a Shoup companion
   using V = uint64_t;
   struct Tw {
     uint64_t w, wp;
@@ -193,11 +198,12 @@ struct U64Path {
   __device__ __forceinline__ V in(int64_t raw) const { return static_cast<uint64_t>(raw); }
   __device__ __forceinline__ int64_t mid(V v) const { return static_cast<int64_t>(v); }
   __device__ __forceinline__ V unmid(int64_t b) const { return static_cast<uint64_t>(b); }
+  __device__ __forceinline__ V settle(V v) const { return v; }
   __device__ __forceinline__ V mul(Tw w, V x) const { return shoup_mulmod(w.w, w.wp, x, q); }
   __device__ __forceinline__ V add(V a, V b) const { return csub(a + b, twoq); }
   // a + 2q - b with 2q - b = (2q + 1) + ~b (no carry chain)
   __device__ __forceinline__ V sub(V a, V b) const { return csub(a + (twoq + 1u) + ~b, twoq); }
-  __device__ __forceinline__ void fwd(V& u, V& l, Tw w) const {
+  __device__ __forceinline__ void fwd(V& u, V& l, Tw w, int) const {
     const V v = mul(w, l);
     const V e = add(u, v);
     l = sub(u, v);
@@ -227,6 +233,7 @@ struct U64Path {
 // forward and inverse outputs are canonical, so they equal the reference's
 // values modulo q exactly as U64Path's do.
 struct U64Fast {
+  static constexpr bool kCompanion = true;  // twiddles carry a Shoup companion
   using V = uint64_t;
   struct Tw {
     uint64_t w, wp;
@@ -244,6 +251,7 @@ struct U64Fast {
   __device__ __forceinline__ V in(int64_t raw) const { return static_cast<uint64_t>(raw); }
   __device__ __forceinline__ int64_t mid(V v) const { return static_cast<int64_t>(v); }
   __device__ __forceinline__ V unmid(int64_t b) const { return static_cast<uint64_t>(b); }
+  __device__ __forceinline__ V settle(V v) const { return v; }
   // w x - t q with t = hi64(w' x), formed as w x + t (2^64 - q): in [0, 2q)
   __device__ __forceinline__ V mul_lazy(Tw w, V x) const {
     const uint64_t t = __umul64hi(w.wp, x);
@@ -252,7 +260,7 @@ struct U64Fast {
   __device__ __forceinline__ V mul(Tw w, V x) const { return csub(mul_lazy(w, x), q); }
   // [0, 4q) -> [0, 2q)
   __device__ __forceinline__ V half(V v) const { return csub(v, twoq); }
-  __device__ __forceinline__ void fwd(V& u, V& l, Tw w) const {
+  __device__ __forceinline__ void fwd(V& u, V& l, Tw w, int) const {
     const V a = half(u);
     const V v = mul_lazy(w, l);
     u = a + v;
@@ -271,6 +279,89 @@ struct U64Fast {
     const Tw c = form == kOutMontgomery ? konst(row->ninv_mont, row->ninv_mont_p)
                                         : konst(row->ninv_std, row->ninv_std_p);
     int64_t r = static_cast<int64_t>(mul(c, v));
+    return form == kOutCentered ? center_canonical(r, q) : r;
+  }
+};
+
+// Integer path for fast arithmetic on primes q = 2^60 - delta, delta < 2^26
+// (every 60-bit prime of the shipped chains): 2^60 = delta mod q, so a
+// 128-bit product folds with two narrow multiplications.  One product takes
+// 7 32-bit multiplies and no companion word, against 10 for the Shoup product
+// of U64Fast, and a fold reduces a whole 64-bit word in one multiply, so
+// forward sums are folded once in four stages instead of once per butterfly.
+// On the five 60-bit rows of a 16-entry key switch at 33 Q rows (logN = 16):
+// tile pass and MAC 329 -> 282 us, ModUp (whose digit products sum exactly
+// before one fold) 339 -> 297 us, both bound by the multiply rate.
+// In units of 2^60: products are below 2.3, forward values below 13.1 (1.1
+// after a fold, a stage adds at most 3), inverse values below 2.3 (sums
+// folded each stage).
+struct U64Pm {
+  static constexpr bool kCompanion = false;
+  using V = uint64_t;
+  struct Tw {
+    uint64_t w;
+    uint32_t w1s;  // 16 (w >> 32)
+  };
+  __device__ __forceinline__ static Tw make(uint64_t w) { return Tw{w, static_cast<uint32_t>(w >> 32) << 4}; }
+  uint64_t q, threeq;
+  uint32_t delta;
+  const NttRow* row;
+  __device__ __forceinline__ explicit U64Pm(const NttRow& r)
+      : q(r.q), threeq(3 * r.q), delta(static_cast<uint32_t>(r.delta60)), row(&r) {}
+  __device__ __forceinline__ Tw tw(const int64_t* w, const int64_t*, int64_t idx) const {
+    return make(static_cast<uint64_t>(w[idx]));
+  }
+  __device__ __forceinline__ Tw tw_make(int64_t w, int64_t) const { return make(static_cast<uint64_t>(w)); }
+  __device__ __forceinline__ Tw konst(uint64_t c, uint64_t) const { return make(c); }
+  __device__ __forceinline__ V in(int64_t raw) const { return static_cast<uint64_t>(raw); }
+  __device__ __forceinline__ int64_t mid(V v) const { return static_cast<int64_t>(v); }
+  __device__ __forceinline__ V unmid(int64_t b) const { return static_cast<uint64_t>(b); }
+  // h 2^60 + l (l < 2^60) -> a word below 2.3 2^60 of the same residue: with
+  // g = (h >> 32) delta, h 2^60 = (h mod 2^32) delta + g 2^32, and
+  // g 2^32 = (g mod 2^28) 2^32 + (g >> 28) delta.
+  __device__ __forceinline__ V fold(uint64_t h, uint64_t l) const {
+    const uint64_t a = opaque(static_cast<uint64_t>(static_cast<uint32_t>(h)) * delta + l);
+    const uint64_t g = opaque(static_cast<uint64_t>(static_cast<uint32_t>(h >> 32)) * delta);
+    const uint32_t b1 = static_cast<uint32_t>(a >> 32) + (static_cast<uint32_t>(g) & 0xfffffffu);
+    const uint64_t b = static_cast<uint64_t>(b1) << 32 | static_cast<uint32_t>(a);
+    return opaque(static_cast<uint64_t>(static_cast<uint32_t>(g >> 28)) * delta + b);
+  }
+  // x below 14.5 2^60 (the middle sum then fits 64 bits), w below 2^60
+  __device__ __forceinline__ V mul(Tw w, V x) const {
+    const uint32_t w0 = static_cast<uint32_t>(w.w), w1 = static_cast<uint32_t>(w.w >> 32);
+    const uint32_t x0 = static_cast<uint32_t>(x), x1 = static_cast<uint32_t>(x >> 32);
+    // (opaque: one multiply-add each; reassociated, they need extra additions)
+    const uint64_t t = opaque(static_cast<uint64_t>(x0) * w0);
+    const uint64_t m0 = opaque(static_cast<uint64_t>(x0) * w1 + (t >> 32));
+    const uint64_t m = opaque(static_cast<uint64_t>(x1) * w0 + m0);
+    const uint64_t h = opaque(static_cast<uint64_t>(x1) * w.w1s + (m >> 28));
+    return fold(h, static_cast<uint64_t>(static_cast<uint32_t>(m) & 0xfffffffu) << 32 | static_cast<uint32_t>(t));
+  }
+  // any word -> below 2^60 + 2^30, the same residue
+  __device__ __forceinline__ V settle(V v) const {
+    return static_cast<uint64_t>(static_cast<uint32_t>(v >> 60)) * delta + (v & 0x0fffffffffffffffull);
+  }
+  __device__ __forceinline__ V canon(V v) const { return csub(settle(v), q); }
+  // an exact sum of products below 2^124 -> below 2.3 2^60
+  __device__ __forceinline__ V reduce(const WideAcc& s) const {
+    return fold(s.c2 << 4 | s.c1 >> 28, static_cast<uint64_t>(s.c1 & 0xfffffffu) << 32 | s.c0);
+  }
+  __device__ __forceinline__ void fwd(V& u, V& l, Tw w, int stage) const {
+    const V a = (stage & 3) == 0 ? settle(u) : u;
+    const V v = mul(w, l);
+    u = a + v;
+    l = opaque(a + (threeq + 1u)) + ~v;  // a - v + 3q without a borrow chain
+  }
+  __device__ __forceinline__ void inv(V& u, V& l, Tw w, int) const {
+    const V d = opaque(u + (threeq + 1u)) + ~l;
+    u = settle(u + l);
+    l = mul(w, d);
+  }
+  __device__ __forceinline__ V to_mont(V x) const { return mul(konst(row->to_mont, 0), x); }
+  __device__ __forceinline__ int64_t out_fwd(V v) const { return static_cast<int64_t>(canon(v)); }
+  __device__ __forceinline__ int64_t out_inv(V v, int form) const {
+    const Tw c = konst(form == kOutMontgomery ? row->ninv_mont : row->ninv_std, 0);
+    const int64_t r = static_cast<int64_t>(canon(mul(c, v)));
     return form == kOutCentered ? center_canonical(r, q) : r;
   }
 };

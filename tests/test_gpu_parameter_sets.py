@@ -67,3 +67,29 @@ def test_product_and_hoisted_rotation_match_composition(eng, offset):
         assert torch.equal(hoisted, eng.rotate_hoisted(one, [1, 5]).data)
     finally:
         eng.fused_keyswitch = True
+
+
+@pytest.mark.parametrize("log_n", [12, 13, 14, 15, 16])
+def test_fast_transforms_match_exact_on_extreme_residues(log_n):
+    """Both arithmetic modes of the NTT over every QP row (the 60-bit primes
+    take the 2^60 - delta folds in fast mode and Shoup products in exact
+    mode), on residues at the ends of their range."""
+
+    chain = "slots8192-scale50-levels5-int64" if log_n <= 14 else "slots32768-scale40-levels34-int64"
+    cfg = CkksConfig.from_preset(chain).with_ring_log(log_n)
+    fast, exact = CkksEngine(cfg, ntt_mode="fast", rng_seed=1), CkksEngine(cfg, ntt_mode="exact", rng_seed=1)
+    q = torch.tensor(cfg.moduli, dtype=torch.int64, device=fast.device)
+    uniform = Csprng(log_n, fast.device).uniform_mod(q, (), cfg.N)
+    top = (q - 1).unsqueeze(1).expand_as(uniform)
+    x = torch.stack([uniform, top, top * (torch.arange(cfg.N, device=q.device) % 2),
+                     top * (torch.arange(cfg.N, device=q.device) == 0)])
+    for name in ("forward_to_montgomery_", "forward_montgomery_"):
+        a, b = x.clone(), x.clone()
+        getattr(fast.runtime.ntt, name)(a, 0)
+        getattr(exact.runtime.ntt, name)(b, 0)
+        assert torch.equal(a, torch.remainder(b, q.unsqueeze(1)))
+    for name in ("inverse_montgomery_", "inverse_to_standard_", "inverse_to_centered_"):
+        a, b = x.clone(), x.clone()
+        getattr(fast.runtime.ntt, name)(a, 0)
+        getattr(exact.runtime.ntt, name)(b, 0)
+        assert torch.equal(a, b)
