@@ -645,6 +645,29 @@ __device__ __forceinline__ void modup_columns_x2(const KsArgs& a, const KsDigit&
   }
 }
 
+// One block of the integer rows' basis extension and column pass: the digit
+// width is uniform over the block, and a fixed-width body lets every digit
+// load issue before the extension arithmetic.
+template <int S1>
+__device__ __forceinline__ void modup_integer_block(const KsArgs& a, const NttRow& row, const KsDigit& d, int64_t di,
+                                                    int64_t b, int64_t j, int cg, int64_t* lds) {
+  if (row.delta60) {
+    switch (static_cast<int>(d.rows)) {
+      case 1: modup_columns<S1, 1>(U64Pm(row), a, d, di, b, j, cg, lds); break;
+      case 2: modup_columns<S1, 2>(U64Pm(row), a, d, di, b, j, cg, lds); break;
+      case 3: modup_columns<S1, 3>(U64Pm(row), a, d, di, b, j, cg, lds); break;
+      case 4: modup_columns<S1, 4>(U64Pm(row), a, d, di, b, j, cg, lds); break;
+      default: modup_columns<S1, 0>(U64Pm(row), a, d, di, b, j, cg, lds); break;
+    }
+    return;
+  }
+  switch (static_cast<int>(d.rows)) {
+    case 1: modup_columns<S1, 1>(U64Fast(row), a, d, di, b, j, cg, lds); break;
+    case 2: modup_columns<S1, 2>(U64Fast(row), a, d, di, b, j, cg, lds); break;
+    default: modup_columns<S1, 0>(U64Fast(row), a, d, di, b, j, cg, lds); break;
+  }
+}
+
 // One launch per arithmetic path, as for the tile pass below.
 template <int S1, int MODE, bool kSmall>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSmall && MODE == 0 ? 2 : 4))) void k_ks_modup_columns(KsArgs a, int64_t j_begin, int64_t j_count) {
@@ -668,8 +691,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSmall &
     const KsDigit& d = a.dig[di];
     const int64_t j = j_begin + 2 * static_cast<int64_t>(jp);
     const bool two = 2 * jp + 1 < jc;
-    // the digit width is uniform over the block: a fixed-width body lets
-    // every digit load issue before the extension arithmetic
     switch (static_cast<int>(d.rows)) {
       case 1: modup_columns_x2<S1, 1>(a, d, di, b, j, two, cg, lds); break;
       case 2: modup_columns_x2<S1, 2>(a, d, di, b, j, two, cg, lds); break;
@@ -690,21 +711,33 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSmall &
   if constexpr (kSmall) {
     modup_columns<S1, 0>(F64Exact(row), a, d, di, b, j, cg, lds);
   } else {
-    if (row.delta60) {
-      switch (static_cast<int>(d.rows)) {
-        case 1: modup_columns<S1, 1>(U64Pm(row), a, d, di, b, j, cg, lds); break;
-        case 2: modup_columns<S1, 2>(U64Pm(row), a, d, di, b, j, cg, lds); break;
-        case 3: modup_columns<S1, 3>(U64Pm(row), a, d, di, b, j, cg, lds); break;
-        case 4: modup_columns<S1, 4>(U64Pm(row), a, d, di, b, j, cg, lds); break;
-        default: modup_columns<S1, 0>(U64Pm(row), a, d, di, b, j, cg, lds); break;
-      }
-      return;
-    }
+    modup_integer_block<S1>(a, row, d, di, b, j, cg, lds);
+  }
+}
+
+// Calls too small to fill the GPU (small_call): both arithmetic paths in one
+// launch, one destination row per block, the longer integer rows first.
+template <int S1>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_ks_modup_small(KsArgs a) {
+  __shared__ int64_t lds[(1 << S1) * (kBlock / ((1 << S1) / 16) + 1)];
+  constexpr uint32_t kGroups = (1u << S1) / 16;
+  const uint32_t items = kGroups * static_cast<uint32_t>(a.dnum * a.batch);  // per destination row
+  const int64_t j = a.lqp - 1 - blockIdx.x / items;
+  const uint32_t w = blockIdx.x % items;
+  const int cg = static_cast<int>(w % kGroups);
+  const uint32_t z = w / kGroups;
+  const int64_t b = z / static_cast<uint32_t>(a.dnum);
+  const int64_t di = z % static_cast<uint32_t>(a.dnum);
+  const KsDigit& d = a.dig[di];
+  const NttRow& row = a.rows[a.level + j];
+  if (j < a.small_rows) {
     switch (static_cast<int>(d.rows)) {
-      case 1: modup_columns<S1, 1>(U64Fast(row), a, d, di, b, j, cg, lds); break;
-      case 2: modup_columns<S1, 2>(U64Fast(row), a, d, di, b, j, cg, lds); break;
-      default: modup_columns<S1, 0>(U64Fast(row), a, d, di, b, j, cg, lds); break;
+      case 1: modup_columns<S1, 1>(F64Fast(row), a, d, di, b, j, cg, lds); break;
+      case 2: modup_columns<S1, 2>(F64Fast(row), a, d, di, b, j, cg, lds); break;
+      default: modup_columns<S1, 0>(F64Fast(row), a, d, di, b, j, cg, lds); break;
     }
+  } else {
+    modup_integer_block<S1>(a, row, d, di, b, j, cg, lds);
   }
 }
 
@@ -827,7 +860,7 @@ __device__ __forceinline__ MacDest hoisted_dest(const KsArgs& a, int r, int t, i
 // the rest of the inverse), then the working-format store the inverse column
 // pass reads.  With kHoist the sums arrive in source order and first move to
 // the destination layout through the exchange buffer.
-template <bool kHoist, class PI, class Acc>
+template <bool kHoist, bool kSplit, class PI, class Acc>
 __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b, int t, const MacDest& dst,
                                            int64_t* sh, int64_t* tww, int64_t* twp, Acc (&acc0)[8],
                                            Acc (&acc1)[8]) {
@@ -855,11 +888,19 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
     to_dst(acc0);
     to_dst(acc1);
   }
-  tile_sync();
+  // kSplit: the whole block has summed its waves' shares and stages the
+  // twiddles; wave 0 then finishes accumulator 0 and wave 1 accumulator 1.
+  const int wave = kSplit ? static_cast<int>(threadIdx.x) / 64 : 0;
+  const int waves = kSplit ? static_cast<int>(blockDim.x) / 64 : 1;
+  if constexpr (kSplit) {
+    __syncthreads();
+  } else {
+    tile_sync();
+  }
   {
     const int64_t* w_row = a.inv_w + grow * n;
     const int64_t* wp_row = a.inv_wp + grow * n;
-    for (int idx = t; idx < kTile - 1; idx += kMacThreads) {
+    for (int idx = wave * kMacThreads + t; idx < kTile - 1; idx += waves * kMacThreads) {
       // stage st owns slots [256 - 2^(8-st), 256 - 2^(7-st)); group g = e >> (st+1)
       const int st = 7 - (31 - __builtin_clz(kTile - 1 - idx));
       const int g = idx - (kTile - (kTile >> st));
@@ -868,7 +909,12 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
       if constexpr (PI::kCompanion) twp[idx] = wp_row[gi];
     }
   }
-  tile_sync();
+  if constexpr (kSplit) {
+    __syncthreads();
+    if (wave > 1) return;
+  } else {
+    tile_sync();
+  }
   auto inv_slot = [](int st, int e) { return (kTile - (kTile >> st)) + (e >> (st + 1)); };
   const PI pi(row);
   auto inverse_tile = [&](auto (&v)[8], auto store) {
@@ -918,28 +964,36 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
 #pragma unroll
     for (int k = 0; k < 8; ++k) store(mac_e1(t, k), v[k]);
     // the exchange buffer is reused by the next accumulator
-    __syncthreads();
+    if constexpr (!kSplit) __syncthreads();
   };
-  if constexpr (kF64) {
-    // binary64 rows of the accumulators travel packed (canonical, 6 bytes)
-    const PackedInter pk0 = packed_slab(a.acc + (0 * a.batch + b) * a.lqp * n, a.small_rows, n);
-    const PackedInter pk1 = packed_slab(a.acc + (1 * a.batch + b) * a.lqp * n, a.small_rows, n);
-    const int64_t row_off = j * n;
-    inverse_tile(acc0, [&](int e, double x) {
-      packed_store(pk0, row_off + packed_index(r_dst, e), f64_to_u64(pi.canon(x)));
-    });
-    inverse_tile(acc1, [&](int e, double x) {
-      packed_store(pk1, row_off + packed_index(r_dst, e), f64_to_u64(pi.canon(x)));
-    });
+  auto finish_one = [&](Acc (&acc)[8], int64_t component) {
+    int64_t* slab = a.acc + (component * a.batch + b) * a.lqp * n;
+    if constexpr (kF64) {
+      // binary64 rows of the accumulators travel packed (canonical, 6 bytes)
+      const PackedInter pk = packed_slab(slab, a.small_rows, n);
+      inverse_tile(acc, [&](int e, double x) {
+        packed_store(pk, j * n + packed_index(r_dst, e), f64_to_u64(pi.canon(x)));
+      });
+    } else {
+      int64_t* out = slab + j * n + static_cast<int64_t>(r_dst) * kTile;
+      inverse_tile(acc, [&](int e, uint64_t x) { out[e] = static_cast<int64_t>(x); });
+    }
+  };
+  if constexpr (kSplit) {
+    if (wave == 1) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) acc0[k] = acc1[k];
+    }
+    finish_one(acc0, wave);
   } else {
-    int64_t* out0 = a.acc + ((0 * a.batch + b) * a.lqp + j) * n + static_cast<int64_t>(r_dst) * kTile;
-    int64_t* out1 = a.acc + ((1 * a.batch + b) * a.lqp + j) * n + static_cast<int64_t>(r_dst) * kTile;
-    inverse_tile(acc0, [&](int e, uint64_t x) { out0[e] = static_cast<int64_t>(x); });
-    inverse_tile(acc1, [&](int e, uint64_t x) { out1[e] = static_cast<int64_t>(x); });
+    finish_one(acc0, 0);
+    finish_one(acc1, 1);
   }
 }
 
-template <class P>
+// kSplit: the block's waves share two tiles, wave w takes digits w, w + W, ...
+// of both, and their sums join in LDS (k_ks_tiles_mac_split).
+template <bool kSplit, class P>
 __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g, int64_t j,
                                           int64_t b, int64_t* lds) {
   using V = typename P::V;
@@ -947,18 +1001,21 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
   const int64_t n = int64_t{1} << a.log_n;
   const int64_t grow = a.level + j;
   const NttRow& row = a.rows[grow];
-  const int m = threadIdx.x / kMacThreads;
+  constexpr int kTiles = kSplit ? 2 : kMacTiles;  // tiles per block
+  const int wave = kSplit ? static_cast<int>(threadIdx.x) / 64 : 0;
+  const int waves = kSplit ? static_cast<int>(blockDim.x) / 64 : 1;
+  const int m = (kSplit ? threadIdx.x % 64 : threadIdx.x) / kMacThreads;
   const int t = threadIdx.x % kMacThreads;
-  const int r = static_cast<int>(g) * kMacTiles + m;
+  const int r = static_cast<int>(g) * kTiles + m;
   const int s0 = a.log_n - kTileLog;
-  int64_t* sh = lds + m * kTilePitch;
-  int64_t* tww = lds + kMacExchange + m * kTile;
-  int64_t* twp = tww + kMacTiles * kTile;  // integer rows only
-  int64_t* key_digit = lds + kMacExchange + kMacTiles * kTile * (kF64 ? 1 : 2);
+  int64_t* sh = lds + (threadIdx.x / kMacThreads) * kTilePitch;
+  int64_t* tww = lds + (kSplit ? waves * 2 * kTilePitch : kMacExchange) + m * kTile;
+  int64_t* twp = tww + kTiles * kTile;  // Shoup companions
+  int64_t* key_digit = tww + (kTiles * (P::kCompanion ? 2 : 1) - m) * kTile;
   {
     const int64_t* w_row = a.fwd_w + grow * n;
     const int64_t* wp_row = a.fwd_wp + grow * n;
-    for (int idx = t; idx < kTile - 1; idx += kMacThreads) {
+    for (int idx = wave * kMacThreads + t; idx < kTile - 1; idx += waves * kMacThreads) {
       const int st = 31 - __builtin_clz(idx + 1);
       const int64_t gi = (int64_t{1} << (s0 + st)) + (static_cast<int64_t>(r) << st) + (idx + 1 - (1 << st));
       tww[idx] = w_row[gi];
@@ -981,8 +1038,8 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
     facc0[k] = facc1[k] = 0.0;
     wacc0[k] = wacc1[k] = WideAcc{0, 0, 0};
   }
-  const int64_t* tile = a.inter + ((b * a.dnum) * a.lqp + j) * n + tile_off;
-  const int64_t digit_stride = a.lqp * n;
+  const int64_t* tile = a.inter + ((b * a.dnum + wave) * a.lqp + j) * n + tile_off;
+  const int64_t digit_stride = a.lqp * n * waves;  // to this wave's next digit
   // Binary64 rows: software pipeline over the digits -- the next digit's
   // packed values (one 32-byte and one 16-byte load: coefficients 8t..8t+7
   // are contiguous in the packed block layout) load while this digit's
@@ -997,13 +1054,13 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
   uint4 nl0{}, nl1{}, nhh{};
   int64_t nv[8];  // other rows: the next digit's values, likewise
   if constexpr (std::is_same<P, F64Fast>::value) {
-    load_packed(0, nl0, nl1, nhh);
+    load_packed(wave, nl0, nl1, nhh);
   } else {
 #pragma unroll
     for (int k = 0; k < 8; ++k) nv[k] = tile[mac_e1(t, k)];
   }
 #pragma nounroll
-  for (int64_t di = 0; di < a.dnum; ++di, tile += digit_stride) {
+  for (int64_t di = wave; di < a.dnum; di += waves, tile += digit_stride) {
     Global<int64_t>* k0 = key + key_digit[di] * a.key_sd + grow * a.key_sr + tile_off;
     Global<int64_t>* k1 = k0 + a.key_sc;
     V v[8];
@@ -1011,7 +1068,7 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
     if constexpr (std::is_same<P, F64Fast>::value) {
       // an LDS pass moves the values to the round-1 ownership
       const uint4 l0 = nl0, l1 = nl1, hh = nhh;
-      if (di + 1 < a.dnum) load_packed(di + 1, nl0, nl1, nhh);
+      if (di + waves < a.dnum) load_packed(di + waves, nl0, nl1, nhh);
       const uint32_t lo[8] = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
       const uint32_t hi2[4] = {hh.x, hh.y, hh.z, hh.w};
       tile_sync();  // the previous digit's last reads of the exchange buffer are done
@@ -1026,7 +1083,7 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
     } else {
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[k] = p.unmid(nv[k]);
-      if (di + 1 < a.dnum) {
+      if (di + waves < a.dnum) {
 #pragma unroll
         for (int k = 0; k < 8; ++k) nv[k] = tile[digit_stride + mac_e1(t, k)];
       }
@@ -1101,7 +1158,7 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
   // scaling) join the Q rows' sums, so that ModDown's exact floor division
   // returns floor(X / P) + d directly.  Thread t holds coefficients 8t + k,
   // stored at tile positions t + 32k (the HMult front's seed layout).
-  if (a.seed0 != nullptr && j < a.lq) {
+  if (a.seed0 != nullptr && j < a.lq && wave == 0) {
     const int64_t off = (b * a.lq + j) * n + tile_off + t;
     if constexpr (kF64) {
       const double sc = static_cast<double>(a.seed_scale[grow]);
@@ -1133,10 +1190,45 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
       uacc1[k] = wide_redc62(wacc1[k], row.q, row.neg_qinv64);
     }
   }
+  const MacDest dst{r, 8 * t, 0u};
+  if constexpr (kSplit) {
+    // Wave c collects accumulator c of every wave (exchange buffers take the
+    // shares).  Binary64 shares add exactly (17 terms below 0.53q in all),
+    // integer shares are below 2q each, at most 8 of them.
+    auto collect = [&](auto (&acc)[8], int owner) {
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < 8; ++k) __builtin_memcpy(&sh[t + 32 * k], &acc[k], sizeof(int64_t));
+      __syncthreads();
+      if (wave == owner) {
+        for (int w = 0; w < waves; ++w) {
+          if (w == owner) continue;
+          const int64_t* share = lds + (2 * w + m) * kTilePitch;
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            V x;
+            __builtin_memcpy(&x, &share[t + 32 * k], sizeof(x));
+            acc[k] += x;
+          }
+        }
+        if constexpr (!kF64) {
+#pragma unroll
+          for (int k = 0; k < 8; ++k) acc[k] = csub(csub(csub(acc[k], 8 * row.q), 4 * row.q), 2 * row.q);
+        }
+      }
+    };
+    if constexpr (kF64) {
+      collect(facc0, 0);
+      collect(facc1, 1);
+    } else {
+      collect(uacc0, 0);
+      collect(uacc1, 1);
+    }
+  }
   if constexpr (kF64) {
-    mac_finish<false, F64Fast>(a, j, b, t, MacDest{r, 8 * t, 0u}, sh, tww, twp, facc0, facc1);
+    mac_finish<false, kSplit, F64Fast>(a, j, b, t, dst, sh, tww, twp, facc0, facc1);
   } else {
-    mac_finish<false, P>(a, j, b, t, MacDest{r, 8 * t, 0u}, sh, tww, twp, uacc0, uacc1);
+    mac_finish<false, kSplit, P>(a, j, b, t, dst, sh, tww, twp, uacc0, uacc1);
   }
 }
 
@@ -1163,17 +1255,43 @@ __global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(kSmal
   const NttRow& row = a.rows[a.level + j];
   if constexpr (kSmall) {
     if constexpr (MODE == 1) {
-      tiles_mac(F64Fast(row), a, g, j, b, lds);
+      tiles_mac<false>(F64Fast(row), a, g, j, b, lds);
     } else {
-      tiles_mac(F64Exact(row), a, g, j, b, lds);
+      tiles_mac<false>(F64Exact(row), a, g, j, b, lds);
     }
   } else {
     if (row.delta60) {
-      tiles_mac(U64Pm(row), a, g, j, b, lds);
+      tiles_mac<false>(U64Pm(row), a, g, j, b, lds);
     } else {
-      tiles_mac(U64Fast(row), a, g, j, b, lds);
+      tiles_mac<false>(U64Fast(row), a, g, j, b, lds);
     }
   }
+}
+
+// Calls too small to fill the GPU (small_call): both arithmetic paths in one
+// launch of W-wave blocks, two tiles each, the digits dealt over the waves.
+// A tile's chain of digits (4-5 us each on the integer rows: load, eight
+// butterfly stages, products) is what such a call waits for, so W shortens it
+// W-fold for one exchange of sums.  Fast arithmetic.
+constexpr int kSplitWaves = 8;
+__global__ __launch_bounds__(kSplitWaves * 64) void k_ks_tiles_mac_split(KsArgs a) {
+  extern __shared__ int64_t lds_dynamic[];
+  const uint32_t pairs = static_cast<uint32_t>((int64_t{1} << a.log_n) / (2 * kTile));
+  const uint32_t batch = static_cast<uint32_t>(a.batch);
+  const int64_t b = blockIdx.x % batch;
+  const int64_t g = (blockIdx.x / batch) % pairs;
+  const int64_t j = a.lqp - 1 - blockIdx.x / (batch * pairs);
+  const NttRow& row = a.rows[a.level + j];
+  if (j < a.small_rows) {
+    tiles_mac<true>(F64Fast(row), a, g, j, b, lds_dynamic);
+  } else if (row.delta60) {
+    tiles_mac<true>(U64Pm(row), a, g, j, b, lds_dynamic);
+  } else {
+    tiles_mac<true>(U64Fast(row), a, g, j, b, lds_dynamic);
+  }
+}
+inline size_t mac_split_lds_bytes(int waves) {
+  return sizeof(int64_t) * (static_cast<size_t>(waves) * 2 * kTilePitch + 2 * 2 * kTile + kMacMaxDigits);
 }
 
 // ---------------------------------------------------------------------------
@@ -1405,7 +1523,7 @@ __device__ __forceinline__ void tiles_mac_hoisted(const P& p, const KsArgs& a, i
     mac_digit(wb0, wb1, vb);
   }
   if constexpr (kF64) {
-    mac_finish<true, F64Fast>(a, j, b, t, dst, sh, tww, twp, facc0, facc1);
+    mac_finish<true, false, F64Fast>(a, j, b, t, dst, sh, tww, twp, facc0, facc1);
   } else {
     // at most 16 products y w with y < 4q, w < 2q: REDC value below 9q
 #pragma unroll
@@ -1413,7 +1531,7 @@ __device__ __forceinline__ void tiles_mac_hoisted(const P& p, const KsArgs& a, i
       uacc0[k] = wide_redc62(wacc0[k], row.q, row.neg_qinv64);
       uacc1[k] = wide_redc62(wacc1[k], row.q, row.neg_qinv64);
     }
-    mac_finish<true, P>(a, j, b, t, dst, sh, tww, twp, uacc0, uacc1);
+    mac_finish<true, false, P>(a, j, b, t, dst, sh, tww, twp, uacc0, uacc1);
   }
 }
 
@@ -1713,7 +1831,7 @@ struct ModDownArgs {
   int64_t batch, lq, lqp, level, small_rows;
   int log_n;
   ParamView params;
-  KsDigit pdig;             // the P primes as one digit (extension over QP0 columns)
+  const KsDigit* pdig;      // the P primes as one digit (extension over QP0 columns), device memory
   const int64_t* p_inverse; // [Q0] P^{-1} mod q, standard
   const NttRow* rows;       // global QP NTT records
   View3 base0, base1, out0, out1;
@@ -1755,6 +1873,7 @@ __global__ __launch_bounds__(kBlock) void k_ks_gather_base(View3 base, const int
 template <int P>
 __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   constexpr int kRows = kModDownRowsPerThread;
+  const KsDigit& pdig = *a.pdig;
   const int64_t n = int64_t{1} << a.log_n;
   // XCD-contiguous work items: all coefficient chunks of one (accumulator,
   // entry, row group) run on one XCD (see k_ks_decompose).
@@ -1823,14 +1942,14 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   };
   // Mixed-radix digits of X mod P (X_P = sum_r c_r prod_{t<r} p_t), each
   // split as c_hi 2^30 + c_lo (both exact in binary64).
-  garner_p<P>(a.pdig, a.rows + a.level + a.lq, dg);
+  garner_p<P>(pdig, a.rows + a.level + a.lq, dg);
   double dlo[P], dhi[P];
 #pragma unroll
   for (int r = 0; r < P; ++r) {
     dlo[r] = static_cast<double>(static_cast<uint32_t>(dg[r] & ((int64_t{1} << 30) - 1)));
     dhi[r] = static_cast<double>(static_cast<uint32_t>(dg[r] >> 30));
   }
-  const int64_t pitch = a.pdig.f64_stride;
+  const int64_t pitch = pdig.f64_stride;
   // Final canonical addition of the base (add_canonical).
   auto with_base = [&](int64_t bval, int64_t value, int64_t twice_q) -> int64_t {
     if (!has_base) return value;
@@ -1873,7 +1992,7 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
     int64_t xp = mont_mul(dg[0], m.r2, m);
 #pragma unroll
     for (int r = 1; r < P; ++r)
-      xp = add_lazy(xp, mont_mul(dg[r], global(a.pdig.basis)[(r - 1) * a.pdig.basis_stride + grow], m), m.twice_q);
+      xp = add_lazy(xp, mont_mul(dg[r], global(pdig.basis)[(r - 1) * pdig.basis_stride + grow], m), m.twice_q);
     const int64_t xr = mont_mul(xval, m.r2, m);
     return with_base(bval, mont_mul(sub_lazy(xr, xp, m.twice_q), a.p_inverse[grow], m), m.twice_q);
   };
@@ -1886,7 +2005,7 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   int64_t round_up = 0;
   if (rescale) {
     if (f64_rows > 0) {
-      Global<double>* rec0 = global(a.pdig.f64_table) + a.level * pitch;
+      Global<double>* rec0 = global(pdig.f64_table) + a.level * pitch;
       c0 = add_base_f64(moddown_f64(rec0, packed_f64(xlo0, xhi0)), bv0, rec0[14]);
       c0_int = static_cast<int64_t>(f64_to_u64(c0));
     } else {
@@ -1898,7 +2017,7 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   for (int rr = 0; rr < kRows; ++rr) {
     const int64_t row = row_begin + rr;
     if (row >= f64_rows) break;
-    Global<double>* rec = global(a.pdig.f64_table) + (a.level + row) * pitch;
+    Global<double>* rec = global(pdig.f64_table) + (a.level + row) * pitch;
     const double q = rec[14];
     double v = add_base_f64(moddown_f64(rec, packed_f64(xlo[rr], xhi[rr])), bv[rr], q);
     if (rescale && row > 0) {
@@ -1941,6 +2060,18 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
     }
   }
 }
+
+// A call whose tile pass has at most this many pairs of tiles (rows x N / 512
+// x entries) takes the small-call launches.  Rotations, small-call launches
+// against the per-path ones on the same box: 52 against 99 us at 288 pairs
+// (one entry, logN = 14, level 0), 101 / 112 at 1216, 133 / 141 at 2432 and
+// 121 / 124 at 2816 pairs; 161 / 156 at 4224 and 199 / 183 at 5632 (one wave
+// does both of its tiles' digits there and the integer rows' register count
+// halves the binary64 rows' occupancy).
+constexpr int64_t kSmallCallPairs = 2816;
+// Waves of the split tile pass: two per SIMD (it holds two; four or eight per
+// SIMD measured the same or slower).
+constexpr int64_t kSplitTargetWaves = 2048;
 
 // The integer-row (60-bit prime) ModUp runs first on the caller's stream;
 // then the integer-row MAC runs on a side stream, forked from the caller's
@@ -2171,7 +2302,33 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
     FH_CHECK_LAUNCH("key switch tile pass + MAC");
     return kOk;
   };
-  if (!use_side_stream) {
+  // Few tiles: the digits are dealt over several waves and both arithmetic
+  // paths share their launches (no side stream, two launches fewer).
+  const int64_t tile_pairs = lqp * (n / (2 * kTile)) * batch;
+  const bool small_call = mode == 1 && !hoist && digit_count >= 2 && tile_pairs <= kSmallCallPairs;
+  if (small_call) {
+    const int64_t modup_blocks = (kTile / C) * lqp * digit_count * batch;
+#define FH_MODUP_SMALL_CASE(S) \
+  case S: hipLaunchKernelGGL(k_ks_modup_small<S>, dim3(static_cast<uint32_t>(modup_blocks)), dim3(kBlock), 0, s, a); break;
+    switch (s1) {
+      FH_MODUP_SMALL_CASE(4)
+      FH_MODUP_SMALL_CASE(5)
+      FH_MODUP_SMALL_CASE(6)
+      FH_MODUP_SMALL_CASE(7)
+      default:
+        FH_MODUP_SMALL_CASE(8)
+    }
+#undef FH_MODUP_SMALL_CASE
+    FH_CHECK_LAUNCH("key switch modup + column pass");
+    // waves per pair of tiles, the digits spread evenly over them
+    int64_t waves = kSplitTargetWaves / tile_pairs;
+    waves = waves < 2 ? 2 : (waves > kSplitWaves ? kSplitWaves : waves);
+    waves = waves > digit_count ? digit_count : waves;
+    waves = ceil_div(digit_count, ceil_div(digit_count, waves));
+    hipLaunchKernelGGL(k_ks_tiles_mac_split, dim3(static_cast<uint32_t>(tile_pairs)),
+                       dim3(static_cast<uint32_t>(64 * waves)), mac_split_lds_bytes(static_cast<int>(waves)), s, a);
+    FH_CHECK_LAUNCH("key switch tile pass + MAC");
+  } else if (!use_side_stream) {
     for (int pass = 0; pass < 2; ++pass) {
       int rc = launch_modup(pass, s);
       if (rc == kOk) rc = launch_mac(pass, s);
@@ -2229,7 +2386,7 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
   md.log_n = static_cast<int>(log_n);
   md.params = a.params;
   md.rows = static_cast<const NttRow*>(ntt_rows);
-  md.pdig = *reinterpret_cast<const KsDigit*>(p_digit_table);
+  md.pdig = reinterpret_cast<const KsDigit*>(p_digit_table);
   md.p_inverse = p_inverse_q;
   md.base0 = View3(base0);
   md.base1 = View3(base1);
