@@ -374,7 +374,7 @@ struct NttRow {
   uint64_t ninv_std_rinv_p;  // binary64 key MAC that skipped REDC's R^{-1})
   uint64_t neg_qinv64;       // -q^{-1} mod 2^64 (REDC with radix 2^64)
   uint64_t delta60;          // 2^60 - q when that is in [1, 2^26), else 0 (U64Pm)
-  uint64_t reserved;
+  uint64_t wide;             // 1: q in [2^42, 2^50 + 2^30), binary64 in fast arithmetic (F64Wide)
 };
 static_assert(sizeof(NttRow) == 128, "NttRow must stay 128 bytes");
 

@@ -71,7 +71,7 @@ struct KsDigit {
   const int64_t* basis;        // [D-1, QP0] M_r R^2 mod p_j, row-major
   int64_t basis_stride;        // QP0
   const int64_t* basis_std;    // [D-1, QP0] M_r R mod p_j
-  int64_t f64_ok;              // every source prime < 2^45: digits stored as binary64
+  int64_t f64_ok;              // digits stored as binary64: 1 every source prime < 2^45, 2 every one < kWidePrimeLimit
   const int64_t* basis_shoup;  // [D-1, QP0] Shoup companions of basis_std
   // P digit: [Q0, 16] binary64 ModDown records (f64_stride = 16).  A Q digit
   // with f64_ok and D > 1: its binary64 Garner record [D-1 normalizers,
@@ -104,7 +104,8 @@ struct KsArgs {
   int64_t key_sd, key_sc, key_sr;   // key strides (digit, component, row)
   const int64_t* gal_idx;   // per-entry int32 gather table addresses [B] or null
   const int64_t* gal_sign;  // per-entry int8 sign table addresses [B]
-  int64_t small_rows;       // leading QP rows on the binary64 path
+  int64_t small_rows;       // leading QP rows on the binary64 path (primes below 2^42)
+  int wide_apart;           // F64Wide rows have tile-pass launches of their own (no row below 2^42)
   // Optional accumulator seeds (null: none): [B, Lq, N] NTT-domain rows in
   // the accumulators' scaling, added to the Q rows times seed_scale[row].
   const int64_t* seed0;
@@ -183,9 +184,11 @@ __device__ __forceinline__ void garner(const KsDigit& d, int64_t* dg) {
 }
 
 // Garner digits with the digit count fixed at compile time (the same
-// recurrence as garner(); no runtime row loops).
+// recurrence as garner(); no runtime row loops, and a difference's residue
+// from its row's reciprocal instead of a division).  rows: the digit's NTT
+// records.
 template <int R>
-__device__ __forceinline__ void garner_fixed(const KsDigit& d, int64_t* dg) {
+__device__ __forceinline__ void garner_fixed(const KsDigit& d, const NttRow* rows, int64_t* dg) {
   const Mont m0 = digit_mont(d, 0);
   int64_t first = dg[0];
   first = first < static_cast<int64_t>(m0.q) ? first : first - static_cast<int64_t>(m0.q);
@@ -198,7 +201,8 @@ __device__ __forceinline__ void garner_fixed(const KsDigit& d, int64_t* dg) {
 #pragma unroll
   for (int row = 1; row < R; ++row) {
     const Mont mr = digit_mont(d, row);
-    const int64_t digit = mont_mul(canonical_operand(src[row] - dg[row], mr.q), global(d.normalizers)[row - 1], mr);
+    const int64_t digit = mont_mul(canonical_operand(src[row] - dg[row], mr.q, rows[row].qinv),
+                                   global(d.normalizers)[row - 1], mr);
     dg[row] = digit;
 #pragma unroll
     for (int t = row + 1; t < R; ++t) dg[t] += mont_mul(digit, global(d.propagation)[(row - 1) * R + t], digit_mont(d, t));
@@ -289,7 +293,7 @@ __device__ __forceinline__ void decompose_one(const KsArgs& a, const KsDigit& d,
   if constexpr (R == 0) {
     garner(d, dg);
   } else {
-    garner_fixed<R>(d, dg);
+    garner_fixed<R>(d, a.rows + a.level + d.row_begin, dg);
   }
   // Digits below 2^45 are stored as binary64 (exact), the form the ModUp
   // kernel multiplies in; the others stay integers.
@@ -375,7 +379,7 @@ __device__ __forceinline__ void modup_columns(const P& p, const KsArgs& a, const
   auto at = [&](int k) { return static_cast<uint32_t>((t + T * k) * kTile + col); };
   V v[16];
   if constexpr (std::is_same<V, double>::value) {
-    if (d.f64_ok) {
+    if (P::kWide ? d.f64_ok != 0 : d.f64_ok == 1) {
       // Binary64 digits times (M_r R mod q).  Exact arithmetic reproduces
       // the reference's canonical REDC terms and add_lazy chain; fast
       // arithmetic keeps the signed congruent sum (|x| < 2.1q), which the
@@ -385,7 +389,11 @@ __device__ __forceinline__ void modup_columns(const P& p, const KsArgs& a, const
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
         const double x = __longlong_as_double(dig0[at(k)]);
-        v[k] = std::is_same<P, F64Fast>::value ? f64_mulmod_signed(c0, x, q, qinv) : f64_mulmod(c0, x, q, qinv);
+        if constexpr (P::kWide) {
+          v[k] = p.product(c0, x);  // |sum| < 0.9q per row of the digit
+        } else {
+          v[k] = std::is_same<P, F64Fast>::value ? f64_mulmod_signed(c0, x, q, qinv) : f64_mulmod(c0, x, q, qinv);
+        }
       }
 #pragma unroll
       for (int r = 1; r < kMaxR; ++r) {
@@ -395,7 +403,9 @@ __device__ __forceinline__ void modup_columns(const P& p, const KsArgs& a, const
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
           const double x = __longlong_as_double(src[at(k)]);
-          if constexpr (std::is_same<P, F64Fast>::value) {
+          if constexpr (P::kWide) {
+            v[k] += p.product(cr, x);
+          } else if constexpr (std::is_same<P, F64Fast>::value) {
             v[k] += f64_mulmod_signed(cr, x, q, qinv);
           } else {
             const double sum = v[k] + f64_mulmod(cr, x, q, qinv);
@@ -571,7 +581,7 @@ __device__ __forceinline__ void modup_columns_x2(const KsArgs& a, const KsDigit&
   const int col = cg * C + c;
   auto at = [&](int k) { return static_cast<uint32_t>((t + T * k) * kTile + col); };
   double v0[16], v1[16];
-  if (d.f64_ok) {
+  if (d.f64_ok == 1) {
     const double q0 = row0.qd, qi0 = row0.qinv, q1 = row1.qd, qi1 = row1.qinv;
     const double c00 = static_cast<double>(row0.to_mont), c10 = static_cast<double>(row1.to_mont);
     if constexpr (kRows < 3) {
@@ -651,6 +661,16 @@ __device__ __forceinline__ void modup_columns_x2(const KsArgs& a, const KsDigit&
 template <int S1>
 __device__ __forceinline__ void modup_integer_block(const KsArgs& a, const NttRow& row, const KsDigit& d, int64_t di,
                                                     int64_t b, int64_t j, int cg, int64_t* lds) {
+  if (row.wide) {
+    switch (static_cast<int>(d.rows)) {
+      case 1: modup_columns<S1, 1>(F64Wide(row), a, d, di, b, j, cg, lds); break;
+      case 2: modup_columns<S1, 2>(F64Wide(row), a, d, di, b, j, cg, lds); break;
+      case 3: modup_columns<S1, 3>(F64Wide(row), a, d, di, b, j, cg, lds); break;
+      case 4: modup_columns<S1, 4>(F64Wide(row), a, d, di, b, j, cg, lds); break;
+      default: modup_columns<S1, 0>(F64Wide(row), a, d, di, b, j, cg, lds); break;
+    }
+    return;
+  }
   if (row.delta60) {
     switch (static_cast<int>(d.rows)) {
       case 1: modup_columns<S1, 1>(U64Pm(row), a, d, di, b, j, cg, lds); break;
@@ -864,11 +884,11 @@ template <bool kHoist, bool kSplit, class PI, class Acc>
 __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b, int t, const MacDest& dst,
                                            int64_t* sh, int64_t* tww, int64_t* twp, Acc (&acc0)[8],
                                            Acc (&acc1)[8]) {
-  constexpr bool kF64 = std::is_same<Acc, double>::value;
   const int64_t n = int64_t{1} << a.log_n;
   const int64_t grow = a.level + j;
   const NttRow& row = a.rows[grow];
   const int r_dst = dst.r_dst;
+  const PI pi(row);
   if constexpr (kHoist) {
     auto to_dst = [&](Acc (&acc)[8]) {
       tile_sync();  // earlier readers of the exchange buffer are done
@@ -905,7 +925,7 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
       const int st = 7 - (31 - __builtin_clz(kTile - 1 - idx));
       const int g = idx - (kTile - (kTile >> st));
       const int64_t gi = (n >> (st + 1)) + (static_cast<int64_t>(r_dst) << (7 - st)) + g;
-      tww[idx] = w_row[gi];
+      tww[idx] = pi.stage(w_row[gi]);
       if constexpr (PI::kCompanion) twp[idx] = wp_row[gi];
     }
   }
@@ -916,7 +936,6 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
     tile_sync();
   }
   auto inv_slot = [](int st, int e) { return (kTile - (kTile >> st)) + (e >> (st + 1)); };
-  const PI pi(row);
   auto inverse_tile = [&](auto (&v)[8], auto store) {
     // Round 1 (slots = bits 2..0 of the element): inverse stages 0..2.
 #pragma unroll
@@ -968,15 +987,15 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
   };
   auto finish_one = [&](Acc (&acc)[8], int64_t component) {
     int64_t* slab = a.acc + (component * a.batch + b) * a.lqp * n;
-    if constexpr (kF64) {
-      // binary64 rows of the accumulators travel packed (canonical, 6 bytes)
+    if constexpr (std::is_same<PI, F64Fast>::value) {
+      // rows below 2^42 of the accumulators travel packed (canonical, 6 bytes)
       const PackedInter pk = packed_slab(slab, a.small_rows, n);
       inverse_tile(acc, [&](int e, double x) {
         packed_store(pk, j * n + packed_index(r_dst, e), f64_to_u64(pi.canon(x)));
       });
     } else {
       int64_t* out = slab + j * n + static_cast<int64_t>(r_dst) * kTile;
-      inverse_tile(acc, [&](int e, uint64_t x) { out[e] = static_cast<int64_t>(x); });
+      inverse_tile(acc, [&](int e, Acc x) { out[e] = pi.mid(x); });
     }
   };
   if constexpr (kSplit) {
@@ -1018,7 +1037,7 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
     for (int idx = wave * kMacThreads + t; idx < kTile - 1; idx += waves * kMacThreads) {
       const int st = 31 - __builtin_clz(idx + 1);
       const int64_t gi = (int64_t{1} << (s0 + st)) + (static_cast<int64_t>(r) << st) + (idx + 1 - (1 << st));
-      tww[idx] = w_row[gi];
+      tww[idx] = p.stage(w_row[gi]);
       if constexpr (P::kCompanion) twp[idx] = wp_row[gi];
     }
     if (threadIdx.x < a.dnum) key_digit[threadIdx.x] = a.dig[threadIdx.x].key_digit;
@@ -1059,6 +1078,7 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
 #pragma unroll
     for (int k = 0; k < 8; ++k) nv[k] = tile[mac_e1(t, k)];
   }
+  [[maybe_unused]] uint32_t terms = 0;  // digits added so far
 #pragma nounroll
   for (int64_t di = wave; di < a.dnum; di += waves, tile += digit_stride) {
     Global<int64_t>* k0 = key + key_digit[di] * a.key_sd + grow * a.key_sr + tile_off;
@@ -1142,7 +1162,13 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      if constexpr (kF64) {
+      if constexpr (P::kWide) {
+        // |y| <= 0.51q, w < 2q: each product is below 0.9q; the sums are
+        // reduced every fourth digit
+        const double y = p.settle(v[k]);
+        facc0[k] += p.product(u64_to_f64(static_cast<uint64_t>(w0[k])), y);
+        facc1[k] += p.product(u64_to_f64(static_cast<uint64_t>(w1[k])), y);
+      } else if constexpr (kF64) {
         mac_f64(facc0[k], v[k], w0[k], row.qd, row.qinv);
         mac_f64(facc1[k], v[k], w1[k], row.qd, row.qinv);
       } else {
@@ -1153,6 +1179,15 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
         wide_mac(wacc1[k], y, static_cast<uint64_t>(w1[k]));
       }
     }
+    if constexpr (P::kWide) {
+      if (++terms % 4 == 0) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          facc0[k] = p.reduce(facc0[k]);
+          facc1[k] = p.reduce(facc1[k]);
+        }
+      }
+    }
   }
   // Relinearization seeds: P d0 and P d1 (NTT domain, in the accumulators'
   // scaling) join the Q rows' sums, so that ModDown's exact floor division
@@ -1160,7 +1195,14 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
   // stored at tile positions t + 32k (the HMult front's seed layout).
   if (a.seed0 != nullptr && j < a.lq && wave == 0) {
     const int64_t off = (b * a.lq + j) * n + tile_off + t;
-    if constexpr (kF64) {
+    if constexpr (P::kWide) {
+      const double sc = static_cast<double>(a.seed_scale[grow]);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        facc0[k] += p.product(sc, __longlong_as_double(a.seed0[off + 32 * k]));
+        facc1[k] += p.product(sc, __longlong_as_double(a.seed1[off + 32 * k]));
+      }
+    } else if constexpr (kF64) {
       const double sc = static_cast<double>(a.seed_scale[grow]);
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
@@ -1190,11 +1232,18 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
       uacc1[k] = wide_redc62(wacc1[k], row.q, row.neg_qinv64);
     }
   }
+  if constexpr (P::kWide) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      facc0[k] = p.reduce(facc0[k]);
+      facc1[k] = p.reduce(facc1[k]);
+    }
+  }
   const MacDest dst{r, 8 * t, 0u};
   if constexpr (kSplit) {
     // Wave c collects accumulator c of every wave (exchange buffers take the
-    // shares).  Binary64 shares add exactly (17 terms below 0.53q in all),
-    // integer shares are below 2q each, at most 8 of them.
+    // shares).  Binary64 shares add exactly (17 terms below 0.53q in all, or
+    // at most 8 shares reduced to 0.51q), integer shares are below 2q each, at most 8 of them.
     auto collect = [&](auto (&acc)[8], int owner) {
       __syncthreads();
 #pragma unroll
@@ -1226,7 +1275,7 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
     }
   }
   if constexpr (kF64) {
-    mac_finish<false, kSplit, F64Fast>(a, j, b, t, dst, sh, tww, twp, facc0, facc1);
+    mac_finish<false, kSplit, std::conditional_t<P::kWide, P, F64Fast>>(a, j, b, t, dst, sh, tww, twp, facc0, facc1);
   } else {
     mac_finish<false, kSplit, P>(a, j, b, t, dst, sh, tww, twp, uacc0, uacc1);
   }
@@ -1240,12 +1289,17 @@ constexpr int kMacTilesPerBlock = kMacTiles;
 
 // One launch per arithmetic path (binary64 rows, then the integer rows) so
 // each kernel is register-allocated for its own path only.
-template <int MODE, bool kSmall>
 // Register budgets: 3 waves per SIMD for the binary64 rows (no spills at 156
 // VGPRs), 2+ for the integer rows.
-__global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(kSmall ? 3 : 2))) void k_ks_tiles_mac(KsArgs a, int64_t groups, int64_t j_begin,
+// kRowsKind: which rows a tile-pass launch serves.  Rows of F64Wide primes run
+// in the integer rows' launch where a chain has them beside narrower ones, and
+// in a launch of their own (blocks of other rows end at once) where no row is
+// below 2^42.
+enum RowsKind : int { kRowsSmall = 0, kRowsInteger = 1, kRowsWide = 2 };
+template <int MODE, int kRowsKind>
+__global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(kRowsKind == kRowsInteger ? 2 : 3))) void k_ks_tiles_mac(KsArgs a, int64_t groups, int64_t j_begin,
                                                          int64_t j_count) {
-  __shared__ int64_t lds[mac_lds_words<kSmall>()];
+  __shared__ int64_t lds[mac_lds_words<kRowsKind != kRowsInteger>()];
   const uint32_t batch = static_cast<uint32_t>(a.batch);
   const uint32_t jc = static_cast<uint32_t>(j_count);
   const uint32_t w = xcd_remap(blockIdx.x, static_cast<uint32_t>(groups) * jc * batch);
@@ -1253,18 +1307,20 @@ __global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(kSmal
   const int64_t j = j_begin + (w / batch) % jc;
   const int64_t g = w / (batch * jc);
   const NttRow& row = a.rows[a.level + j];
-  if constexpr (kSmall) {
+  if constexpr (kRowsKind == kRowsSmall) {
     if constexpr (MODE == 1) {
       tiles_mac<false>(F64Fast(row), a, g, j, b, lds);
     } else {
       tiles_mac<false>(F64Exact(row), a, g, j, b, lds);
     }
+  } else if constexpr (kRowsKind == kRowsWide) {
+    if (row.wide) tiles_mac<false>(F64Wide(row), a, g, j, b, lds);
+  } else if (row.wide) {
+    if (!a.wide_apart) tiles_mac<false>(F64Wide(row), a, g, j, b, lds);
+  } else if (row.delta60) {
+    tiles_mac<false>(U64Pm(row), a, g, j, b, lds);
   } else {
-    if (row.delta60) {
-      tiles_mac<false>(U64Pm(row), a, g, j, b, lds);
-    } else {
-      tiles_mac<false>(U64Fast(row), a, g, j, b, lds);
-    }
+    tiles_mac<false>(U64Fast(row), a, g, j, b, lds);
   }
 }
 
@@ -1284,6 +1340,8 @@ __global__ __launch_bounds__(kSplitWaves * 64) void k_ks_tiles_mac_split(KsArgs 
   const NttRow& row = a.rows[a.level + j];
   if (j < a.small_rows) {
     tiles_mac<true>(F64Fast(row), a, g, j, b, lds_dynamic);
+  } else if (row.wide) {
+    tiles_mac<true>(F64Wide(row), a, g, j, b, lds_dynamic);
   } else if (row.delta60) {
     tiles_mac<true>(U64Pm(row), a, g, j, b, lds_dynamic);
   } else {
@@ -1328,7 +1386,7 @@ __device__ __forceinline__ void tiles_forward_store(const P& p, const KsArgs& a,
     for (int idx = t; idx < kTile - 1; idx += kMacThreads) {
       const int st = 31 - __builtin_clz(idx + 1);
       const int64_t gi = (int64_t{1} << (s0 + st)) + (static_cast<int64_t>(r) << st) + (idx + 1 - (1 << st));
-      tww[idx] = w_row[gi];
+      tww[idx] = p.stage(w_row[gi]);
       if constexpr (P::kCompanion) twp[idx] = wp_row[gi];
     }
   }
@@ -1425,7 +1483,9 @@ __global__ __launch_bounds__(kMacBlock) void k_ks_tiles_fwd(KsArgs a, int64_t gr
       tiles_forward_store(F64Exact(row), a, g, j, di, lds);
     }
   } else {
-    if (row.delta60) {
+    if (row.wide) {
+      tiles_forward_store(F64Wide(row), a, g, j, di, lds);
+    } else if (row.delta60) {
       tiles_forward_store(U64Pm(row), a, g, j, di, lds);
     } else {
       tiles_forward_store(U64Fast(row), a, g, j, di, lds);
@@ -1505,7 +1565,11 @@ __device__ __forceinline__ void tiles_mac_hoisted(const P& p, const KsArgs& a, i
   auto mac_digit = [&](int64_t (&w0)[8], int64_t (&w1)[8], V (&v)[8]) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      if constexpr (kF64) {
+      if constexpr (P::kWide) {
+        // reduced each digit (values arrive settled): below 1.4q
+        facc0[k] = p.reduce(facc0[k]) + p.product(u64_to_f64(static_cast<uint64_t>(w0[k])), v[k]);
+        facc1[k] = p.reduce(facc1[k]) + p.product(u64_to_f64(static_cast<uint64_t>(w1[k])), v[k]);
+      } else if constexpr (kF64) {
         mac_f64(facc0[k], v[k], w0[k], row.qd, row.qinv);
         mac_f64(facc1[k], v[k], w1[k], row.qd, row.qinv);
       } else {
@@ -1523,7 +1587,7 @@ __device__ __forceinline__ void tiles_mac_hoisted(const P& p, const KsArgs& a, i
     mac_digit(wb0, wb1, vb);
   }
   if constexpr (kF64) {
-    mac_finish<true, false, F64Fast>(a, j, b, t, dst, sh, tww, twp, facc0, facc1);
+    mac_finish<true, false, std::conditional_t<P::kWide, P, F64Fast>>(a, j, b, t, dst, sh, tww, twp, facc0, facc1);
   } else {
     // at most 16 products y w with y < 4q, w < 2q: REDC value below 9q
 #pragma unroll
@@ -1557,7 +1621,9 @@ __global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(2))) 
       tiles_mac_hoisted(F64Exact(row), a, g, j, b, lds);
     }
   } else {
-    if (row.delta60) {
+    if (row.wide) {
+      tiles_mac_hoisted(F64Wide(row), a, g, j, b, lds);
+    } else if (row.delta60) {
       tiles_mac_hoisted(U64Pm(row), a, g, j, b, lds);
     } else {
       tiles_mac_hoisted(U64Fast(row), a, g, j, b, lds);
@@ -1581,6 +1647,7 @@ struct HmArgs {
   int64_t* out;       // [3, B, L, N] working-format rows for the inverse column pass
   int64_t batch, limbs, row_start;
   int log_n;
+  int wide_apart;     // as in KsArgs
   ParamView params;   // global QP rows
   const NttRow* rows; // global QP NTT records
   const int64_t* fwd_w;
@@ -1612,7 +1679,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
     for (int idx = t; idx < kTile - 1; idx += kMacThreads) {
       const int st = 31 - __builtin_clz(idx + 1);
       const int64_t gi = (int64_t{1} << (s0 + st)) + (static_cast<int64_t>(r) << st) + (idx + 1 - (1 << st));
-      tww[idx] = w_row[gi];
+      tww[idx] = p.stage(w_row[gi]);
       if constexpr (P::kCompanion) twp[idx] = wp_row[gi];
     }
   }
@@ -1669,6 +1736,14 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
       }
     }
   };
+  // binary64 rows: product of two reduced values
+  [[maybe_unused]] auto product = [&](double x, double y) -> double {
+    if constexpr (P::kWide) {
+      return p.product(x, y);
+    } else {
+      return f64_mulmod_signed(x, y, row.qd, row.qinv);
+    }
+  };
   V d0[8], d1[8], d2[8];
   {
     V x0[8], x1[8], y[8];
@@ -1682,8 +1757,8 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
         x0[k] = p.reduce(x0[k]);
         x1[k] = p.reduce(x1[k]);
         const double yb = p.reduce(y[k]);
-        d0[k] = f64_mulmod_signed(x0[k], yb, row.qd, row.qinv);
-        d1[k] = f64_mulmod_signed(x1[k], yb, row.qd, row.qinv);
+        d0[k] = product(x0[k], yb);
+        d1[k] = product(x1[k], yb);
       }
     } else {
       // exact products of the forward outputs (below 4q), one REDC per
@@ -1705,8 +1780,8 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const double yb = p.reduce(y[k]);
-        d1[k] += f64_mulmod_signed(x0[k], yb, row.qd, row.qinv);
-        d2[k] = f64_mulmod_signed(x1[k], yb, row.qd, row.qinv);
+        d1[k] += product(x0[k], yb);
+        d2[k] = product(x1[k], yb);
       }
     } else {
 #pragma unroll
@@ -1729,7 +1804,7 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
       const int st = 7 - (31 - __builtin_clz(kTile - 1 - idx));
       const int gg = idx - (kTile - (kTile >> st));
       const int64_t gi = (n >> (st + 1)) + (static_cast<int64_t>(r) << (7 - st)) + gg;
-      tww[idx] = w_row[gi];
+      tww[idx] = p.stage(w_row[gi]);
       if constexpr (P::kCompanion) twp[idx] = wp_row[gi];
     }
   }
@@ -1798,10 +1873,10 @@ __device__ __forceinline__ void tiles_hmult(const P& p, const HmArgs& a, int64_t
   inverse_tile(d2, out + 2 * comp_stride);
 }
 
-template <bool kSmall, bool kNttD01>
-__global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(kSmall ? 3 : 2))) void k_hmult_tiles(
+template <int kRowsKind, bool kNttD01>
+__global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(kRowsKind == kRowsInteger ? 2 : 3))) void k_hmult_tiles(
     HmArgs a, int64_t groups, int64_t j_begin, int64_t j_count) {
-  __shared__ int64_t lds[kMacExchange + kMacTiles * kTile * (kSmall ? 1 : 2)];
+  __shared__ int64_t lds[kMacExchange + kMacTiles * kTile * (kRowsKind == kRowsInteger ? 2 : 1)];
   const uint32_t batch = static_cast<uint32_t>(a.batch);
   const uint32_t jc = static_cast<uint32_t>(j_count);
   const uint32_t w = xcd_remap(blockIdx.x, static_cast<uint32_t>(groups) * jc * batch);
@@ -1809,14 +1884,16 @@ __global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(kSmal
   const int64_t j = j_begin + (w / batch) % jc;
   const int64_t g = w / (batch * jc);
   const NttRow& row = a.rows[a.row_start + j];
-  if constexpr (kSmall) {
+  if constexpr (kRowsKind == kRowsSmall) {
     tiles_hmult<kNttD01>(F64Fast(row), a, g, j, b, lds);
+  } else if constexpr (kRowsKind == kRowsWide) {
+    if (row.wide) tiles_hmult<kNttD01>(F64Wide(row), a, g, j, b, lds);
+  } else if (row.wide) {
+    if (!a.wide_apart) tiles_hmult<kNttD01>(F64Wide(row), a, g, j, b, lds);
+  } else if (row.delta60) {
+    tiles_hmult<kNttD01>(U64Pm(row), a, g, j, b, lds);
   } else {
-    if (row.delta60) {
-      tiles_hmult<kNttD01>(U64Pm(row), a, g, j, b, lds);
-    } else {
-      tiles_hmult<kNttD01>(U64Fast(row), a, g, j, b, lds);
-    }
+    tiles_hmult<kNttD01>(U64Fast(row), a, g, j, b, lds);
   }
 }
 
@@ -1870,7 +1947,9 @@ __global__ __launch_bounds__(kBlock) void k_ks_gather_base(View3 base, const int
 // products, one reduction).  logN = 16, four P primes: 186 -> 141 us at 7
 // entries of 29 Q rows (3.9 TB/s of accumulators, base and output), 520 ->
 // 385 us at 16 entries of 33 rows with the fused rescale.
-template <int P>
+// kPacked: binary64 rows are those below 2^42, packed; otherwise (no row below
+// 2^42) those of F64Wide primes, canonical words, found by their records.
+template <int P, bool kPacked>
 __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   constexpr int kRows = kModDownRowsPerThread;
   const KsDigit& pdig = *a.pdig;
@@ -1902,7 +1981,7 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   const View3& out = c == 0 ? a.out0 : a.out1;
   const int64_t row_begin = group * kRows;
   const int64_t row_end = row_begin + kRows < a.lq ? row_begin + kRows : a.lq;
-  const int64_t f64_rows = a.small_rows < a.lq ? a.small_rows : a.lq;
+  const int64_t f64_rows = kPacked ? (a.small_rows < a.lq ? a.small_rows : a.lq) : a.lq;
   // Issue every load of the thread's binary64 rows first, with no branch
   // between them (a row past the end reads the last one): joined branches
   // made the compiler wait for each row's load in turn, which cost more than
@@ -1915,19 +1994,25 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
 #pragma unroll
     for (int r = 0; r < P; ++r) dg[r] = acc_row(a.lq + r);
   }
-  uint32_t xlo[kRows], xlo0 = 0;
-  uint16_t xhi[kRows], xhi0 = 0;
+  struct Word {
+    uint32_t lo;
+    uint32_t hi;  // packed rows: the u16 plane's half
+  };
+  auto load_word = [&](int64_t row) -> Word {
+    if constexpr (kPacked) {
+      const uint32_t idx = static_cast<uint32_t>(row * n + pidx);
+      return Word{pk.lo[idx], pk.hi[idx]};
+    } else {
+      const uint64_t x = static_cast<uint64_t>(slab[static_cast<uint32_t>(row * n + i)]);
+      return Word{static_cast<uint32_t>(x), static_cast<uint32_t>(x >> 32)};
+    }
+  };
+  Word xv[kRows], x0{0, 0};
   int64_t bv[kRows], bv0 = 0;
   if (f64_rows > 0) {
 #pragma unroll
-    for (int rr = 0; rr < kRows; ++rr) {
-      const int64_t row = row_begin + rr < f64_rows ? row_begin + rr : f64_rows - 1;
-      const uint32_t idx = static_cast<uint32_t>(row * n + pidx);
-      xlo[rr] = pk.lo[idx];
-      xhi[rr] = pk.hi[idx];
-    }
-    xlo0 = pk.lo[static_cast<uint32_t>(pidx)];  // row 0, for the fused rescale
-    xhi0 = pk.hi[static_cast<uint32_t>(pidx)];
+    for (int rr = 0; rr < kRows; ++rr) xv[rr] = load_word(row_begin + rr < f64_rows ? row_begin + rr : f64_rows - 1);
+    x0 = load_word(0);  // for the fused rescale
     if (has_base) {
 #pragma unroll
       for (int rr = 0; rr < kRows; ++rr) {
@@ -1937,8 +2022,8 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
       bv0 = base.at(b, 0, i);
     }
   }
-  auto packed_f64 = [](uint32_t lo, uint16_t hi) -> double {
-    return u64_to_f64(static_cast<uint64_t>(lo) | static_cast<uint64_t>(hi) << 32);
+  auto word_f64 = [](Word w) -> double {
+    return u64_to_f64(static_cast<uint64_t>(w.lo) | static_cast<uint64_t>(w.hi) << 32);
   };
   // Mixed-radix digits of X mod P (X_P = sum_r c_r prod_{t<r} p_t), each
   // split as c_hi 2^30 + c_lo (both exact in binary64).
@@ -1961,9 +2046,9 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   // 2P + 1 products (x P^{-1}, and the digit halves of X_P times their
   // negated constants), reduced once.  x and the constants are below q, the
   // halves below 2^30, so the sum is below q (q + 2P 2^30) and its reduced
-  // value within 0.52q.  The result of a binary64 row stays in binary64
-  // (exact integers below 2^47) through the base addition and the fused
-  // rescale.
+  // value within 0.52q (F64Wide primes: within 5.3q, reduced once more).  The
+  // result of a binary64 row stays in binary64 (exact integers) through the
+  // base addition and the fused rescale.
   auto moddown_f64 = [&](Global<double>* rec, double x) -> double {
     const double q = rec[14], qinv = rec[15];
     const double start = f64_sum_start(q * (q + 2.0 * P * 0x1.0p30));
@@ -1974,7 +2059,8 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
       f64_sum_add(sum, rec[r], dlo[r]);
       f64_sum_add(sum, rec[P + r], dhi[r]);
     }
-    const double res = f64_sum_reduce(sum, start, q, qinv);
+    double res = f64_sum_reduce(sum, start, q, qinv);
+    if constexpr (!kPacked) res = __builtin_fma(-__builtin_rint(res * qinv), q, res);
     return res < 0.0 ? res + q : res;
   };
   // add_canonical of a canonical value and a base below 2q
@@ -2004,9 +2090,9 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   int64_t c0_int = 0;
   int64_t round_up = 0;
   if (rescale) {
-    if (f64_rows > 0) {
-      Global<double>* rec0 = global(pdig.f64_table) + a.level * pitch;
-      c0 = add_base_f64(moddown_f64(rec0, packed_f64(xlo0, xhi0)), bv0, rec0[14]);
+    Global<double>* rec0 = global(pdig.f64_table) + a.level * pitch;
+    if (kPacked ? f64_rows > 0 : rec0[14] != 0.0) {
+      c0 = add_base_f64(moddown_f64(rec0, word_f64(x0)), bv0, rec0[14]);
       c0_int = static_cast<int64_t>(f64_to_u64(c0));
     } else {
       c0_int = moddown_integer(a.level, acc_row(0), has_base ? base.at(b, 0, i) : 0);
@@ -2019,11 +2105,19 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
     if (row >= f64_rows) break;
     Global<double>* rec = global(pdig.f64_table) + (a.level + row) * pitch;
     const double q = rec[14];
-    double v = add_base_f64(moddown_f64(rec, packed_f64(xlo[rr], xhi[rr])), bv[rr], q);
+    if (!kPacked && q == 0.0) continue;
+    double v = add_base_f64(moddown_f64(rec, word_f64(xv[rr])), bv[rr], q);
     if (rescale && row > 0) {
-      // ((v - c0) q0^{-1} + round_up) mod q, |v - c0| < 2^47 exact
+      // ((v - c0) q0^{-1} + round_up) mod q, |v - c0| exact
       const double inv = u64_to_f64(static_cast<uint64_t>(global(a.rescale_inv)[row - 1]));
-      double r = f64_mulmod_signed(inv, v - c0, q, rec[15]);
+      double r;
+      if constexpr (kPacked) {
+        r = f64_mulmod_signed(inv, v - c0, q, rec[15]);
+      } else {
+        // quotients up to 2^50: a rounding instruction, as F64Wide's product
+        const double x = v - c0, h = inv * x;
+        r = __builtin_fma(-__builtin_rint(h * rec[15]), q, h) + __builtin_fma(inv, x, -h);
+      }
       r += static_cast<double>(round_up);
       v = r < 0.0 ? r + q : (r >= q ? r - q : r);
     }
@@ -2036,8 +2130,9 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   }
   // Integer rows (the base prime), one body outside the unrolled loop.
 #pragma nounroll
-  for (int64_t row = row_begin > f64_rows ? row_begin : f64_rows; row < row_end; ++row) {
+  for (int64_t row = kPacked && f64_rows > row_begin ? f64_rows : row_begin; row < row_end; ++row) {
     const int64_t grow = a.level + row;
+    if (!kPacked && global(pdig.f64_table)[grow * pitch + 14] != 0.0) continue;
     int64_t value = moddown_integer(grow, acc_row(row), has_base ? base.at(b, row, i) : 0);
     if (rescale && row > 0) {
       // the dropped prime may exceed this one: c0 mod q first (c0 >= q is
@@ -2209,6 +2304,7 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
   a.gal_idx = galois_index_tables;
   a.gal_sign = galois_sign_tables;
   a.small_rows = small_rows;
+  a.wide_apart = small_rows == 0 ? 1 : 0;
   a.seed0 = seed0;
   a.seed1 = seed1;
   a.seed_scale = seed_scale;
@@ -2270,9 +2366,11 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
     FH_CHECK_LAUNCH("key switch modup + column pass");
     return kOk;
   };
+  // pass 0 of a chain without rows below 2^42: its F64Wide rows, wherever they are.
   auto launch_mac = [&](int pass, hipStream_t st) -> int {
+    const bool wide = pass == 0 && a.wide_apart && !hoist;
     const int64_t j_begin = pass == 0 ? 0 : small_rows;
-    const int64_t j_count = pass == 0 ? small_rows : lqp - small_rows;
+    const int64_t j_count = pass == 0 ? (wide ? lqp : small_rows) : lqp - small_rows;
     if (j_count == 0) return kOk;
     const dim3 grid(static_cast<uint32_t>(groups * j_count * batch));
 #define FH_MAC_LAUNCH(K, ARGS)                                                                               \
@@ -2296,7 +2394,15 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
       FH_CHECK_LAUNCH("hoisted key switch forward tile pass");
       FH_MAC_LAUNCH(k_ks_mac_hoisted, a)
     } else {
-      FH_MAC_LAUNCH(k_ks_tiles_mac, a)
+      if (wide) {
+        hipLaunchKernelGGL((k_ks_tiles_mac<0, kRowsWide>), grid, dim3(kMacBlock), 0, st, a, groups, j_begin, j_count);
+      } else if (pass == 1) {
+        hipLaunchKernelGGL((k_ks_tiles_mac<0, kRowsInteger>), grid, dim3(kMacBlock), 0, st, a, groups, j_begin, j_count);
+      } else if (mode == 1) {
+        hipLaunchKernelGGL((k_ks_tiles_mac<1, kRowsSmall>), grid, dim3(kMacBlock), 0, st, a, groups, j_begin, j_count);
+      } else {
+        hipLaunchKernelGGL((k_ks_tiles_mac<0, kRowsSmall>), grid, dim3(kMacBlock), 0, st, a, groups, j_begin, j_count);
+      }
     }
 #undef FH_MAC_LAUNCH
     FH_CHECK_LAUNCH("key switch tile pass + MAC");
@@ -2339,7 +2445,7 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
     SideStream* side = nullptr;
     int rc = side_stream(&side);
     if (rc != kOk) return rc;
-    const bool split = small_rows > 0 && small_rows < lqp;
+    const bool split = small_rows < lqp && (small_rows > 0 || (a.wide_apart && !hoist));
     if (split) {
       rc = launch_modup(1, s);
       if (rc != kOk) return rc;
@@ -2414,14 +2520,24 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
   const int64_t md_blocks = (n / kBlock) * ceil_div(lq, kModDownRowsPerThread) * 2 * batch;
   FH_CHECK_ARG(md_blocks <= 0x7fffffff, "key switch grid too large");
   const dim3 md_grid(static_cast<uint32_t>(md_blocks));
+#define FH_MODDOWN_CASE(P)                                                                       \
+  case P:                                                                                        \
+    if (small_rows > 0) {                                                                        \
+      hipLaunchKernelGGL((k_ks_moddown_add<P, true>), md_grid, dim3(kBlock), 0, s, md);          \
+    } else {                                                                                     \
+      hipLaunchKernelGGL((k_ks_moddown_add<P, false>), md_grid, dim3(kBlock), 0, s, md);         \
+    }                                                                                            \
+    break;
   switch (lqp - lq) {
-    case 1: hipLaunchKernelGGL(k_ks_moddown_add<1>, md_grid, dim3(kBlock), 0, s, md); break;
-    case 2: hipLaunchKernelGGL(k_ks_moddown_add<2>, md_grid, dim3(kBlock), 0, s, md); break;
-    case 3: hipLaunchKernelGGL(k_ks_moddown_add<3>, md_grid, dim3(kBlock), 0, s, md); break;
-    case 4: hipLaunchKernelGGL(k_ks_moddown_add<4>, md_grid, dim3(kBlock), 0, s, md); break;
-    case 5: hipLaunchKernelGGL(k_ks_moddown_add<5>, md_grid, dim3(kBlock), 0, s, md); break;
-    default: hipLaunchKernelGGL(k_ks_moddown_add<6>, md_grid, dim3(kBlock), 0, s, md); break;
+    FH_MODDOWN_CASE(1)
+    FH_MODDOWN_CASE(2)
+    FH_MODDOWN_CASE(3)
+    FH_MODDOWN_CASE(4)
+    FH_MODDOWN_CASE(5)
+    default:
+      FH_MODDOWN_CASE(6)
   }
+#undef FH_MODDOWN_CASE
   FH_CHECK_LAUNCH("key switch moddown + add");
   return kOk;
 }
@@ -2584,6 +2700,7 @@ FH_API int fh_ckks_hmult_tensor_coefficient(const int64_t* a, const int64_t* b, 
   h.log_n = static_cast<int>(log_n);
   h.params = ParamView{rns_params.data, rns_params.stride_row, rns_params.stride_col};
   h.rows = rows;
+  h.wide_apart = small_rows == 0 ? 1 : 0;
   h.fwd_w = forward_twiddles;
   h.fwd_wp = forward_twiddles_shoup;
   h.inv_w = inverse_twiddles;
@@ -2593,19 +2710,28 @@ FH_API int fh_ckks_hmult_tensor_coefficient(const int64_t* a, const int64_t* b, 
   if (small_rows > 0) {
     const dim3 grid(static_cast<uint32_t>(groups * small_rows * batch));
     if (ntt_d01) {
-      hipLaunchKernelGGL((k_hmult_tiles<true, true>), grid, dim3(kMacBlock), 0, s, h, groups, int64_t{0}, small_rows);
+      hipLaunchKernelGGL((k_hmult_tiles<kRowsSmall, true>), grid, dim3(kMacBlock), 0, s, h, groups, int64_t{0}, small_rows);
     } else {
-      hipLaunchKernelGGL((k_hmult_tiles<true, false>), grid, dim3(kMacBlock), 0, s, h, groups, int64_t{0}, small_rows);
+      hipLaunchKernelGGL((k_hmult_tiles<kRowsSmall, false>), grid, dim3(kMacBlock), 0, s, h, groups, int64_t{0}, small_rows);
     }
     FH_CHECK_LAUNCH("fused tensor product tiles (binary64 rows)");
   }
   if (small_rows < limbs) {
     const dim3 grid(static_cast<uint32_t>(groups * (limbs - small_rows) * batch));
+    if (h.wide_apart) {
+      if (ntt_d01) {
+        hipLaunchKernelGGL((k_hmult_tiles<kRowsWide, true>), grid, dim3(kMacBlock), 0, s, h, groups, small_rows,
+                           limbs - small_rows);
+      } else {
+        hipLaunchKernelGGL((k_hmult_tiles<kRowsWide, false>), grid, dim3(kMacBlock), 0, s, h, groups, small_rows,
+                           limbs - small_rows);
+      }
+    }
     if (ntt_d01) {
-      hipLaunchKernelGGL((k_hmult_tiles<false, true>), grid, dim3(kMacBlock), 0, s, h, groups, small_rows,
+      hipLaunchKernelGGL((k_hmult_tiles<kRowsInteger, true>), grid, dim3(kMacBlock), 0, s, h, groups, small_rows,
                          limbs - small_rows);
     } else {
-      hipLaunchKernelGGL((k_hmult_tiles<false, false>), grid, dim3(kMacBlock), 0, s, h, groups, small_rows,
+      hipLaunchKernelGGL((k_hmult_tiles<kRowsInteger, false>), grid, dim3(kMacBlock), 0, s, h, groups, small_rows,
                          limbs - small_rows);
     }
     FH_CHECK_LAUNCH("fused tensor product tiles (integer rows)");

@@ -172,6 +172,9 @@ __device__ __forceinline__ uint64_t ntt_product(const U64Fast& p, uint64_t x, in
   return wide_redc62(acc, p.q, p.row->neg_qinv64);
 }
 
+__device__ __forceinline__ double ntt_product(const F64Wide& p, double x, int64_t w) {
+  return p.product(u64_to_f64(static_cast<uint64_t>(w)), p.settle(x));
+}
 __device__ __forceinline__ uint64_t ntt_product(const U64Pm& p, uint64_t x, int64_t w) {
   WideAcc acc{0, 0, 0};
   wide_mac(acc, p.settle(x), static_cast<uint64_t>(w));
@@ -443,7 +446,10 @@ enum Mode : int { kExact = 0, kFast = 1 };
         CALL;                                              \
       }                                                    \
     } else {                                               \
-      if (MODE == kFast && (ROW).delta60) {                \
+      if (MODE == kFast && (ROW).wide) {                   \
+        F64Wide p(ROW);                                    \
+        CALL;                                              \
+      } else if (MODE == kFast && (ROW).delta60) {         \
         U64Pm p(ROW);                                      \
         CALL;                                              \
       } else if (MODE == kFast) {                          \
@@ -468,7 +474,7 @@ __device__ __forceinline__ void words_in(const P& p, const int64_t (&words)[16],
 // make each wait for its own load).
 template <class P>
 __device__ __forceinline__ void words_lift(const P& p, const int64_t (&words)[16], typename P::V (&v)[16]) {
-  if constexpr (std::is_same<P, F64Fast>::value) {
+  if constexpr (std::is_same<P, F64Fast>::value || P::kWide) {
     uint64_t any = 0;
 #pragma unroll
     for (int k = 0; k < 16; ++k) any |= static_cast<uint64_t>(words[k] ^ (words[k] >> 63));
@@ -555,6 +561,8 @@ __global__ __launch_bounds__(kBlock) void k_product_tiles(NttArgs a, const int64
   const int g = static_cast<int>(blockIdx.x);
   if (rr.row->small) {
     product_tiles(F64Fast(*rr.row), a.log_n, g, rr.base, rr.tw, rr.twp, itw + off, itwp + off, w, lds);
+  } else if (rr.row->wide) {
+    product_tiles(F64Wide(*rr.row), a.log_n, g, rr.base, rr.tw, rr.twp, itw + off, itwp + off, w, lds);
   } else if (rr.row->delta60) {
     product_tiles(U64Pm(*rr.row), a.log_n, g, rr.base, rr.tw, rr.twp, itw + off, itwp + off, w, lds);
   } else {
@@ -792,8 +800,10 @@ __device__ uint64_t shoup_companion(uint64_t w, uint64_t q) {
 // lets values grow to 11q over its 16 unreduced stages and every binary64
 // product needs |w x| / q < 2^46.4 (w < q) to be exact, so 11q must stay
 // below 2^46.4; the key switch's accumulators (below 9.1q) need the same.
-// Larger primes take the integer path, which is exact for any q < 2^62.
+// Larger primes take the integer path, which is exact for any q < 2^62, or,
+// in fast arithmetic and below kWidePrimeLimit, F64Wide.
 constexpr uint64_t kSmallPrimeLimit = uint64_t{1} << 42;
+constexpr uint64_t kWidePrimeLimit = (uint64_t{1} << 50) + (uint64_t{1} << 30);
 
 __global__ void k_prepare_rows(ParamView params, int64_t limbs, NttRow* rows) {
   const int64_t l = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -814,6 +824,7 @@ __global__ void k_prepare_rows(ParamView params, int64_t limbs, NttRow* rows) {
   r.to_mont_p = shoup_companion(r.to_mont, m.q);
   r.ninv_mont_p = shoup_companion(r.ninv_mont, m.q);
   r.ninv_std_p = shoup_companion(r.ninv_std, m.q);
+  r.wide = m.q >= kSmallPrimeLimit && m.q < kWidePrimeLimit ? 1 : 0;
   const uint64_t delta = (uint64_t{1} << 60) - m.q;
   r.delta60 = m.q < (uint64_t{1} << 60) && delta < (uint64_t{1} << 26) ? delta : 0;
   // k = -q^{-1} mod 2^62 lifts by one Newton step: q k (2 + q k) = -1 mod 2^124

@@ -58,6 +58,7 @@ __device__ __forceinline__ int64_t center_canonical(int64_t r, uint64_t q) {
 //   mid/unmid        working value <-> 64-bit intermediate between passes
 //   out_fwd(v)       final forward value -> int64 residue
 //   out_inv(v, f)    N^{-1} scaling and representation f -> int64 residue
+//   stage(w)         a twiddle table word as tw_make takes it
 //   settle(v)        forward output as an operand of the exact product sums
 //   fwd/inv          butterflies, told their stage within the pass (a
 //                    compile-time constant after unrolling).
@@ -66,6 +67,7 @@ __device__ __forceinline__ int64_t center_canonical(int64_t r, uint64_t q) {
 // Exact binary64 path (q < 2^42): reference lazy semantics, see fh_common.h.
 struct F64Exact {
   static constexpr bool kCompanion = false;  // twiddles carry a Shoup companion
+  static constexpr bool kWide = false;
   using V = double;
   struct Tw {
     double w;
@@ -79,6 +81,7 @@ struct F64Exact {
   }
   // twiddle from its table words (w, Shoup companion)
   __device__ __forceinline__ Tw tw_make(int64_t w, int64_t) const { return Tw{__longlong_as_double(w)}; }
+  __device__ __forceinline__ int64_t stage(int64_t w) const { return w; }
   __device__ __forceinline__ Tw konst(uint64_t c, uint64_t) const {
     return Tw{static_cast<double>(c)};
   }
@@ -123,6 +126,7 @@ struct F64Exact {
 // (-0.52q, 0.52q) without the final correction.
 struct F64Fast {
   static constexpr bool kCompanion = false;  // twiddles carry a Shoup companion
+  static constexpr bool kWide = false;
   using V = double;
   using Tw = F64Exact::Tw;
   double q, qinv;
@@ -132,6 +136,7 @@ struct F64Fast {
     return Tw{__longlong_as_double(w[idx])};
   }
   __device__ __forceinline__ Tw tw_make(int64_t w, int64_t) const { return Tw{__longlong_as_double(w)}; }
+  __device__ __forceinline__ int64_t stage(int64_t w) const { return w; }
   __device__ __forceinline__ Tw konst(uint64_t c, uint64_t) const {
     return Tw{static_cast<double>(c)};
   }
@@ -178,9 +183,79 @@ struct F64Fast {
   }
 };
 
+// Binary64 path for fast arithmetic on primes from 2^42 to just above 2^50
+// (the 50-bit scale primes).  The quotient of a product reaches 2^53, so it
+// is rounded by an instruction instead of the 2^52 magic constant, its
+// estimate is off by up to 3/8 per q of the operand, and sums need more
+// reductions than F64Fast's; every value stays an exact integer below 2^53.
+// In units of q: a product of an operand x is below 0.5 + 0.375 x; forward
+// sums reduced at even stages stay below 3.9, inverse sums reduced at every
+// stage leave products below 1.1.  Against the integer path (at least 10
+// 32-bit multiplies per product) a butterfly is 9.5 or 11 binary64
+// operations: the 24 50-bit rows of a 3-entry key switch at logN = 16 take 174
+// us in the tile pass and MAC and 190 us in ModUp, where with the integer path
+// the 29 rows took 313 and 264 us.
+struct F64Wide {
+  static constexpr bool kCompanion = false;
+  static constexpr bool kWide = true;
+  using V = double;
+  using Tw = F64Exact::Tw;
+  double q, qinv;
+  const NttRow* row;
+  __device__ __forceinline__ explicit F64Wide(const NttRow& r) : q(r.qd), qinv(r.qinv), row(&r) {}
+  __device__ __forceinline__ int64_t stage(int64_t w) const {
+    return __double_as_longlong(u64_to_f64(static_cast<uint64_t>(w)));
+  }
+  __device__ __forceinline__ Tw tw(const int64_t* w, const int64_t*, int64_t idx) const {
+    return Tw{u64_to_f64(static_cast<uint64_t>(w[idx]))};
+  }
+  __device__ __forceinline__ Tw tw_make(int64_t staged, int64_t) const { return Tw{__longlong_as_double(staged)}; }
+  __device__ __forceinline__ Tw konst(uint64_t c, uint64_t) const { return Tw{u64_to_f64(c)}; }
+  __device__ __forceinline__ V in(int64_t raw) const { return u64_to_f64(static_cast<uint64_t>(raw)); }
+  __device__ __forceinline__ int64_t mid(V v) const { return __double_as_longlong(v); }
+  __device__ __forceinline__ V unmid(int64_t b) const { return __longlong_as_double(b); }
+  // w x - round(w x / q) q, exact, for |w x| / q below 2^53
+  __device__ __forceinline__ V product(double w, V x) const {
+    const double h = w * x;
+    const double l = __builtin_fma(w, x, -h);
+    const double t = __builtin_rint(h * qinv);
+    return __builtin_fma(-t, q, h) + l;
+  }
+  __device__ __forceinline__ V mul(Tw w, V x) const { return product(w.w, x); }
+  __device__ __forceinline__ V reduce(V x) const { return __builtin_fma(-__builtin_rint(x * qinv), q, x); }
+  __device__ __forceinline__ V settle(V v) const { return reduce(v); }
+  __device__ __forceinline__ V canon(V x) const {
+    const V r = reduce(x);
+    return r < 0.0 ? r + q : r;
+  }
+  __device__ __forceinline__ void fwd(V& u, V& l, Tw w, int stage) const {
+    const V a = (stage & 1) == 0 ? reduce(u) : u;
+    const V v = mul(w, l);
+    l = a - v;
+    u = a + v;
+  }
+  __device__ __forceinline__ void inv(V& u, V& l, Tw w, int) const {
+    const V d = u - l;
+    u = reduce(u + l);
+    l = mul(w, d);
+  }
+  __device__ __forceinline__ V to_mont(V x) const { return mul(konst(row->to_mont, 0), x); }
+  __device__ __forceinline__ int64_t out_fwd(V v) const { return static_cast<int64_t>(f64_to_u64(canon(v))); }
+  // (the key switch's accumulators of these rows carry R^2 as those of the
+  // narrower binary64 rows: kOutStdMac)
+  __device__ __forceinline__ int64_t out_inv(V v, int form) const {
+    const Tw c = form == kOutMontgomery ? konst(row->ninv_mont, 0)
+                 : form == kOutStdMac      ? konst(row->ninv_std_rinv, 0)
+                                           : konst(row->ninv_std, 0);
+    const int64_t r = static_cast<int64_t>(f64_to_u64(canon(mul(c, v))));
+    return form == kOutCentered ? center_canonical(r, row->q) : r;
+  }
+};
+
 // Integer Shoup path (any q < 2^62), reference lazy semantics (exact mode).
 struct U64Path {
   static constexpr bool kCompanion = true;  // twiddles carry a Shoup companion
+  static constexpr bool kWide = false;
   using V = uint64_t;
   struct Tw {
     uint64_t w, wp;
@@ -194,6 +269,7 @@ struct U64Path {
   __device__ __forceinline__ Tw tw_make(int64_t w, int64_t wp) const {
     return Tw{static_cast<uint64_t>(w), static_cast<uint64_t>(wp)};
   }
+  __device__ __forceinline__ int64_t stage(int64_t w) const { return w; }
   __device__ __forceinline__ Tw konst(uint64_t c, uint64_t cp) const { return Tw{c, cp}; }
   __device__ __forceinline__ V in(int64_t raw) const { return static_cast<uint64_t>(raw); }
   __device__ __forceinline__ int64_t mid(V v) const { return static_cast<int64_t>(v); }
@@ -234,6 +310,7 @@ struct U64Path {
 // values modulo q exactly as U64Path's do.
 struct U64Fast {
   static constexpr bool kCompanion = true;  // twiddles carry a Shoup companion
+  static constexpr bool kWide = false;
   using V = uint64_t;
   struct Tw {
     uint64_t w, wp;
@@ -247,6 +324,7 @@ struct U64Fast {
   __device__ __forceinline__ Tw tw_make(int64_t w, int64_t wp) const {
     return Tw{static_cast<uint64_t>(w), static_cast<uint64_t>(wp)};
   }
+  __device__ __forceinline__ int64_t stage(int64_t w) const { return w; }
   __device__ __forceinline__ Tw konst(uint64_t c, uint64_t cp) const { return Tw{c, cp}; }
   __device__ __forceinline__ V in(int64_t raw) const { return static_cast<uint64_t>(raw); }
   __device__ __forceinline__ int64_t mid(V v) const { return static_cast<int64_t>(v); }
@@ -297,6 +375,7 @@ struct U64Fast {
 // folded each stage).
 struct U64Pm {
   static constexpr bool kCompanion = false;
+  static constexpr bool kWide = false;
   using V = uint64_t;
   struct Tw {
     uint64_t w;
@@ -311,6 +390,7 @@ struct U64Pm {
   __device__ __forceinline__ Tw tw(const int64_t* w, const int64_t*, int64_t idx) const {
     return make(static_cast<uint64_t>(w[idx]));
   }
+  __device__ __forceinline__ int64_t stage(int64_t w) const { return w; }
   __device__ __forceinline__ Tw tw_make(int64_t w, int64_t) const { return make(static_cast<uint64_t>(w)); }
   __device__ __forceinline__ Tw konst(uint64_t c, uint64_t) const { return make(c); }
   __device__ __forceinline__ V in(int64_t raw) const { return static_cast<uint64_t>(raw); }

@@ -90,8 +90,9 @@ class HybridKeySwitcher:
                      moddown_table: torch.Tensor | None = None) -> list[int]:
         d = len(t.prime_ids)
         multi = d > 1
-        # binary64 basis extension needs every digit below 2^45
-        f64_ok = int(all(self.config.moduli[i] < F64_DIGIT_LIMIT for i in t.prime_ids))
+        # digits carried as binary64: below 2^45 (1), or as wide rows are (2)
+        top = max(self.config.moduli[i] for i in t.prime_ids)
+        f64_ok = 1 if top < F64_DIGIT_LIMIT else (2 if top < rns.WIDE_PRIME_LIMIT else 0)
         # words 14, 15: the P digit's ModDown records, or a Q digit's
         # binary64 Garner record (f64_ok, D > 1)
         if moddown_table is not None:

@@ -191,6 +191,9 @@ def _as_signed64(v: int) -> int:
 # butterfly stages and the key-switch accumulators up to 0.53 (digits + 1) q,
 # and every binary64 product needs |w x| / q below 2^46.4 to stay exact.
 BINARY64_PRIME_LIMIT = 1 << 42
+# Larger primes below this (the 50-bit scale primes) take the wider binary64
+# arithmetic in fast mode (kWidePrimeLimit in csrc/ntt.hip).
+WIDE_PRIME_LIMIT = (1 << 50) + (1 << 30)
 
 # Binary64 ModDown split: a P digit c < 2^60 is taken as c_hi 2^30 + c_lo.
 MODDOWN_SPLIT_BITS = 30
@@ -202,7 +205,7 @@ MODDOWN_RECORD_WORDS = 16
 def moddown_binary64_table(moduli: tuple[int, ...], p_ids: tuple[int, ...],
                            q_ids: tuple[int, ...]) -> torch.Tensor:
     """[Q0, 16] float64 ModDown records, one per Q row whose prime is below
-    BINARY64_PRIME_LIMIT.  With M_r = prod_{t<r} p_t, words 0..P-1 hold
+    WIDE_PRIME_LIMIT.  With M_r = prod_{t<r} p_t, words 0..P-1 hold
     -M_r P^{-1} mod q, words P..2P-1 hold -2^30 M_r P^{-1} mod q, word 2P
     holds P^{-1} mod q, word 14 holds q and word 15 holds 1/q, so that
     floor(X / P) = (x - X_P) P^{-1} mod q is one sum of 2P + 1 products (the
@@ -220,7 +223,7 @@ def moddown_binary64_table(moduli: tuple[int, ...], p_ids: tuple[int, ...],
     out = torch.zeros((len(q_ids), MODDOWN_RECORD_WORDS), dtype=torch.float64)
     for j, qi in enumerate(q_ids):
         q = moduli[qi]
-        if q >= BINARY64_PRIME_LIMIT:
+        if q >= WIDE_PRIME_LIMIT:
             continue
         p_inverse = pow(p_product, -1, q)
         for r, m in enumerate(prefix):
@@ -266,7 +269,7 @@ class HostTables:
         # (their accumulators hold x R^2 and the seeds a b R^2), P R mod q for
         # the integer rows (exact sums reduced by one REDC: x R, seeds a b R).
         self.seed_scale = torch.tensor(
-            [p_product % moduli[i] if moduli[i] < BINARY64_PRIME_LIMIT else (p_product * R) % moduli[i]
+            [p_product % moduli[i] if moduli[i] < WIDE_PRIME_LIMIT else (p_product * R) % moduli[i]
              for i in self.layout.prime_ids(0)], dtype=torch.int64
         )
         self.moddown_binary64 = moddown_binary64_table(moduli, self.layout.p_prime_ids,

@@ -229,12 +229,16 @@ int fh_ckks_keyswitch_accumulate_multi_key(fh_view3 acc0, fh_view3 acc1, fh_view
  * captured with it).
  *   component        [batch, lq, N] canonical standard Q rows at `level`
  *   small_rows       number of leading QP rows at `level` whose prime is
- *                    below 2^42 (binary64 arithmetic; the rest are integer
- *                    rows, whose primes must be below 2^60)
+ *                    below 2^42 (binary64 arithmetic, 6-byte intermediates;
+ *                    of the rest, primes below 2^50 + 2^30 use binary64 in
+ *                    8-byte words and the others, which must be below 2^60,
+ *                    integers)
  *   digit_table      [digit_count, 16] int64 digit descriptors (row_begin,
  *                    rows, key_digit, addresses of the digit's mixed-radix
  *                    and basis-extension tables, basis row stride, address
- *                    of the standard-form basis table, binary64 flag)
+ *                    of the standard-form basis table, binary64 flag: 1 when
+ *                    every prime of the digit is below 2^45, 2 when below
+ *                    2^50 + 2^30)
  *   p_digit_table    [16] int64 descriptor of the P primes taken as one
  *                    digit (mixed-radix tables, extension onto QP0)
  *   p_inverse_q      [Q0] P^{-1} mod q_j, standard form
@@ -260,7 +264,7 @@ int fh_ckks_keyswitch_accumulate_multi_key(fh_view3 acc0, fh_view3 acc1, fh_view
  *                    the accumulators' scaling (what
  *                    fh_ckks_hmult_tensor_coefficient leaves in d0, d1 with
  *                    ntt_d01 = 1), with seed_scale [Q0] (P mod q for rows
- *                    below 2^42, P 2^62 mod q for the others): seed_scale x
+ *                    below 2^50 + 2^30, P 2^62 mod q for the others): seed_scale x
  *                    seed is added to the Q rows of accumulator 0 / 1, so the
  *                    results gain exactly d0 / d1 (floor((X + P d) / P) =
  *                    floor(X / P) + d), as base0 / base1 = d0 / d1 would. */
@@ -355,7 +359,7 @@ int fh_keyswitch_fused_static(fh_view3 component, int64_t batch, int64_t lq, int
  *   ntt_d01          0: d0, d1, d2 all in the coefficient domain; 1: d0 and
  *                    d1 stay in the NTT domain as accumulator seeds for
  *                    fh_keyswitch_fused (working format: binary64 bits of
- *                    a b R^2 for rows below 2^42, a b R as u64 below 2q for
+ *                    a b R^2 for rows below 2^50 + 2^30, a b R as u64 below 2q for
  *                    the others; within each 256-coefficient tile the value
  *                    of coefficient 8t + k at position t + 32k), d2 in the
  *                    coefficient domain
