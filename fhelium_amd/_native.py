@@ -93,6 +93,9 @@ SIGNATURES: dict[str, list] = {
     "fh_keyswitch_hoisted": [fh_view3, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _i64, _ptr, _ptr, fh_table2,
                              _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr,
                              _ptr, fh_view3, fh_view3, fh_view3, _i32, _ptr],
+    "fh_keyswitch_hoisted_ntt": [fh_view3, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _i64, _ptr, _ptr, _ptr, fh_table2,
+                                 _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr,
+                                 _ptr, _ptr],
     "fh_runtime_version": [_ptr],
     "fh_stream_copy": [_ptr, _ptr, _i64, _ptr],
     "fh_arena_create": [_i64, _ptr],

@@ -116,6 +116,9 @@ struct KsArgs {
   // entry reads that entry's intermediate through the NTT-domain Galois map
   // of its own g.
   const int64_t* hoist_galois;
+  // Hoisted rotations that stay in the NTT domain: the Q rows of the
+  // accumulators keep their NTT-domain sums (no inverse stages).
+  int keep_ntt;
 };
 
 
@@ -907,6 +910,36 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
     };
     to_dst(acc0);
     to_dst(acc1);
+    if (a.keep_ntt && j < a.lq) {
+      // elements 8t .. 8t+7 of the destination tile: rows below 2^42 packed
+      // and canonical, the others as they are (below 2q)
+      auto keep = [&](Acc (&acc)[8], int64_t component) {
+        int64_t* slab = a.acc + (component * a.batch + b) * a.lqp * n;
+        if constexpr (std::is_same<PI, F64Fast>::value) {
+          const PackedInter pk = packed_slab(slab, a.small_rows, n);
+          const uint32_t idx = static_cast<uint32_t>(j * n + packed_index(r_dst, 8 * t));
+          uint32_t lo[8], hi[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            const uint64_t u = f64_to_u64(pi.canon(acc[k]));
+            lo[k] = static_cast<uint32_t>(u);
+            hi[k] = static_cast<uint32_t>(u >> 32);
+          }
+          uint4* dlo = reinterpret_cast<uint4*>(pk.lo + idx);
+          dlo[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+          dlo[1] = make_uint4(lo[4], lo[5], lo[6], lo[7]);
+          *reinterpret_cast<uint4*>(pk.hi + idx) = make_uint4(hi[0] | hi[1] << 16, hi[2] | hi[3] << 16,
+                                                             hi[4] | hi[5] << 16, hi[6] | hi[7] << 16);
+        } else {
+          int64_t* out = slab + j * n + static_cast<int64_t>(r_dst) * kTile;
+#pragma unroll
+          for (int k = 0; k < 8; ++k) out[8 * t + k] = pi.mid(acc[k]);
+        }
+      };
+      keep(acc0, 0);
+      keep(acc1, 1);
+      return;
+    }
   }
   // kSplit: the whole block has summed its waves' shares and stages the
   // twiddles; wave 0 then finishes accumulator 0 and wave 1 accumulator 1.
@@ -2156,6 +2189,300 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Hoisted rotations left in the NTT domain.  floor(X / P) = (X - X_P) P^{-1}
+// is linear given X_P = X mod P, so a rotation whose next step is a product in
+// the NTT domain needs neither the accumulators' Q rows in the coefficient
+// domain nor a forward transform of the result: only the P rows go through
+// the inverse transform, z = -X_P P^{-1} is formed on the Q rows and
+// transformed, and the result is X P^{-1} + NTT(z) + sigma_g(NTT(c0)), the
+// same canonical residues.  Both kernels are bound by memory (accumulators,
+// z out and back, result).  31 rotations of 27 Q rows at logN = 16: inverse
+// columns of all rows, ModDown, gather and forward transform 1890 us; the P
+// rows' inverse and digits, xp_columns (547) and xp_tiles (534) 1230 us.
+// ---------------------------------------------------------------------------
+struct HoistNttArgs {
+  int64_t* acc;             // [2, K, Lqp, N]: Q rows NTT-domain sums, P rows coefficients, then digits
+  int64_t* out;             // [2, K, Lq, N]
+  const int64_t* c0;        // [Lq, N] NTT-domain Montgomery
+  const int64_t* p_scale;   // [Q0] P^{-1} R^{-1} mod q (rows below 2^42), P^{-1} R mod q (others)
+  const int64_t* p_inverse; // [Q0] P^{-1} mod q
+  const int64_t* galois;    // [K, 2] (g, g^{-1})
+  const KsDigit* pdig;
+  const NttRow* rows;
+  const int64_t* fwd_w;
+  const int64_t* fwd_wp;
+  ParamView params;
+  int64_t entries, lq, lqp, level, small_rows;
+  int log_n;
+};
+
+// The P rows' canonical residues replaced by their mixed-radix digits.  Grid
+// (N / 256, 2 K).
+template <int P>
+__global__ __launch_bounds__(kBlock) void k_ks_p_digits(HoistNttArgs a) {
+  const int64_t n = int64_t{1} << a.log_n;
+  int64_t* row = a.acc + (static_cast<int64_t>(blockIdx.y) * a.lqp + a.lq) * n + blockIdx.x * kBlock + threadIdx.x;
+  int64_t dg[P];
+#pragma unroll
+  for (int r = 0; r < P; ++r) dg[r] = row[r * n];
+  garner_p<P>(*a.pdig, a.rows + a.level + a.lq, dg);
+#pragma unroll
+  for (int r = 0; r < P; ++r) row[r * n] = dg[r];
+}
+
+// z R = -X_P P^{-1} R of one Q row through the forward column stages.  Work
+// items (column group, row, (component, entry)), XCD-contiguous so that the
+// rows of one entry read its digits from one L2.
+template <int S1, class P>
+__device__ __forceinline__ void xp_columns(const P& p, const HoistNttArgs& a, int64_t ce, int64_t j, int cg,
+                                           int64_t* lds) {
+  constexpr int R1 = 1 << S1;
+  constexpr int T = R1 / 16;
+  constexpr int C = kBlock / T;
+  const int64_t n = int64_t{1} << a.log_n;
+  const int64_t grow = a.level + j;
+  const KsDigit& pdig = *a.pdig;
+  const int prows = static_cast<int>(a.lqp - a.lq);
+  const int c = threadIdx.x % C;
+  const int t = threadIdx.x / C;
+  const int col = cg * C + c;
+  auto at = [&](int k) { return static_cast<uint32_t>((t + T * k) * kTile + col); };
+  const int64_t* digits = a.acc + (ce * a.lqp + a.lq) * n;
+  typename P::V v[16];
+  if constexpr (std::is_same<P, F64Fast>::value) {
+    // as ModDown's sum, without the x P^{-1} term
+    Global<double>* rec = global(pdig.f64_table) + grow * pdig.f64_stride;
+    const double start = f64_sum_start(2.0 * prows * 0x1.0p30 * p.q);
+    F64Sum s[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) s[k] = F64Sum{start, 0.0};
+#pragma nounroll
+    for (int r = 0; r < prows; ++r) {
+      const double clo = rec[r], chi = rec[prows + r];
+      int64_t x[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) x[k] = digits[static_cast<uint32_t>(r * n) + at(k)];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        f64_sum_add(s[k], clo, u64_to_f64(static_cast<uint64_t>(x[k]) & ((uint64_t{1} << 30) - 1)));
+        f64_sum_add(s[k], chi, u64_to_f64(static_cast<uint64_t>(x[k]) >> 30));
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 16; ++k) v[k] = p.to_mont(f64_sum_reduce(s[k], start, p.q, p.qinv));
+  } else {
+    const Mont m = load_mont(a.params, grow);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      int64_t xp = mont_mul(digits[at(k)], m.r2, m);
+      for (int r = 1; r < prows; ++r)
+        xp = add_lazy(xp, mont_mul(digits[static_cast<uint32_t>(r * n) + at(k)],
+                                   global(pdig.basis)[(r - 1) * pdig.basis_stride + grow], m), m.twice_q);
+      // X_P R times P^{-1} by REDC is X_P P^{-1}; negated, then times R
+      const int64_t z = canonicalize(sub_lazy(0, mont_mul(xp, a.p_inverse[grow], m), m.twice_q), m.twice_q);
+      v[k] = p.to_mont(static_cast<uint64_t>(z));
+    }
+  }
+  const int64_t* tw = a.fwd_w + grow * n;
+  const int64_t* twp = a.fwd_wp + grow * n;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int half = 8 >> s;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      if (k & half) continue;
+      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << s) + (k >> (4 - s))), s);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) lds[(t + T * k) * C + c] = p.mid(v[k]);
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = p.unmid(lds[(16 * t + k) * C + c]);
+#pragma unroll
+  for (int s = 4; s < S1; ++s) {
+    const int half = 1 << (S1 - 1 - s);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      if (k & half) continue;
+      p.fwd(v[k], v[k + half], p.tw(tw, twp, (1 << s) + ((16 * t + k) >> (S1 - s))), s);
+    }
+  }
+  int64_t* out = a.out + (ce * a.lq + j) * n;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) out[static_cast<uint32_t>((16 * t + k) * kTile + col)] = p.mid(v[k]);
+}
+
+template <int S1>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_ks_xp_columns(HoistNttArgs a) {
+  __shared__ int64_t lds[(1 << S1) * (kBlock / ((1 << S1) / 16))];
+  constexpr uint32_t kGroups = (1u << S1) / 16;
+  const uint32_t lq = static_cast<uint32_t>(a.lq);
+  const uint32_t w = xcd_remap(blockIdx.x, kGroups * lq * 2 * static_cast<uint32_t>(a.entries));
+  const int cg = static_cast<int>(w % kGroups);
+  const int64_t j = (w / kGroups) % lq;
+  const int64_t ce = w / (kGroups * lq);
+  const NttRow& row = a.rows[a.level + j];
+  if (j < a.small_rows) {
+    xp_columns<S1>(F64Fast(row), a, ce, j, cg, lds);
+  } else if (row.delta60) {
+    xp_columns<S1>(U64Pm(row), a, ce, j, cg, lds);
+  } else {
+    xp_columns<S1>(U64Fast(row), a, ce, j, cg, lds);
+  }
+}
+
+// The tile stages of z, plus X P^{-1} and (component 0) the rotated c0.
+template <class P>
+__device__ __forceinline__ void xp_tiles(const P& p, const HoistNttArgs& a, int64_t ce, int64_t j, int64_t g,
+                                         int64_t* lds) {
+  using V = typename P::V;
+  constexpr bool kF64 = std::is_same<V, double>::value;
+  const int64_t n = int64_t{1} << a.log_n;
+  const int64_t grow = a.level + j;
+  const NttRow& row = a.rows[grow];
+  const int m = threadIdx.x / kMacThreads;
+  const int t = threadIdx.x % kMacThreads;
+  const int r = static_cast<int>(g) * kMacTiles + m;
+  const int s0 = a.log_n - kTileLog;
+  int64_t* sh = lds + m * kTilePitch;
+  int64_t* tww = lds + kMacExchange + m * kTile;
+  int64_t* twp = tww + kMacTiles * kTile;  // Shoup companions
+  int64_t* tile = a.out + (ce * a.lq + j) * n + static_cast<int64_t>(r) * kTile;
+  V v[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) v[k] = p.unmid(tile[mac_e1(t, k)]);
+  // the accumulator's elements 8t .. 8t+7
+  const int64_t* slab = a.acc + ce * a.lqp * n;
+  uint64_t x[8];
+  if constexpr (kF64) {
+    const PackedInter pk = packed_slab(const_cast<int64_t*>(slab), a.small_rows, n);
+    const uint32_t idx = static_cast<uint32_t>(j * n + packed_index(r, 8 * t));
+    const uint4 l0 = *reinterpret_cast<const uint4*>(pk.lo + idx);
+    const uint4 l1 = *reinterpret_cast<const uint4*>(pk.lo + idx + 4);
+    const uint4 hh = *reinterpret_cast<const uint4*>(pk.hi + idx);
+    const uint32_t lo[8] = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
+    const uint32_t hi2[4] = {hh.x, hh.y, hh.z, hh.w};
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      x[k] = static_cast<uint64_t>(lo[k]) | static_cast<uint64_t>((hi2[k >> 1] >> (16 * (k & 1))) & 0xffffu) << 32;
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = static_cast<uint64_t>(slab[j * n + r * kTile + 8 * t + k]);
+  }
+  // sigma_g(c0) at those elements: out[i] = in[br(((2 br(i) + 1) g mod 2N - 1) / 2)]
+  int64_t c0[8] = {};
+  if (ce < a.entries) {
+    const uint32_t gal = static_cast<uint32_t>(a.galois[2 * ce]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint32_t i = static_cast<uint32_t>(r * kTile + 8 * t + k);
+      const uint32_t e = ((2 * brev_bits(i, a.log_n) + 1) * gal) & ((2u << a.log_n) - 1);
+      c0[k] = a.c0[j * n + brev_bits((e - 1) >> 1, a.log_n)];
+    }
+  }
+  {
+    const int64_t* w_row = a.fwd_w + grow * n;
+    const int64_t* wp_row = a.fwd_wp + grow * n;
+    for (int idx = t; idx < kTile - 1; idx += kMacThreads) {
+      const int st = 31 - __builtin_clz(idx + 1);
+      const int64_t gi = (int64_t{1} << (s0 + st)) + (static_cast<int64_t>(r) << st) + (idx + 1 - (1 << st));
+      tww[idx] = p.stage(w_row[gi]);
+      if constexpr (P::kCompanion) twp[idx] = wp_row[gi];
+    }
+  }
+  tile_sync();
+  auto tw_at = [&](int st, int e) {
+    const int slot = mac_tw_slot(st, e);
+    return p.tw_make(tww[slot], P::kCompanion ? twp[slot] : 0);
+  };
+#pragma unroll
+  for (int st = 0; st < 3; ++st) {
+    const int half = 4 >> st;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (k & half) continue;
+      p.fwd(v[k], v[k + half], tw_at(st, mac_e1(t, k)), st);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) sh[mac_lds(mac_e1(t, k))] = p.mid(v[k]);
+  tile_sync();
+#pragma unroll
+  for (int k = 0; k < 8; ++k) v[k] = p.unmid(sh[mac_lds(mac_e2(t, k))]);
+#pragma unroll
+  for (int st = 3; st < 6; ++st) {
+    const int half = 1 << (5 - st);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (k & half) continue;
+      p.fwd(v[k], v[k + half], tw_at(st, mac_e2(t, k)), st);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) sh[mac_lds(mac_e2(t, k))] = p.mid(v[k]);
+  tile_sync();
+#pragma unroll
+  for (int k = 0; k < 8; ++k) v[k] = p.unmid(sh[mac_lds(mac_e3(t, k))]);
+#pragma unroll
+  for (int st = 6; st < 8; ++st) {
+    const int half = 1 << (7 - st);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (k & half) continue;
+      p.fwd(v[k], v[k + half], tw_at(st, mac_e3(t, k)), st);
+    }
+  }
+  const uint64_t sc = static_cast<uint64_t>(a.p_scale[grow]);
+  int64_t res[8];
+  if constexpr (kF64) {
+    const double scd = u64_to_f64(sc);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      // |v| < 11q, the product below 0.53q, c0 below 2q
+      const double y = v[k] + f64_mulmod_signed(scd, u64_to_f64(x[k]), row.qd, row.qinv) +
+                       u64_to_f64(static_cast<uint64_t>(c0[k]));
+      res[k] = static_cast<int64_t>(f64_to_u64(p.canon(y)));
+    }
+  } else {
+    const Mont mt = load_mont(a.params, grow);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int64_t y = add_lazy(p.out_fwd(v[k]), mont_mul(static_cast<int64_t>(x[k]), static_cast<int64_t>(sc), mt),
+                                 mt.twice_q);
+      res[k] = canonicalize(add_lazy(y, canonicalize(c0[k], mt.twice_q), mt.twice_q), mt.twice_q);
+    }
+  }
+  // back through the exchange buffer for whole-line stores
+  tile_sync();
+#pragma unroll
+  for (int k = 0; k < 8; ++k) sh[mac_lds(mac_e3(t, k))] = res[k];
+  tile_sync();
+#pragma unroll
+  for (int k = 0; k < 8; ++k) tile[mac_e1(t, k)] = sh[mac_lds(mac_e1(t, k))];
+}
+
+// Work items ((component, entry) fastest, then row, then tile group).
+__global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_ks_xp_tiles(HoistNttArgs a) {
+  __shared__ int64_t lds[kMacExchange + 2 * kMacTiles * kTile];
+  const uint32_t groups = static_cast<uint32_t>((int64_t{1} << a.log_n) / (kTile * kMacTiles));
+  const uint32_t ces = 2 * static_cast<uint32_t>(a.entries);
+  const uint32_t lq = static_cast<uint32_t>(a.lq);
+  const uint32_t w = xcd_remap(blockIdx.x, groups * lq * ces);
+  const int64_t ce = w % ces;
+  const int64_t j = (w / ces) % lq;
+  const int64_t g = w / (ces * lq);
+  const NttRow& row = a.rows[a.level + j];
+  if (j < a.small_rows) {
+    xp_tiles(F64Fast(row), a, ce, j, g, lds);
+  } else if (row.delta60) {
+    xp_tiles(U64Pm(row), a, ce, j, g, lds);
+  } else {
+    xp_tiles(U64Fast(row), a, ce, j, g, lds);
+  }
+}
+
 // A call whose tile pass has at most this many pairs of tiles (rows x N / 512
 // x entries) takes the small-call launches.  Rotations, small-call launches
 // against the per-path ones on the same box: 52 against 99 us at 288 pairs
@@ -2258,7 +2585,8 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
                          fh_view3 out1, int32_t mode, const int64_t* rescale_inverse,
                          const int64_t* rescale_inverse_shoup, int64_t half_drop,
                          const int64_t* seed0, const int64_t* seed1, const int64_t* seed_scale,
-                         const int64_t* hoist_galois, bool use_side_stream, void* stream) {
+                         const int64_t* hoist_galois, bool use_side_stream, void* stream,
+                         const HoistNttArgs* ntt_result = nullptr) {
   FH_CHECK_ARG(log_n >= 12 && log_n <= 16, "fused key switch supports logN 12..16");
   FH_CHECK_ARG(batch >= 1 && batch <= 32767, "fused key switch batch %lld out of range",
                (long long)batch);
@@ -2268,7 +2596,7 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
   FH_CHECK_ARG(component.data && digit_table && p_digit_table && p_inverse_q && rns_params.data &&
                    ntt_rows && forward_twiddles && forward_twiddles_shoup && inverse_twiddles &&
                    inverse_twiddles_shoup && workspace_digits && workspace_inter && workspace_acc &&
-                   out0.data && out1.data,
+                   (ntt_result != nullptr || (out0.data && out1.data)),
                "fused key switch: null operand");
   FH_CHECK_ARG((key != nullptr) != (key_bases != nullptr), "pass exactly one of key / key_bases");
   FH_CHECK_ARG((galois_index_tables == nullptr) == (galois_sign_tables == nullptr),
@@ -2309,6 +2637,7 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
   a.seed1 = seed1;
   a.seed_scale = seed_scale;
   a.hoist_galois = hoist_galois;
+  a.keep_ntt = ntt_result != nullptr ? 1 : 0;
   // Hoisted rotations decompose and extend the one input entry once; the
   // MAC and everything after it run per entry.
   const bool hoist = hoist_galois != nullptr;
@@ -2475,6 +2804,56 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
     }
   }
 
+  if (ntt_result != nullptr) {
+    const int64_t prows = lqp - lq;
+    int rc = ntt::inverse_columns_internal(workspace_acc + lq * n, 2 * batch, prows, static_cast<int>(log_n), lqp * n, n,
+                                           static_cast<const NttRow*>(ntt_rows), inverse_twiddles,
+                                           inverse_twiddles_shoup, level + lq, kOutStdMac, 0, s);
+    if (rc != kOk) return rc;
+    HoistNttArgs h = *ntt_result;
+    h.acc = workspace_acc;
+    h.p_inverse = p_inverse_q;
+    h.galois = hoist_galois;
+    h.pdig = reinterpret_cast<const KsDigit*>(p_digit_table);
+    h.rows = static_cast<const NttRow*>(ntt_rows);
+    h.fwd_w = forward_twiddles;
+    h.fwd_wp = forward_twiddles_shoup;
+    h.params = a.params;
+    h.entries = batch;
+    h.lq = lq;
+    h.lqp = lqp;
+    h.level = level;
+    h.small_rows = small_rows;
+    h.log_n = static_cast<int>(log_n);
+    const dim3 pgrid(static_cast<uint32_t>(n / kBlock), static_cast<uint32_t>(2 * batch));
+    switch (prows) {
+      case 1: hipLaunchKernelGGL(k_ks_p_digits<1>, pgrid, dim3(kBlock), 0, s, h); break;
+      case 2: hipLaunchKernelGGL(k_ks_p_digits<2>, pgrid, dim3(kBlock), 0, s, h); break;
+      case 3: hipLaunchKernelGGL(k_ks_p_digits<3>, pgrid, dim3(kBlock), 0, s, h); break;
+      case 4: hipLaunchKernelGGL(k_ks_p_digits<4>, pgrid, dim3(kBlock), 0, s, h); break;
+      case 5: hipLaunchKernelGGL(k_ks_p_digits<5>, pgrid, dim3(kBlock), 0, s, h); break;
+      default: hipLaunchKernelGGL(k_ks_p_digits<6>, pgrid, dim3(kBlock), 0, s, h); break;
+    }
+    FH_CHECK_LAUNCH("hoisted rotations: P digits");
+    const int64_t xp_blocks = (kTile / C) * lq * 2 * batch;
+    FH_CHECK_ARG(xp_blocks <= 0x7fffffff && groups * lq * 2 * batch <= 0x7fffffff, "key switch grid too large");
+#define FH_XP_CASE(S) \
+  case S: hipLaunchKernelGGL(k_ks_xp_columns<S>, dim3(static_cast<uint32_t>(xp_blocks)), dim3(kBlock), 0, s, h); break;
+    switch (s1) {
+      FH_XP_CASE(4)
+      FH_XP_CASE(5)
+      FH_XP_CASE(6)
+      FH_XP_CASE(7)
+      default:
+        FH_XP_CASE(8)
+    }
+#undef FH_XP_CASE
+    FH_CHECK_LAUNCH("hoisted rotations: X mod P columns");
+    hipLaunchKernelGGL(k_ks_xp_tiles, dim3(static_cast<uint32_t>(groups * lq * 2 * batch)), dim3(kMacBlock), 0, s, h);
+    FH_CHECK_LAUNCH("hoisted rotations: X mod P tiles");
+    return kOk;
+  }
+
   // Both accumulators as one [2B, Lqp, N] inverse transform.
   // The tile stages of this inverse ran inside the MAC kernel.
   int st = ntt::inverse_columns_internal(workspace_acc, 2 * batch, lqp, static_cast<int>(log_n), lqp * n, n,
@@ -2599,6 +2978,36 @@ FH_API int fh_keyswitch_hoisted(fh_view3 component, int64_t entries, int64_t lq,
                               galois_sign_tables, workspace_digits, workspace_inter, workspace_acc, c0, none,
                               out0, out1, mode, nullptr, nullptr, 0, nullptr, nullptr, nullptr, galois_elements,
                               /*use_side_stream=*/true, stream);
+}
+
+// Hoisted rotations whose results stay in the NTT domain.  See
+// include/fhelium_amd.h.
+FH_API int fh_keyswitch_hoisted_ntt(fh_view3 component, int64_t entries, int64_t lq, int64_t lqp, int64_t level,
+                                    int64_t log_n, int64_t small_rows, const int64_t* digit_table,
+                                    int64_t digit_count, const int64_t* p_digit_table, const int64_t* p_inverse_q,
+                                    const int64_t* p_scale, fh_table2 rns_params, const void* ntt_rows,
+                                    const int64_t* forward_twiddles, const int64_t* forward_twiddles_shoup,
+                                    const int64_t* inverse_twiddles, const int64_t* inverse_twiddles_shoup,
+                                    const int64_t* key_bases, int64_t key_stride_digit, int64_t key_stride_comp,
+                                    int64_t key_stride_row, const int64_t* galois_elements,
+                                    int64_t* workspace_digits, int64_t* workspace_inter, int64_t* workspace_acc,
+                                    const int64_t* c0_ntt, int64_t* out, void* stream) {
+  FH_CHECK_ARG(galois_elements != nullptr && key_bases != nullptr && c0_ntt != nullptr && out != nullptr &&
+                   p_scale != nullptr,
+               "hoisted rotations need per-entry keys, Galois elements, the scale table and the base c0");
+  FH_CHECK_ARG(small_rows > 0 && small_rows <= lq && entries <= 32767,
+               "NTT-domain hoisted rotations need leading rows below 2^42 and integer P rows");
+  HoistNttArgs h{};
+  h.out = out;
+  h.c0 = c0_ntt;
+  h.p_scale = p_scale;
+  const fh_view3 none{nullptr, 0, 0, 0};
+  return keyswitch_fused_impl(component, entries, lq, lqp, level, log_n, small_rows, digit_table, digit_count,
+                              p_digit_table, p_inverse_q, rns_params, ntt_rows, forward_twiddles,
+                              forward_twiddles_shoup, inverse_twiddles, inverse_twiddles_shoup, nullptr, key_bases,
+                              key_stride_digit, key_stride_comp, key_stride_row, nullptr, nullptr, workspace_digits,
+                              workspace_inter, workspace_acc, none, none, none, none, /*mode=*/1, nullptr, nullptr, 0,
+                              nullptr, nullptr, nullptr, galois_elements, /*use_side_stream=*/true, stream, &h);
 }
 
 // fh_keyswitch_fused with its workspaces carved from the device's static

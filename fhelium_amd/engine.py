@@ -1341,6 +1341,24 @@ class CkksEngine:
             out[:, zero] = ct.data.reshape(2, 1, lq, n)
         return Ciphertext(out, ct.level, ct.scale, "coefficient", "standard", ct.modulus_basis)
 
+    def rotate_hoisted_ntt(self, ct: Ciphertext, rotation_steps: list[int],
+                           ct_ntt: Ciphertext | None = None) -> Ciphertext:
+        """coefficient_domain_to_ntt_domain(rotate_hoisted(ct, steps)).  Where
+        the chain allows it the rotations stay in the NTT domain after the key
+        products and meet ``ct_ntt`` (ct in the NTT domain, transformed here
+        if not given) there."""
+
+        self._assert_rotation_ciphertext(ct)
+        steps = [RotationKey.canonical_step(s, self.config.N) for s in rotation_steps]
+        if (ct.batch_shape not in ((), (1,)) or not self.fused_keyswitch or not steps or 0 in steps
+                or not self.key_switcher.hoisted_ntt_ready(ct.level)):
+            return self.coefficient_domain_to_ntt_domain(self.rotate_hoisted(ct, rotation_steps))
+        if ct_ntt is None:
+            ct_ntt = self.coefficient_domain_to_ntt_domain(ct)
+        data = self.key_switcher.key_switch_hoisted(ct.data[1], ct.data[0], [self.rotation_key(s) for s in steps],
+                                                    ct.level, base0_ntt=ct_ntt.data[0])
+        return Ciphertext(data, ct.level, ct.scale, "ntt", "montgomery", ct.modulus_basis)
+
     # convenience: HMult as the reference's examples compose it (README.md:66-69)
     def hmult(self, a: Ciphertext, b: Ciphertext) -> Ciphertext:
         """rescale(relinearize(multiply(NTT(a), NTT(b)))).  With the fused

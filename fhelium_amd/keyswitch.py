@@ -278,8 +278,21 @@ class HybridKeySwitcher:
             cache[tag] = hit
         return hit
 
+    def hoisted_ntt_ready(self, level: int) -> bool:
+        """Whether key_switch_hoisted can leave its results in the NTT domain:
+        fast arithmetic, leading Q rows below 2^42, and every other row,
+        the P rows among them, an integer row."""
+
+        start = self.rt.row_start(level)
+        small = [q < SMALL_PRIME_LIMIT for q in self.config.moduli[start:]]
+        rest = self.config.moduli[start + sum(small):]
+        return (self.rt.ntt._mode == 1 and 12 <= self.config.logN <= 16 and small[0]
+                and sum(small) <= self.config.num_q_primes - start
+                and all(q >= rns.WIDE_PRIME_LIMIT for q in rest))
+
     def key_switch_hoisted(self, component: torch.Tensor, base0: torch.Tensor,
-                           keys: list[KeySwitchKey], level: int) -> torch.Tensor:
+                           keys: list[KeySwitchKey], level: int,
+                           base0_ntt: torch.Tensor | None = None) -> torch.Tensor:
         """Hoisted rotations of one ciphertext (c0 = ``base0``, c1 =
         ``component``, each [Q_level, N] or [1, Q_level, N], canonical
         standard) by several rotation keys, in nine launches
@@ -288,7 +301,12 @@ class HybridKeySwitcher:
         map of the key's element, as prepare_rotation_digits +
         _apply_prepared_rotation do (hybrid_keyswitch.py:373-504), with
         sigma_g(c0) added canonically (ckks_engine.py:3767-3820).  Returns
-        [2, K, Q_level, N]: entry e is the rotation by keys[e]."""
+        [2, K, Q_level, N]: entry e is the rotation by keys[e].
+
+        With ``base0_ntt`` (base0 in the NTT domain, Montgomery; needs
+        hoisted_ntt_ready) the results are in the NTT domain, canonical
+        Montgomery (fh_keyswitch_hoisted_ntt): only the accumulators' P rows
+        are inverse transformed and only -X_P P^{-1} is transformed forward."""
 
         from fhelium_amd import _native as nat
 
@@ -315,14 +333,16 @@ class HybridKeySwitcher:
         c0 = base0.reshape(1, lq, n)
         table = self.digit_table(level)
         dnum = table.size(0)
-        ws_digits = torch.empty((k, lq, n), dtype=torch.int64, device=dev)
+        if base0_ntt is not None:
+            if not self.hoisted_ntt_ready(level):
+                raise ValueError("this chain's hoisted rotations do not stay in the NTT domain")
+            _check_operand("base0_ntt", base0_ntt, 1, lq, n, dev)
+            c0_ntt = base0_ntt.reshape(lq, n).contiguous()
+        ws_digits = torch.empty((k if base0_ntt is None else 1, lq, n), dtype=torch.int64, device=dev)
         ws_inter = torch.empty((1, dnum, lqp, n), dtype=torch.int64, device=dev)
         ws_acc = torch.empty((2, k, lqp, n), dtype=torch.int64, device=dev)
         out = torch.empty((2, k, lq, n), dtype=torch.int64, device=dev)
         bases = self._address_table(data, dev)
-        tables = [rt.coefficient_galois(g) for g in elements]
-        gal_idx = self._address_table([t[0] for t in tables], dev)
-        gal_sgn = self._address_table([t[1] for t in tables], dev)
         pairs = self._galois_pairs(elements, dev)
         start = rt.row_start(level)
         small = [q < SMALL_PRIME_LIMIT for q in cfg.moduli[start: start + lqp]]
@@ -335,13 +355,23 @@ class HybridKeySwitcher:
             ev0 = torch.cuda.Event(enable_timing=True)
             ev1 = torch.cuda.Event(enable_timing=True)
             ev0.record()
-        nat.call("fh_keyswitch_hoisted", nat.v3(comp), k, lq, lqp, start, cfg.logN, small_rows,
-                 table.data_ptr(), dnum, self.p_digit_table().data_ptr(), rt.p_inverse_q.data_ptr(),
-                 nat.t2(rt.rns_params), nt.rows.data_ptr(), nt.fwd.data_ptr(), nt.fwd_shoup.data_ptr(),
-                 nt.inv.data_ptr(), nt.inv_shoup.data_ptr(), bases.data_ptr(), ref.stride(0), ref.stride(1),
-                 ref.stride(2), pairs.data_ptr(), gal_idx.data_ptr(), gal_sgn.data_ptr(), ws_digits.data_ptr(),
-                 ws_inter.data_ptr(), ws_acc.data_ptr(), nat.v3(c0), nat.v3(out[0]), nat.v3(out[1]),
-                 rt.ntt._mode, nat.stream_ptr(dev))
+        common = (nat.t2(rt.rns_params), nt.rows.data_ptr(), nt.fwd.data_ptr(), nt.fwd_shoup.data_ptr(),
+                  nt.inv.data_ptr(), nt.inv_shoup.data_ptr(), bases.data_ptr(), ref.stride(0), ref.stride(1),
+                  ref.stride(2), pairs.data_ptr())
+        workspaces = (ws_digits.data_ptr(), ws_inter.data_ptr(), ws_acc.data_ptr())
+        if base0_ntt is not None:
+            nat.call("fh_keyswitch_hoisted_ntt", nat.v3(comp), k, lq, lqp, start, cfg.logN, small_rows,
+                     table.data_ptr(), dnum, self.p_digit_table().data_ptr(), rt.p_inverse_q.data_ptr(),
+                     rt.moddown_ntt_scale.data_ptr(), *common, *workspaces, c0_ntt.data_ptr(), out.data_ptr(),
+                     nat.stream_ptr(dev))
+        else:
+            tables = [rt.coefficient_galois(g) for g in elements]
+            gal_idx = self._address_table([t[0] for t in tables], dev)
+            gal_sgn = self._address_table([t[1] for t in tables], dev)
+            nat.call("fh_keyswitch_hoisted", nat.v3(comp), k, lq, lqp, start, cfg.logN, small_rows,
+                     table.data_ptr(), dnum, self.p_digit_table().data_ptr(), rt.p_inverse_q.data_ptr(),
+                     *common, gal_idx.data_ptr(), gal_sgn.data_ptr(), *workspaces, nat.v3(c0), nat.v3(out[0]),
+                     nat.v3(out[1]), rt.ntt._mode, nat.stream_ptr(dev))
         if rec is not None:
             ev1.record()
             limb = n * 8

@@ -4,10 +4,11 @@ The reference's packed matrix-vector benchmark
 (fhelium/benchmarks/standalone/packed_matrix_vector.py:120-170) computes
 y = sum_i d_i * rot(x, i) with hoisted rotations (rotate_many_with_keys),
 plaintext products and additions.  Here the K - 1 rotations of the one
-ciphertext run as one hoisted fused key switch (``CkksEngine.rotate_hoisted``:
-c1 is decomposed and extended once, and every rotation key's MAC reads that
-intermediate through its NTT-domain Galois map), so the rotated ciphertexts
-carry exactly the reference's hoisted residues.  The plaintext products and
+ciphertext run as one hoisted fused key switch
+(``CkksEngine.rotate_hoisted_ntt``: c1 is decomposed and extended once, every
+rotation key's MAC reads that intermediate through its NTT-domain Galois map,
+and the results stay in the NTT domain for the products), so the rotated
+ciphertexts carry exactly the reference's hoisted residues.  The plaintext products and
 their sum run as one inner-product pass over the rotated batch (canonical
 modular sums do not depend on the order of addition, so this equals
 multiply_plaintext followed by additions); one inverse NTT and one rescale
@@ -59,8 +60,7 @@ def diagonal_matvec(engine, ct: Ciphertext, diagonals: Plaintext, *, chunk: int 
     accumulate(K.plaintext_inner_product(x0.data.unsqueeze(1), diagonals.data[0:1], params))
     for start in range(1, k_total, chunk):
         stop = min(start + chunk, k_total)
-        rotated = engine.rotate_hoisted(ct, list(range(start, stop)))  # entry i: rot(x, start + i)
-        ntt = engine.coefficient_domain_to_ntt_domain(rotated)
+        ntt = engine.rotate_hoisted_ntt(ct, list(range(start, stop)), x0)  # entry i: rot(x, start + i)
         accumulate(K.plaintext_inner_product(ntt.data, diagonals.data[start:stop], params))
     summed = Ciphertext(acc, ct.level, ct.scale * diagonals.scale, "ntt", "montgomery")
     return engine.rescale_to_next_level(engine.ntt_domain_to_coefficient_domain(summed))

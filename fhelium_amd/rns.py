@@ -272,6 +272,14 @@ class HostTables:
             [p_product % moduli[i] if moduli[i] < WIDE_PRIME_LIMIT else (p_product * R) % moduli[i]
              for i in self.layout.prime_ids(0)], dtype=torch.int64
         )
+        # P^{-1} for accumulators that stay in the NTT domain, to Montgomery
+        # form: they hold x R^2 on the rows below 2^42 (a plain product by
+        # P^{-1} R^{-1} leaves x P^{-1} R) and x R on the others (REDC by
+        # P^{-1} R).
+        self.moddown_ntt_scale = torch.tensor(
+            [pow(p_product * R, -1, moduli[i]) if moduli[i] < BINARY64_PRIME_LIMIT
+             else pow(p_product, -1, moduli[i]) * R % moduli[i] for i in self.layout.prime_ids(0)], dtype=torch.int64
+        )
         self.moddown_binary64 = moddown_binary64_table(moduli, self.layout.p_prime_ids,
                                                        self.layout.prime_ids(0))
 

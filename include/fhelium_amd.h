@@ -315,6 +315,26 @@ int fh_keyswitch_hoisted(fh_view3 component, int64_t entries, int64_t lq, int64_
                          int64_t* workspace_acc, fh_view3 base0, fh_view3 out0, fh_view3 out1, int32_t mode,
                          void* stream);
 
+/* The same rotations left in the NTT domain for a product there: out is
+ * [2, entries, lq, N], canonical Montgomery, equal to fh_keyswitch_hoisted
+ * (fast arithmetic) followed by a forward NTT to Montgomery form.
+ *   p_scale          [Q0] (P 2^62)^{-1} mod q for q < 2^42, P^{-1} 2^62 mod q
+ *                    for the others
+ *   c0_ntt           [lq, N] contiguous: c0 in the NTT domain, Montgomery, below 2q
+ *   workspace_digits [lq, N]; the other workspaces as above
+ * Needs 0 < small_rows <= lq and every other row (the P rows among them) at
+ * least 2^50 + 2^30. */
+int fh_keyswitch_hoisted_ntt(fh_view3 component, int64_t entries, int64_t lq, int64_t lqp, int64_t level,
+                             int64_t log_n, int64_t small_rows, const int64_t* digit_table,
+                             int64_t digit_count, const int64_t* p_digit_table, const int64_t* p_inverse_q,
+                             const int64_t* p_scale, fh_table2 rns_params, const void* ntt_rows,
+                             const int64_t* forward_twiddles, const int64_t* forward_twiddles_shoup,
+                             const int64_t* inverse_twiddles, const int64_t* inverse_twiddles_shoup,
+                             const int64_t* key_bases, int64_t key_stride_digit, int64_t key_stride_comp,
+                             int64_t key_stride_row, const int64_t* galois_elements,
+                             int64_t* workspace_digits, int64_t* workspace_inter, int64_t* workspace_acc,
+                             const int64_t* c0_ntt, int64_t* out, void* stream);
+
 /* fh_keyswitch_fused without caller workspaces: no counterpart in the
  * reference.  It is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
