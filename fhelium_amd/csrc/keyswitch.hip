@@ -829,77 +829,68 @@ __device__ __forceinline__ int mac_tw_slot(int st, int e) { return (1 << st) - 1
 // slot k.
 __device__ __forceinline__ uint32_t brev_bits(uint32_t x, int bits) { return __brev(x) >> (32 - bits); }
 
-struct HoistSlot {
-  int dst_tile;   // destination tile of source tile r'
-  int dst_base;   // 8 * destination thread of source thread t
-  int h;          // carry of the destination thread's slot map
-};
-
-__device__ __forceinline__ HoistSlot hoist_slot(int r_src, int t, uint32_t g, uint32_t ginv, int log_n) {
+// Destination tile of source tile r_src under the NTT-domain map of g: the
+// map takes whole tiles to tiles.
+__device__ __forceinline__ int hoisted_tile(int r_src, uint32_t ginv, int log_n) {
   const int l8 = log_n - kTileLog;
   const uint32_t low_mask = (1u << (log_n - 7)) - 1;  // mod 2^(L-7)
-  const uint32_t e_src = 2 * brev_bits(static_cast<uint32_t>(r_src), l8) + 1;
-  const uint32_t e_dst = (e_src * ginv) & low_mask;
-  HoistSlot hs;
-  hs.dst_tile = static_cast<int>(brev_bits((e_dst - 1) >> 1, l8));
-  const uint32_t u = ((2 * brev_bits(static_cast<uint32_t>(hs.dst_tile), l8) + 1) * g) & ((2u << log_n) - 1);
-  const uint32_t c = u >> (log_n - 7);
-  const uint32_t td = brev_bits(((brev_bits(static_cast<uint32_t>(t), 5) - c) * ginv) & 31u, 5);
-  hs.dst_base = static_cast<int>(8 * td);
-  hs.h = static_cast<int>((((g * brev_bits(td, 5) + c) & 255u) >> 5));
-  return hs;
+  const uint32_t e_dst = ((2 * brev_bits(static_cast<uint32_t>(r_src), l8) + 1) * ginv) & low_mask;
+  return static_cast<int>(brev_bits((e_dst - 1) >> 1, l8));
 }
-// Destination slot (0..7) of source slot k.
-__device__ __forceinline__ int hoist_dst_slot(int k, int h, uint32_t ginv) {
-  return static_cast<int>(brev_bits(((brev_bits(static_cast<uint32_t>(k), 3) - static_cast<uint32_t>(h)) * ginv) & 7u, 3));
+// Source of coefficient i: out[i] = in[br(((2 br(i) + 1) g mod 2N - 1) / 2)].
+__device__ __forceinline__ uint32_t hoisted_source(uint32_t i, uint32_t g, int log_n) {
+  const uint32_t e = ((2 * brev_bits(i, log_n) + 1) * g) & ((2u << log_n) - 1);
+  return brev_bits((e - 1) >> 1, log_n);
 }
+// Destination elements of a hoisted MAC thread: pairs, so that 32 threads read
+// whole lines of the key in 16-byte words.
+__device__ __forceinline__ int mac_pair(int t, int k) { return ((k >> 1) << 6) | 2 * t | (k & 1); }
 
-// Destination of a MAC block's sums.  For a hoisted rotation the block's
-// tiles r are source tiles of the NTT-domain Galois map: the accumulators
-// belong to tile r_dst, and this thread's source slot k to destination
-// element dst_base + slot k (3 bits per slot in slot_map).  Otherwise
-// r_dst = r and slot k is element 8t + k.
-struct MacDest {
-  int r_dst;
-  int dst_base;
-  uint32_t slot_map;
-  __device__ __forceinline__ int slot(int k) const {
-    return dst_base + static_cast<int>((slot_map >> (3 * k)) & 7u);
-  }
-};
-
-__device__ __forceinline__ MacDest hoisted_dest(const KsArgs& a, int r, int t, int64_t b) {
-  const uint32_t hg = static_cast<uint32_t>(a.hoist_galois[2 * b]);
-  const uint32_t hginv = static_cast<uint32_t>(a.hoist_galois[2 * b + 1]);
-  const HoistSlot hs = hoist_slot(r, t, hg, hginv, a.log_n);
-  MacDest d{hs.dst_tile, hs.dst_base, 0u};
-#pragma unroll
-  for (int k = 0; k < 8; ++k) d.slot_map |= static_cast<uint32_t>(hoist_dst_slot(k, hs.h, hginv)) << (3 * k);
-  return d;
-}
-
-// The accumulators of tile dst.r_dst (thread t holding elements 8t..8t+7):
+// The accumulators of tile r_dst (thread t holding elements 8t..8t+7):
 // the first 8 inverse stages, which act inside the tile (fast arithmetic, as
 // the rest of the inverse), then the working-format store the inverse column
-// pass reads.  With kHoist the sums arrive in source order and first move to
-// the destination layout through the exchange buffer.
+// pass reads.  With kHoist the sums arrive as the elements mac_pair(t, k) and
+// first move to that layout through the exchange buffer.
 template <bool kHoist, bool kSplit, class PI, class Acc>
-__device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b, int t, const MacDest& dst,
+__device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b, int t, int r_dst,
                                            int64_t* sh, int64_t* tww, int64_t* twp, Acc (&acc0)[8],
                                            Acc (&acc1)[8]) {
   const int64_t n = int64_t{1} << a.log_n;
   const int64_t grow = a.level + j;
   const NttRow& row = a.rows[grow];
-  const int r_dst = dst.r_dst;
   const PI pi(row);
   if constexpr (kHoist) {
-    auto to_dst = [&](Acc (&acc)[8]) {
+    if (a.keep_ntt && j < a.lq) {
+      // rows below 2^42 packed and canonical, the others as they are (below 2q)
+      auto keep = [&](Acc (&acc)[8], int64_t component) {
+        int64_t* slab = a.acc + (component * a.batch + b) * a.lqp * n;
+        if constexpr (std::is_same<PI, F64Fast>::value) {
+          const PackedInter pk = packed_slab(slab, a.small_rows, n);
+#pragma unroll
+          for (int k = 0; k < 8; k += 2) {
+            const uint32_t idx = static_cast<uint32_t>(j * n + packed_index(r_dst, mac_pair(t, k)));
+            const uint64_t u0 = f64_to_u64(pi.canon(acc[k])), u1 = f64_to_u64(pi.canon(acc[k + 1]));
+            *reinterpret_cast<uint2*>(pk.lo + idx) = make_uint2(static_cast<uint32_t>(u0), static_cast<uint32_t>(u1));
+            *reinterpret_cast<uint32_t*>(pk.hi + idx) =
+                static_cast<uint32_t>(u0 >> 32) | static_cast<uint32_t>(u1 >> 32) << 16;
+          }
+        } else {
+          int64_t* out = slab + j * n + static_cast<int64_t>(r_dst) * kTile;
+#pragma unroll
+          for (int k = 0; k < 8; ++k) out[mac_pair(t, k)] = pi.mid(acc[k]);
+        }
+      };
+      keep(acc0, 0);
+      keep(acc1, 1);
+      return;
+    }
+    auto to_e3 = [&](Acc (&acc)[8]) {
       tile_sync();  // earlier readers of the exchange buffer are done
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         int64_t bits;
         __builtin_memcpy(&bits, &acc[k], sizeof(bits));
-        sh[mac_lds(dst.slot(k))] = bits;
+        sh[mac_lds(mac_pair(t, k))] = bits;
       }
       tile_sync();
 #pragma unroll
@@ -908,38 +899,8 @@ __device__ __forceinline__ void mac_finish(const KsArgs& a, int64_t j, int64_t b
         __builtin_memcpy(&acc[k], &bits, sizeof(bits));
       }
     };
-    to_dst(acc0);
-    to_dst(acc1);
-    if (a.keep_ntt && j < a.lq) {
-      // elements 8t .. 8t+7 of the destination tile: rows below 2^42 packed
-      // and canonical, the others as they are (below 2q)
-      auto keep = [&](Acc (&acc)[8], int64_t component) {
-        int64_t* slab = a.acc + (component * a.batch + b) * a.lqp * n;
-        if constexpr (std::is_same<PI, F64Fast>::value) {
-          const PackedInter pk = packed_slab(slab, a.small_rows, n);
-          const uint32_t idx = static_cast<uint32_t>(j * n + packed_index(r_dst, 8 * t));
-          uint32_t lo[8], hi[8];
-#pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            const uint64_t u = f64_to_u64(pi.canon(acc[k]));
-            lo[k] = static_cast<uint32_t>(u);
-            hi[k] = static_cast<uint32_t>(u >> 32);
-          }
-          uint4* dlo = reinterpret_cast<uint4*>(pk.lo + idx);
-          dlo[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-          dlo[1] = make_uint4(lo[4], lo[5], lo[6], lo[7]);
-          *reinterpret_cast<uint4*>(pk.hi + idx) = make_uint4(hi[0] | hi[1] << 16, hi[2] | hi[3] << 16,
-                                                             hi[4] | hi[5] << 16, hi[6] | hi[7] << 16);
-        } else {
-          int64_t* out = slab + j * n + static_cast<int64_t>(r_dst) * kTile;
-#pragma unroll
-          for (int k = 0; k < 8; ++k) out[8 * t + k] = pi.mid(acc[k]);
-        }
-      };
-      keep(acc0, 0);
-      keep(acc1, 1);
-      return;
-    }
+    to_e3(acc0);
+    to_e3(acc1);
   }
   // kSplit: the whole block has summed its waves' shares and stages the
   // twiddles; wave 0 then finishes accumulator 0 and wave 1 accumulator 1.
@@ -1272,7 +1233,7 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
       facc1[k] = p.reduce(facc1[k]);
     }
   }
-  const MacDest dst{r, 8 * t, 0u};
+  const int r_dst = r;
   if constexpr (kSplit) {
     // Wave c collects accumulator c of every wave (exchange buffers take the
     // shares).  Binary64 shares add exactly (17 terms below 0.53q in all, or
@@ -1308,9 +1269,9 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
     }
   }
   if constexpr (kF64) {
-    mac_finish<false, kSplit, std::conditional_t<P::kWide, P, F64Fast>>(a, j, b, t, dst, sh, tww, twp, facc0, facc1);
+    mac_finish<false, kSplit, std::conditional_t<P::kWide, P, F64Fast>>(a, j, b, t, r_dst, sh, tww, twp, facc0, facc1);
   } else {
-    mac_finish<false, kSplit, P>(a, j, b, t, dst, sh, tww, twp, uacc0, uacc1);
+    mac_finish<false, kSplit, P>(a, j, b, t, r_dst, sh, tww, twp, uacc0, uacc1);
   }
 }
 
@@ -1550,9 +1511,17 @@ __device__ __forceinline__ void tiles_mac_hoisted(const P& p, const KsArgs& a, i
   int64_t* key_digit = lds + kMacExchange + kMacTiles * kTile * (kF64 ? 1 : 2);
   if (threadIdx.x < a.dnum) key_digit[threadIdx.x] = a.dig[threadIdx.x].key_digit;
   __syncthreads();
-  const MacDest dst = hoisted_dest(a, r, t, b);
+  const uint32_t hg = static_cast<uint32_t>(a.hoist_galois[2 * b]);
+  const int r_dst = hoisted_tile(r, static_cast<uint32_t>(a.hoist_galois[2 * b + 1]), a.log_n);
+  // exchange slot of the source of each of this thread's elements
+  int src[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const uint32_t i = static_cast<uint32_t>(r_dst * kTile + mac_pair(t, k));
+    src[k] = mac_lds(static_cast<int>(hoisted_source(i, hg, a.log_n) & (kTile - 1)));
+  }
   Global<int64_t>* key = global(a.key_bases ? reinterpret_cast<const int64_t*>(a.key_bases[b]) : a.key);
-  const int64_t dst_off = static_cast<int64_t>(dst.r_dst) * kTile;
+  const int64_t dst_off = static_cast<int64_t>(r_dst) * kTile;
   double facc0[8], facc1[8];
   uint64_t uacc0[8], uacc1[8];
   WideAcc wacc0[8], wacc1[8];
@@ -1566,61 +1535,87 @@ __device__ __forceinline__ void tiles_mac_hoisted(const P& p, const KsArgs& a, i
   const uint32_t pidx = static_cast<uint32_t>(j * n + packed_index(r, 8 * t));
   // software pipeline: the next digit's key words and values load while
   // this digit's products run
-  auto load_digit = [&](int64_t di, int64_t (&w0)[8], int64_t (&w1)[8], V (&v)[8]) {
-    Global<int64_t>* k0 = key + key_digit[di] * a.key_sd + grow * a.key_sr + dst_off;
+  using Pair = int64_t __attribute__((ext_vector_type(2), aligned(8)));
+  constexpr int kRaw = kPacked ? 3 : 4;
+  auto load_digit = [&](int64_t di, Pair (&w0)[4], Pair (&w1)[4], uint4 (&raw)[kRaw]) {
+    Global<int64_t>* k0 = key + key_digit[di] * a.key_sd + grow * a.key_sr + dst_off + 2 * t;
     Global<int64_t>* k1 = k0 + a.key_sc;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      w0[k] = k0[dst.slot(k)];
-      w1[k] = k1[dst.slot(k)];
+    for (int k = 0; k < 4; ++k) {
+      w0[k] = *reinterpret_cast<Global<Pair>*>(k0 + 64 * k);
+      w1[k] = *reinterpret_cast<Global<Pair>*>(k1 + 64 * k);
     }
     if constexpr (kPacked) {
       const PackedInter pk = packed_slab(a.inter + di * digit_stride, a.small_rows, n);
-      const uint4 l0 = *reinterpret_cast<const uint4*>(pk.lo + pidx);
-      const uint4 l1 = *reinterpret_cast<const uint4*>(pk.lo + pidx + 4);
-      const uint4 hh = *reinterpret_cast<const uint4*>(pk.hi + pidx);
-      const uint32_t lo[8] = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
-      const uint32_t hi2[4] = {hh.x, hh.y, hh.z, hh.w};
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const uint64_t h = (hi2[k >> 1] >> (16 * (k & 1))) & 0xffffu;
-        v[k] = u64_to_f64(static_cast<uint64_t>(lo[k]) | (h << 32));
-      }
+      raw[0] = *reinterpret_cast<const uint4*>(pk.lo + pidx);
+      raw[1] = *reinterpret_cast<const uint4*>(pk.lo + pidx + 4);
+      raw[2] = *reinterpret_cast<const uint4*>(pk.hi + pidx);
     } else {
       const int64_t* tl = tile + di * digit_stride;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = p.unmid(tl[mac_e3(t, k)]);
+      for (int k = 0; k < 4; ++k) raw[k] = *reinterpret_cast<const uint4*>(tl + mac_pair(t, 2 * k));
     }
   };
-  int64_t wa0[8], wa1[8], wb0[8], wb1[8];
-  V va[8], vb[8];
-  load_digit(0, wa0, wa1, va);
-  auto mac_digit = [&](int64_t (&w0)[8], int64_t (&w1)[8], V (&v)[8]) {
+  // the digit's values, through the Galois map by way of the exchange buffer
+  auto values = [&](const uint4 (&raw)[kRaw], V (&v)[8]) {
+    tile_sync();
+    if constexpr (kPacked) {
+      const uint32_t lo[8] = {raw[0].x, raw[0].y, raw[0].z, raw[0].w, raw[1].x, raw[1].y, raw[1].z, raw[1].w};
+      const uint32_t hi2[4] = {raw[2].x, raw[2].y, raw[2].z, raw[2].w};
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint64_t h = (hi2[k >> 1] >> (16 * (k & 1))) & 0xffffu;
+        sh[mac_lds(mac_e3(t, k))] = static_cast<int64_t>(static_cast<uint64_t>(lo[k]) | (h << 32));
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        sh[mac_lds(mac_pair(t, 2 * k))] = static_cast<int64_t>(static_cast<uint64_t>(raw[k].x) | static_cast<uint64_t>(raw[k].y) << 32);
+        sh[mac_lds(mac_pair(t, 2 * k + 1))] = static_cast<int64_t>(static_cast<uint64_t>(raw[k].z) | static_cast<uint64_t>(raw[k].w) << 32);
+      }
+    }
+    tile_sync();
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
+      if constexpr (kPacked) {
+        v[k] = u64_to_f64(static_cast<uint64_t>(sh[src[k]]));
+      } else {
+        v[k] = p.unmid(sh[src[k]]);
+      }
+    }
+  };
+  Pair wa0[4], wa1[4], wb0[4], wb1[4];
+  uint4 ra[kRaw], rb[kRaw];
+  load_digit(0, wa0, wa1, ra);
+  auto mac_digit = [&](const Pair (&p0)[4], const Pair (&p1)[4], const uint4 (&raw)[kRaw]) {
+    V v[8];
+    values(raw, v);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int64_t w0 = p0[k >> 1][k & 1], w1 = p1[k >> 1][k & 1];
       if constexpr (P::kWide) {
         // reduced each digit (values arrive settled): below 1.4q
-        facc0[k] = p.reduce(facc0[k]) + p.product(u64_to_f64(static_cast<uint64_t>(w0[k])), v[k]);
-        facc1[k] = p.reduce(facc1[k]) + p.product(u64_to_f64(static_cast<uint64_t>(w1[k])), v[k]);
+        facc0[k] = p.reduce(facc0[k]) + p.product(u64_to_f64(static_cast<uint64_t>(w0)), v[k]);
+        facc1[k] = p.reduce(facc1[k]) + p.product(u64_to_f64(static_cast<uint64_t>(w1)), v[k]);
       } else if constexpr (kF64) {
-        mac_f64(facc0[k], v[k], w0[k], row.qd, row.qinv);
-        mac_f64(facc1[k], v[k], w1[k], row.qd, row.qinv);
+        mac_f64(facc0[k], v[k], w0, row.qd, row.qinv);
+        mac_f64(facc1[k], v[k], w1, row.qd, row.qinv);
       } else {
-        wide_mac(wacc0[k], v[k], static_cast<uint64_t>(w0[k]));
-        wide_mac(wacc1[k], v[k], static_cast<uint64_t>(w1[k]));
+        wide_mac(wacc0[k], v[k], static_cast<uint64_t>(w0));
+        wide_mac(wacc1[k], v[k], static_cast<uint64_t>(w1));
       }
     }
   };
 #pragma nounroll
   for (int64_t di = 0; di < a.dnum; di += 2) {
-    if (di + 1 < a.dnum) load_digit(di + 1, wb0, wb1, vb);
-    mac_digit(wa0, wa1, va);
+    if (di + 1 < a.dnum) load_digit(di + 1, wb0, wb1, rb);
+    mac_digit(wa0, wa1, ra);
     if (di + 1 >= a.dnum) break;
-    if (di + 2 < a.dnum) load_digit(di + 2, wa0, wa1, va);
-    mac_digit(wb0, wb1, vb);
+    if (di + 2 < a.dnum) load_digit(di + 2, wa0, wa1, ra);
+    mac_digit(wb0, wb1, rb);
   }
   if constexpr (kF64) {
-    mac_finish<true, false, std::conditional_t<P::kWide, P, F64Fast>>(a, j, b, t, dst, sh, tww, twp, facc0, facc1);
+    mac_finish<true, false, std::conditional_t<P::kWide, P, F64Fast>>(a, j, b, t, r_dst, sh, tww, twp, facc0, facc1);
   } else {
     // at most 16 products y w with y < 4q, w < 2q: REDC value below 9q
 #pragma unroll
@@ -1628,14 +1623,19 @@ __device__ __forceinline__ void tiles_mac_hoisted(const P& p, const KsArgs& a, i
       uacc0[k] = wide_redc62(wacc0[k], row.q, row.neg_qinv64);
       uacc1[k] = wide_redc62(wacc1[k], row.q, row.neg_qinv64);
     }
-    mac_finish<true, false, P>(a, j, b, t, dst, sh, tww, twp, uacc0, uacc1);
+    mac_finish<true, false, P>(a, j, b, t, r_dst, sh, tww, twp, uacc0, uacc1);
   }
 }
 
-// Two waves per SIMD on both paths: with the next digit's loads in flight
-// the binary64 body needs 182 VGPRs; a three-wave budget spilled 44 bytes per
-// thread, and the scratch traffic cost more than the extra wave gained
-// (128-diagonal matrix-vector product 27.5 against 26.3 ms).
+// Bound by the key words from HBM.  A thread owns pairs of destination
+// elements, so the keys arrive in 16-byte words of whole lines, and the shared
+// digit values take the Galois map instead, through the exchange buffer (with
+// the keys read at mapped slots, eight 8-byte loads touched each line).
+// 31 rotations of 27 Q and 4 P rows at logN = 16, 7 digits (7.1 GB of keys),
+// both launches overlapped: 2140 -> 1800 us, 3.9 TB/s of keys.  Two waves per
+// SIMD with the next digit's loads in flight (212 VGPRs); one buffer refilled
+// as it is used, at three or four waves, is 0.5 to 1.5% slower, two buffers at
+// three waves spill 140 bytes per thread and lose 10%.
 template <int MODE, bool kSmall>
 __global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_ks_mac_hoisted(
     KsArgs a, int64_t groups, int64_t j_begin, int64_t j_count) {
@@ -2371,16 +2371,13 @@ __device__ __forceinline__ void xp_tiles(const P& p, const HoistNttArgs& a, int6
 #pragma unroll
     for (int k = 0; k < 8; ++k) x[k] = static_cast<uint64_t>(slab[j * n + r * kTile + 8 * t + k]);
   }
-  // sigma_g(c0) at those elements: out[i] = in[br(((2 br(i) + 1) g mod 2N - 1) / 2)]
+  // sigma_g(c0) at those elements
   int64_t c0[8] = {};
   if (ce < a.entries) {
     const uint32_t gal = static_cast<uint32_t>(a.galois[2 * ce]);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const uint32_t i = static_cast<uint32_t>(r * kTile + 8 * t + k);
-      const uint32_t e = ((2 * brev_bits(i, a.log_n) + 1) * gal) & ((2u << a.log_n) - 1);
-      c0[k] = a.c0[j * n + brev_bits((e - 1) >> 1, a.log_n)];
-    }
+    for (int k = 0; k < 8; ++k)
+      c0[k] = a.c0[j * n + hoisted_source(static_cast<uint32_t>(r * kTile + 8 * t + k), gal, a.log_n)];
   }
   {
     const int64_t* w_row = a.fwd_w + grow * n;
