@@ -7,7 +7,8 @@
 // (nine for a rotation) instead of ~100 (ModUp and the tile pass launch once
 // for the binary64 rows
 // and once for the integer rows; the integer rows' MAC runs on a side
-// stream, concurrently with the binary64 rows' launches):
+// stream, concurrently with the binary64 rows' launches; small calls take
+// both kinds of rows in one launch of each):
 //
 //   1. k_ks_decompose     Garner digits of every active hybrid digit (one
 //                         launch for all digits); optionally reads its input
