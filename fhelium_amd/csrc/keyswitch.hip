@@ -820,14 +820,10 @@ __device__ __forceinline__ int mac_tw_slot(int st, int e) { return (1 << st) - 1
 
 // NTT-domain Galois automorphism on tiles (hybrid_keyswitch.py:506-528):
 // out[k] = in[br(((2 br(k) + 1) g mod 2N - 1) / 2)].  With k = 256 r + i the
-// source of every element of destination tile r lies in one source tile r',
-// and inside the tile the map is affine in bit-reversed coordinates:
-// br8(src_i) = (g br8(i) + c_r) mod 256, c_r = ((2 br(r) + 1) g mod 2N) >> (L-7).
-// In the MAC's slot layout (thread t holds elements 8t..8t+7) the elements
-// of destination thread t all come from one source thread.  A hoisted MAC
-// block is source-stationary: it reads source tile r' and finds the
-// destination tile, and for its thread t the destination element of each
-// slot k.
+// source of every element of destination tile r lies in one source tile r'.
+// A hoisted MAC block takes source tile r', so that consecutive blocks (the
+// rotations of one tile) read the same digits, finds its destination tile, and
+// permutes the digit values inside the tile.
 __device__ __forceinline__ uint32_t brev_bits(uint32_t x, int bits) { return __brev(x) >> (32 - bits); }
 
 // Destination tile of source tile r_src under the NTT-domain map of g: the
