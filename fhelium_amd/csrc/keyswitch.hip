@@ -2758,11 +2758,12 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
                        dim3(static_cast<uint32_t>(64 * waves)), mac_split_lds_bytes(static_cast<int>(waves)), s, a);
     FH_CHECK_LAUNCH("key switch tile pass + MAC");
   } else if (!use_side_stream) {
-    for (int pass = 0; pass < 2; ++pass) {
-      int rc = launch_modup(pass, s);
-      if (rc == kOk) rc = launch_mac(pass, s);
-      if (rc != kOk) return rc;
-    }
+    // both ModUp passes before either tile pass: without rows below 2^42, tile
+    // pass 0 reads what ModUp pass 1 writes
+    int rc = kOk;
+    for (int pass = 0; pass < 2 && rc == kOk; ++pass) rc = launch_modup(pass, s);
+    for (int pass = 0; pass < 2 && rc == kOk; ++pass) rc = launch_mac(pass, s);
+    if (rc != kOk) return rc;
   } else {
     std::lock_guard<std::mutex> lock(g_side_mutex);
     SideStream* side = nullptr;

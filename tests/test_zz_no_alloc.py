@@ -2,7 +2,8 @@
 scratch, no allocation) against fh_keyswitch_fused (caller workspaces):
 bit-identical outputs on two calls in a row, the second smaller, for a
 relinearization with rescale and seeds, a per-entry-key rotation and a
-plain key switch; a call beyond the scratch size is rejected before any
+plain key switch, and over chains, arithmetic modes and call sizes that take
+each launch order; a call beyond the scratch size is rejected before any
 launch."""
 
 from __future__ import annotations
@@ -11,6 +12,8 @@ import numpy as np
 import pytest
 import torch
 
+from fhelium_amd.config import CkksConfig
+from fhelium_amd.csprng import Csprng
 from fhelium_amd.engine import CkksEngine
 from tests import helpers as H
 
@@ -72,6 +75,30 @@ def test_static_batch_at_high_level(eng14):
     got = ks.key_switch_fused(c.data[1], keys, level, base0=c.data[0], galois_elements=g, static_workspace=True)
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+# Chains with and without a prime below 2^42; calls above the small-call limit
+# of 2816 pairs of tiles (QP rows x 8 x batch at logN = 12), below it, and with
+# one digit.
+@pytest.mark.parametrize("mode", ["fast", "exact"])
+@pytest.mark.parametrize("preset,level,batch", [("slots32768-scale50-levels27-int64", 0, 1),
+                                                ("slots32768-scale50-levels27-int64", 26, 60),
+                                                ("slots16384-scale50-levels12-int64", 10, 72),
+                                                ("slots8192-scale50-levels5-int64", 4, 120),
+                                                ("slots32768-scale40-levels34-int64", 33, 60),
+                                                ("slots32768-scale30-levels45-int64", 44, 3)])
+def test_static_matches_allocating_over_chains_and_modes(preset, level, batch, mode):
+    eng = CkksEngine(CkksConfig.from_preset(preset).with_ring_log(12), ntt_mode=mode, rng_seed=41)
+    ks = eng.key_switcher
+    key = eng.generate_relinearization_key()
+    q = torch.tensor(eng.config.moduli[level: eng.config.num_q_primes], dtype=torch.int64, device=eng.device)
+    # two inputs in turn: nothing of the first call may reach the second
+    for x in Csprng(level, eng.device).uniform_mod(q, (2, batch), eng.config.N):
+        base = x.flip(0).contiguous()
+        for rescale in (False, True):
+            want = ks.key_switch_fused(x, key, level, base0=base, rescale=rescale)
+            got = ks.key_switch_fused(x, key, level, base0=base, rescale=rescale, static_workspace=True)
+            assert torch.equal(got, want)
 
 
 def test_static_rejects_oversize(eng14):
