@@ -2113,9 +2113,11 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
     return with_base(bval, mont_mul(sub_lazy(xr, xp, m.twice_q), a.p_inverse[grow], m), m.twice_q);
   };
   // Fused rescale: every thread needs the final row-0 value of its
-  // coefficient.  Row 0 is a binary64 row, or, when the scale primes are at
-  // or above 2^42, an integer row as every other row then is.
+  // coefficient.  Row 0 is a binary64 row, or, without rows below 2^42, may be
+  // an integer row beside binary64 ones (c0_in_f64 false: each row then takes
+  // c0_int modulo its own prime).
   const bool rescale = a.rescale_inv != nullptr;
+  bool c0_in_f64 = true;
   double c0 = 0.0;
   int64_t c0_int = 0;
   int64_t round_up = 0;
@@ -2125,6 +2127,7 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
       c0 = add_base_f64(moddown_f64(rec0, word_f64(x0)), bv0, rec0[14]);
       c0_int = static_cast<int64_t>(f64_to_u64(c0));
     } else {
+      c0_in_f64 = false;
       c0_int = moddown_integer(a.level, acc_row(0), has_base ? base.at(b, 0, i) : 0);
     }
     round_up = c0_int > a.half_drop ? 1 : 0;
@@ -2145,7 +2148,9 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
         r = f64_mulmod_signed(inv, v - c0, q, rec[15]);
       } else {
         // quotients up to 2^50: a rounding instruction, as F64Wide's product
-        const double x = v - c0, h = inv * x;
+        const double dropped =
+            c0_in_f64 ? c0 : u64_to_f64(static_cast<uint64_t>(canonical_operand(c0_int, a.rows[a.level + row].q, rec[15])));
+        const double x = v - dropped, h = inv * x;
         r = __builtin_fma(-__builtin_rint(h * rec[15]), q, h) + __builtin_fma(inv, x, -h);
       }
       r += static_cast<double>(round_up);

@@ -1,9 +1,9 @@
 """The fused key switch against the per-digit op sequence it replaces
 (hybrid_keyswitch.py:321-371), bit for bit, over every shipped parameter set
-on a small ring: digit widths 1 to 4 (a level that cuts into the leading
-digit narrows it), one to four P primes, 30-, 40- and 50-bit scale primes,
-and residues at both ends of their range, where the sums of products are
-largest."""
+and a longer chain on a small ring: digit widths 1 to 6 (a level that cuts
+into the leading digit narrows it), one to six P primes, 30-, 40- and 50-bit
+scale primes, and residues at both ends of their range, where the sums of
+products are largest."""
 
 from __future__ import annotations
 
@@ -19,9 +19,15 @@ from fhelium_amd.engine import CkksEngine
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module", params=[p.value for p in Preset])
+CHAINS = {p.value: CkksConfig.from_preset(p).with_ring_log(12) for p in Preset}
+# the last five scale primes lie above and below 2^50 + 2^30 in turn: integer
+# rows beside binary64 ones, an integer row the first to be dropped at level 71
+CHAINS["scale50-levels76-p6"] = CkksConfig(12, 50, 76, 6, 1 << 16)
+
+
+@pytest.fixture(scope="module", params=CHAINS)
 def eng(request):
-    return CkksEngine(CkksConfig.from_preset(request.param).with_ring_log(12), rng_seed=17)
+    return CkksEngine(CHAINS[request.param], rng_seed=17)
 
 
 def components(eng, level):
@@ -34,7 +40,7 @@ def components(eng, level):
     return torch.stack([uniform, top, mixed])
 
 
-@pytest.mark.parametrize("offset", [0, 1, 2, 3, -2])
+@pytest.mark.parametrize("offset", [0, 1, 2, 3, -2, -5])
 def test_key_switch_matches_per_digit_sequence(eng, offset):
     level = offset if offset >= 0 else eng.config.public_level_count + offset
     if not 0 <= level < eng.config.public_level_count - 1:
@@ -51,7 +57,7 @@ def test_key_switch_matches_per_digit_sequence(eng, offset):
     assert torch.equal(rescaled, eng.rescale_to_next_level(Ciphertext(want, level, 1.0)).data)
 
 
-@pytest.mark.parametrize("offset", [0, -2])
+@pytest.mark.parametrize("offset", [0, -2, -5])
 def test_product_and_hoisted_rotation_match_composition(eng, offset):
     level = offset if offset >= 0 else eng.config.public_level_count + offset
     eng.generate_relinearization_key()
