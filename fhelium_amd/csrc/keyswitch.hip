@@ -1233,8 +1233,10 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
   const int r_dst = r;
   if constexpr (kSplit) {
     // Wave c collects accumulator c of every wave (exchange buffers take the
-    // shares).  Binary64 shares add exactly (17 terms below 0.53q in all, or
-    // at most 8 shares reduced to 0.51q), integer shares are below 2q each, at most 8 of them.
+    // shares).  Binary64 shares add exactly (17 terms below 0.53q in all, or,
+    // for F64Wide, at most 8 shares within 0.51q: their sum is reduced once,
+    // into the inverse's operand range), integer shares are below 2q each, at
+    // most 8 of them.
     auto collect = [&](auto (&acc)[8], int owner) {
       __syncthreads();
 #pragma unroll
@@ -1251,7 +1253,10 @@ __device__ __forceinline__ void tiles_mac(const P& p, const KsArgs& a, int64_t g
             acc[k] += x;
           }
         }
-        if constexpr (!kF64) {
+        if constexpr (P::kWide) {
+#pragma unroll
+          for (int k = 0; k < 8; ++k) acc[k] = p.reduce(acc[k]);
+        } else if constexpr (!kF64) {
 #pragma unroll
           for (int k = 0; k < 8; ++k) acc[k] = csub(csub(csub(acc[k], 8 * row.q), 4 * row.q), 2 * row.q);
         }
@@ -2076,9 +2081,10 @@ __global__ __launch_bounds__(kBlock) void k_ks_moddown_add(ModDownArgs a) {
   // 2P + 1 products (x P^{-1}, and the digit halves of X_P times their
   // negated constants), reduced once.  x and the constants are below q, the
   // halves below 2^30, so the sum is below q (q + 2P 2^30) and its reduced
-  // value within 0.52q (F64Wide primes: within 5.3q, reduced once more).  The
-  // result of a binary64 row stays in binary64 (exact integers) through the
-  // base addition and the fused rescale.
+  // value within 0.52q (F64Wide primes: within (P + 1.3) q, below 2^53 for the
+  // at most six P primes, and reduced once more).  The result of a binary64
+  // row stays in binary64 (exact integers) through the base addition and the
+  // fused rescale.
   auto moddown_f64 = [&](Global<double>* rec, double x) -> double {
     const double q = rec[14], qinv = rec[15];
     const double start = f64_sum_start(q * (q + 2.0 * P * 0x1.0p30));

@@ -188,9 +188,11 @@ struct F64Fast {
 // is rounded by an instruction instead of the 2^52 magic constant, its
 // estimate is off by up to 3/8 per q of the operand, and sums need more
 // reductions than F64Fast's; every value stays an exact integer below 2^53.
-// In units of q: a product of an operand x is below 0.5 + 0.375 x; forward
-// sums reduced at even stages stay below 3.9, inverse sums reduced at every
-// stage leave products below 1.1.  Against the integer path (at least 10
+// In units of q: a product of an operand x is below 0.5 + 0.375 x.  Forward
+// sums, reduced at even stages, stay below 3.9 from inputs below that, and
+// below 5.6 from ModUp's extended digits (0.9 for each of at most 8 rows).
+// Inverse sums are reduced at every stage; from operands within 2, differences
+// stay within 4 and products within 2.  Against the integer path (at least 10
 // 32-bit multiplies per product) a butterfly is 9.5 or 11 binary64
 // operations: the 24 50-bit rows of a 3-entry key switch at logN = 16 take 174
 // us in the tile pass and MAC and 190 us in ModUp, where with the integer path
@@ -370,8 +372,8 @@ struct U64Fast {
 // On the five 60-bit rows of a 16-entry key switch at 33 Q rows (logN = 16):
 // tile pass and MAC 329 -> 282 us, ModUp (whose digit products sum exactly
 // before one fold) 339 -> 297 us, both bound by the multiply rate.
-// In units of 2^60: products are below 2.3, forward values below 13.1 (1.1
-// after a fold, a stage adds at most 3), inverse values below 2.3 (sums
+// In units of 2^60: products are below 2.32, forward values below 13.1 (1.1
+// after a fold, a stage adds at most 3), inverse values below 2.32 (sums
 // folded each stage).
 struct U64Pm {
   static constexpr bool kCompanion = false;
@@ -396,7 +398,7 @@ struct U64Pm {
   __device__ __forceinline__ V in(int64_t raw) const { return static_cast<uint64_t>(raw); }
   __device__ __forceinline__ int64_t mid(V v) const { return static_cast<int64_t>(v); }
   __device__ __forceinline__ V unmid(int64_t b) const { return static_cast<uint64_t>(b); }
-  // h 2^60 + l (l < 2^60) -> a word below 2.3 2^60 of the same residue: with
+  // h 2^60 + l (l < 2^60) -> a word below 2.32 2^60 of the same residue: with
   // g = (h >> 32) delta, h 2^60 = (h mod 2^32) delta + g 2^32, and
   // g 2^32 = (g mod 2^28) 2^32 + (g >> 28) delta.
   __device__ __forceinline__ V fold(uint64_t h, uint64_t l) const {
@@ -422,7 +424,7 @@ struct U64Pm {
     return static_cast<uint64_t>(static_cast<uint32_t>(v >> 60)) * delta + (v & 0x0fffffffffffffffull);
   }
   __device__ __forceinline__ V canon(V v) const { return csub(settle(v), q); }
-  // an exact sum of products below 2^124 -> below 2.3 2^60
+  // an exact sum of products below 2^124 -> below 2.32 2^60
   __device__ __forceinline__ V reduce(const WideAcc& s) const {
     return fold(s.c2 << 4 | s.c1 >> 28, static_cast<uint64_t>(s.c1 & 0xfffffffu) << 32 | s.c0);
   }

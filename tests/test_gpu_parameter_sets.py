@@ -129,3 +129,27 @@ def test_small_calls_match_large_ones(preset, batch):
         one_b = Ciphertext(data[2:, e: e + 1].contiguous(), 0, a.scale)
         assert torch.equal(eng.hmult(one_a, one_b).data[:, 0], product[:, e])
         assert torch.equal(eng.rotate_by_steps(one_a, [steps[e]]).data[:, 0], rotated[:, e])
+
+
+def test_small_call_sums_extreme_shares():
+    """Eight digits dealt to eight waves, on a prime above 2^50: key words that
+    bring every wave's share of one accumulator near (q - 1) / 2 and of its
+    neighbour near -(q - 1) / 2, whose difference no binary64 integer holds."""
+
+    eng = CkksEngine(CkksConfig(12, 50, 7, 1, 1 << 16), rng_seed=3)
+    cfg, row = eng.config, 1
+    q = cfg.moduli[row]
+    assert q > 1 << 50 and len(eng.layout.digit_specs(0)) == 8
+    # every digit is the constant 1: its transform is R mod q everywhere
+    x = torch.zeros((1, cfg.num_q_primes, cfg.N), dtype=torch.int64, device=eng.device)
+    x[..., 0] = 1
+    key = eng.generate_relinearization_key()
+    key.data.zero_()
+    r_inverse = pow(1 << 62, -1, q)
+    half = (q - 1) // 2 - 1000
+    for digit in range(8):
+        key.data[digit, :, row, 0::2] = (half - (digit == 0)) * r_inverse % q
+        key.data[digit, :, row, 1::2] = -half * r_inverse % q
+    assert 2 * 8 * half - 1 > 1 << 53
+    want = torch.stack(eng.key_switcher.apply_key_switch(x, key, 0))
+    assert torch.equal(eng.key_switcher.key_switch_fused(x, key, 0), want)
