@@ -1345,10 +1345,16 @@ class CkksEngine:
                            ct_ntt: Ciphertext | None = None) -> Ciphertext:
         """coefficient_domain_to_ntt_domain(rotate_hoisted(ct, steps)).  Where
         the chain allows it the rotations stay in the NTT domain after the key
-        products and meet ``ct_ntt`` (ct in the NTT domain, transformed here
-        if not given) there."""
+        products and meet ``ct_ntt`` (ct in the NTT domain, of its level,
+        layout and scale; transformed here if not given) there."""
 
         self._assert_rotation_ciphertext(ct)
+        if ct_ntt is not None:
+            ct_ntt.assert_state(polynomial_domain="ntt", residue_representation="montgomery", components=2)
+            self._same_layout(ct, ct_ntt)
+            if ct_ntt.scale != ct.scale:
+                raise ScaleMismatchError(f"rotate_hoisted_ntt: ciphertext scale {ct.scale} != transform's scale "
+                                         f"{ct_ntt.scale}")
         steps = [RotationKey.canonical_step(s, self.config.N) for s in rotation_steps]
         if (ct.batch_shape not in ((), (1,)) or not self.fused_keyswitch or not steps or 0 in steps
                 or not self.key_switcher.hoisted_ntt_ready(ct.level)):

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from fhelium_amd.config import CkksConfig, Preset
-from fhelium_amd.core import Ciphertext
+from fhelium_amd.core import Ciphertext, CkksStateError, ScaleMismatchError
 from fhelium_amd.csprng import Csprng
 from fhelium_amd.engine import CkksEngine
 
@@ -54,3 +54,20 @@ def test_general_path_keeps_every_step_and_error():
     batched = eng.encrypt([[0.5], [0.25]], level=1)
     with pytest.raises(ValueError, match="unbatched"):
         eng.rotate_hoisted_ntt(batched, [1])
+
+
+@pytest.mark.parametrize("preset", ["slots8192-scale40-levels7-int64", "slots8192-scale50-levels5-int64"])
+def test_given_transform_must_be_the_ciphertexts(preset):
+    """On the NTT-domain path and on the general one."""
+
+    eng = CkksEngine(CkksConfig.from_preset(preset).with_ring_log(12), rng_seed=25)
+    ct = eng.encrypt([0.5, -0.25], level=1)
+    ntt = eng.coefficient_domain_to_ntt_domain(ct)
+    with pytest.raises(CkksStateError, match="ntt-domain"):
+        eng.rotate_hoisted_ntt(ct, [1, 2], ct)
+    with pytest.raises(ScaleMismatchError):
+        eng.rotate_hoisted_ntt(ct, [1, 2], Ciphertext(ntt.data, 1, 2 * ct.scale, "ntt", "montgomery"))
+    with pytest.raises(ValueError, match="level"):
+        eng.rotate_hoisted_ntt(ct, [1, 2], Ciphertext(ntt.data, 2, ct.scale, "ntt", "montgomery"))
+    with pytest.raises(ValueError, match="shape"):
+        eng.rotate_hoisted_ntt(ct, [1, 2], Ciphertext(ntt.data[:, 1:], 1, ct.scale, "ntt", "montgomery"))
