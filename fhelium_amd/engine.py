@@ -329,7 +329,7 @@ class CkksEngine:
             raise ValueError(f"at most {cfg.slots} slots per plaintext")
         batch_shape = tuple(v.shape[:-1])
         if v.size(-1) == cfg.slots and v.dtype == torch.complex128 and v.numel():
-            flat = v.reshape(-1, cfg.slots).resolve_conj().contiguous()
+            flat = v.reshape(-1, cfg.slots).resolve_conj().resolve_neg().contiguous()
         else:
             flat = torch.zeros((int(np.prod(batch_shape)) if batch_shape else 1, cfg.slots), dtype=torch.complex128,
                                device=self.device)

@@ -60,6 +60,10 @@ def test_encode_equals_the_stage_encoder(eng, scale_bits, batch):
     padded[:, : short.size(1)] = short
     assert torch.equal(eng.encode_on_device(short, level=level, scale=scale).data,
                        eng.encode_on_device(padded, level=level, scale=scale).data)
+    # conjugate and negative views are read as the values they stand for
+    for lazy, plain in ((z.conj(), z.conj_physical()), (torch._neg_view(z), -z)):
+        assert torch.equal(eng.encode_on_device(lazy, level=level, scale=scale).data,
+                           eng.encode_on_device(plain, level=level, scale=scale).data)
 
 
 @pytest.mark.parametrize("batch", [1, 5])
