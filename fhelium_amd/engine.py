@@ -396,10 +396,15 @@ class CkksEngine:
             if rows.stride(-1) != 1:
                 rows = rows.contiguous()
             nat.require_device(rows, sk.data)
-            if rows.dtype != torch.int64 or rows.device != sk.data.device:
+            if rows.dtype != torch.int64 or sk.data.dtype != torch.int64 or rows.device != sk.data.device:
                 raise TypeError("decryption needs int64 residues on the secret key's device")
             c0, c1 = rows[0].reshape(b, 2, cfg.N), rows[1].reshape(b, 2, cfg.N)
             s = sk.data[start: start + 2]
+            if tuple(s.shape) != (2, cfg.N):
+                raise RuntimeError(f"decryption needs a secret key of [QP, {cfg.N}] rows, got "
+                                   f"{tuple(sk.data.shape)}")
+            if s.stride(-1) != 1:
+                s = s.contiguous()
             product = torch.empty((b, 2, cfg.N), dtype=torch.int64, device=self.device)
             nt = self.runtime.ntt_tables
             twiddles, slot_map = self._codec_tables()

@@ -14,7 +14,7 @@ from fhelium_amd import _native as nat
 from fhelium_amd import codec
 from fhelium_amd import kernels as K
 from fhelium_amd.config import CkksConfig
-from fhelium_amd.core import Ciphertext
+from fhelium_amd.core import Ciphertext, SecretKey
 from fhelium_amd.engine import CkksEngine
 
 pytestmark = pytest.mark.gpu
@@ -103,3 +103,24 @@ def test_decode_of_extreme_residues(eng):
     centred = np.array([float(v - qa * qb if v > qa * qb // 2 else v) for v in x])
     want = codec.embed(centred)
     assert np.abs(got - want).max() < 1e-12 * np.abs(want).max()
+
+
+def test_decrypt_with_other_secret_keys(eng):
+    """A strided secret key decrypts; one of another ring, row count or type is refused."""
+
+    ct = eng.encrypt(slots(eng, 2, 9), level=1)
+    want = eng.decrypt_on_device(ct)
+    secret = eng.secret_key
+    data = torch.empty((*secret.data.shape[:-1], 2 * eng.config.N), dtype=torch.int64, device=eng.device)[..., ::2]
+    data.copy_(secret.data)
+    rows = eng.config.num_q_primes
+    try:
+        eng.secret_key = SecretKey(data, secret.coefficients)
+        assert torch.equal(eng.decrypt_on_device(ct), want)
+        for bad in (secret.data[:, ::2].contiguous(), secret.data[: rows - 1].contiguous(), secret.data[1:, :1],
+                    secret.data.to(torch.int32)):
+            eng.secret_key = SecretKey(bad, secret.coefficients)
+            with pytest.raises((RuntimeError, TypeError)):
+                eng.decrypt_on_device(ct)
+    finally:
+        eng.secret_key = secret
