@@ -105,8 +105,9 @@ def test_seeded_keyswitch_matches_bases(eng, level, rescale):
                                           ("slots16384-scale50-levels12-int64", 3),
                                           ("slots32768-scale50-levels27-int64", 25)])
 def test_fused_rescale_by_a_50_bit_prime(preset, level):
-    """The dropped prime of a 50-bit parameter set is no binary64 row: the
-    fused product still equals the method composition."""
+    """The dropped prime of a 50-bit parameter set is a binary64 row above
+    2^42 (8-byte words, its own launches): the fused product still equals the
+    method composition."""
 
     e = CkksEngine(CkksConfig.from_preset(preset).with_ring_log(12), rng_seed=7)
     rng = np.random.default_rng(level)

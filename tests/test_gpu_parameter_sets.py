@@ -1,9 +1,9 @@
 """The fused key switch against the per-digit op sequence it replaces
 (hybrid_keyswitch.py:321-371), bit for bit, over every shipped parameter set
-and a longer chain on a small ring: digit widths 1 to 6 (a level that cuts
-into the leading digit narrows it), one to six P primes, 30-, 40- and 50-bit
-scale primes, and residues at both ends of their range, where the sums of
-products are largest."""
+and a longer chain on a small ring, in both arithmetic modes: digit widths 1
+to 6 (a level that cuts into the leading digit narrows it), one to six P
+primes, 30-, 40- and 50-bit scale primes, and residues at both ends of their
+range, where the sums of products are largest."""
 
 from __future__ import annotations
 
@@ -25,9 +25,10 @@ CHAINS = {p.value: CkksConfig.from_preset(p).with_ring_log(12) for p in Preset}
 CHAINS["scale50-levels76-p6"] = CkksConfig(12, 50, 76, 6, 1 << 16)
 
 
-@pytest.fixture(scope="module", params=CHAINS)
+@pytest.fixture(scope="module", params=[(c, m) for c in CHAINS for m in ("fast", "exact")], ids="-".join)
 def eng(request):
-    return CkksEngine(CHAINS[request.param], rng_seed=17)
+    chain, mode = request.param
+    return CkksEngine(CHAINS[chain], ntt_mode=mode, rng_seed=17)
 
 
 def components(eng, level):
