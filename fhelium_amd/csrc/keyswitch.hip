@@ -106,7 +106,7 @@ struct KsArgs {
   const int64_t* gal_idx;   // per-entry int32 gather table addresses [B] or null
   const int64_t* gal_sign;  // per-entry int8 sign table addresses [B]
   int64_t small_rows;       // leading QP rows on the binary64 path (primes below 2^42)
-  int wide_apart;           // F64Wide rows have tile-pass launches of their own (no row below 2^42)
+  int wide_apart;           // F64Wide rows have tile-pass launches of their own (wide_rows_apart)
   // Optional accumulator seeds (null: none): [B, Lq, N] NTT-domain rows in
   // the accumulators' scaling, added to the Q rows times seed_scale[row].
   const int64_t* seed0;
@@ -1288,9 +1288,8 @@ constexpr int kMacTilesPerBlock = kMacTiles;
 // Register budgets: 3 waves per SIMD for the binary64 rows (no spills at 156
 // VGPRs), 2+ for the integer rows.
 // kRowsKind: which rows a tile-pass launch serves.  Rows of F64Wide primes run
-// in the integer rows' launch where a chain has them beside narrower ones, and
-// in a launch of their own (blocks of other rows end at once) where no row is
-// below 2^42.
+// in the integer rows' launch or, with wide_apart, in one of their own over
+// every row (blocks of other rows end at once).
 enum RowsKind : int { kRowsSmall = 0, kRowsInteger = 1, kRowsWide = 2 };
 template <int MODE, int kRowsKind>
 __global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(kRowsKind == kRowsInteger ? 2 : 3))) void k_ks_tiles_mac(KsArgs a, int64_t groups, int64_t j_begin,
@@ -1682,7 +1681,7 @@ struct HmArgs {
   int64_t* out;       // [3, B, L, N] working-format rows for the inverse column pass
   int64_t batch, limbs, row_start;
   int log_n;
-  int wide_apart;     // as in KsArgs
+  int wide_apart;     // as in KsArgs, by this launch's own size
   ParamView params;   // global QP rows
   const NttRow* rows; // global QP NTT records
   const int64_t* fwd_w;
@@ -2496,6 +2495,18 @@ __global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(4))) 
 // does both of its tiles' digits there and the integer rows' register count
 // halves the binary64 rows' occupancy).
 constexpr int64_t kSmallCallPairs = 2816;
+// F64Wide rows take tile-pass launches of their own, the integer rows' launch
+// running beside theirs on the side stream, in chains without rows below 2^42
+// and above the same size.  Otherwise they share the integer rows' launch: for
+// few tiles a second launch, its fork and its join cost more than they give.
+// One rotation in exact arithmetic, apart against together: 112 / 62 us at 224
+// pairs (logN = 14), 118 / 101 at 960 (logN = 15), 159 / 141 at 2432 (logN =
+// 16); at 4096 pairs 297 us apart, 310 with both launches on one stream.  The
+// product's tile pass follows the same line by its own rows: 198 / 184 us for
+// a whole product of three entries at level 24 (logN = 16, 1536 pairs).
+inline bool wide_rows_apart(int64_t small_rows, int64_t tile_pairs) {
+  return small_rows == 0 && tile_pairs > kSmallCallPairs;
+}
 // Waves of the split tile pass: two per SIMD (it holds two; four or eight per
 // SIMD measured the same or slower).
 constexpr int64_t kSplitTargetWaves = 2048;
@@ -2637,7 +2648,8 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
   a.gal_idx = galois_index_tables;
   a.gal_sign = galois_sign_tables;
   a.small_rows = small_rows;
-  a.wide_apart = small_rows == 0 ? 1 : 0;
+  const int64_t tile_pairs = lqp * (n / (2 * kTile)) * batch;
+  a.wide_apart = wide_rows_apart(small_rows, tile_pairs) && hoist_galois == nullptr ? 1 : 0;
   a.seed0 = seed0;
   a.seed1 = seed1;
   a.seed_scale = seed_scale;
@@ -2700,9 +2712,9 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
     FH_CHECK_LAUNCH("key switch modup + column pass");
     return kOk;
   };
-  // pass 0 of a chain without rows below 2^42: its F64Wide rows, wherever they are.
+  // pass 0 with wide_apart: the F64Wide rows, wherever they are.
   auto launch_mac = [&](int pass, hipStream_t st) -> int {
-    const bool wide = pass == 0 && a.wide_apart && !hoist;
+    const bool wide = pass == 0 && a.wide_apart;
     const int64_t j_begin = pass == 0 ? 0 : small_rows;
     const int64_t j_count = pass == 0 ? (wide ? lqp : small_rows) : lqp - small_rows;
     if (j_count == 0) return kOk;
@@ -2744,7 +2756,6 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
   };
   // Few tiles: the digits are dealt over several waves and both arithmetic
   // paths share their launches (no side stream, two launches fewer).
-  const int64_t tile_pairs = lqp * (n / (2 * kTile)) * batch;
   const bool small_call = mode == 1 && !hoist && digit_count >= 2 && tile_pairs <= kSmallCallPairs;
   if (small_call) {
     const int64_t modup_blocks = (kTile / C) * lqp * digit_count * batch;
@@ -2769,8 +2780,8 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
                        dim3(static_cast<uint32_t>(64 * waves)), mac_split_lds_bytes(static_cast<int>(waves)), s, a);
     FH_CHECK_LAUNCH("key switch tile pass + MAC");
   } else if (!use_side_stream) {
-    // both ModUp passes before either tile pass: without rows below 2^42, tile
-    // pass 0 reads what ModUp pass 1 writes
+    // both ModUp passes before either tile pass: with wide_apart, tile pass 0
+    // reads what ModUp pass 1 writes
     int rc = kOk;
     for (int pass = 0; pass < 2 && rc == kOk; ++pass) rc = launch_modup(pass, s);
     for (int pass = 0; pass < 2 && rc == kOk; ++pass) rc = launch_mac(pass, s);
@@ -2780,7 +2791,7 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
     SideStream* side = nullptr;
     int rc = side_stream(&side);
     if (rc != kOk) return rc;
-    const bool split = small_rows < lqp && (small_rows > 0 || (a.wide_apart && !hoist));
+    const bool split = small_rows < lqp && (small_rows > 0 || a.wide_apart);
     if (split) {
       rc = launch_modup(1, s);
       if (rc != kOk) return rc;
@@ -3115,7 +3126,7 @@ FH_API int fh_ckks_hmult_tensor_coefficient(const int64_t* a, const int64_t* b, 
   h.log_n = static_cast<int>(log_n);
   h.params = ParamView{rns_params.data, rns_params.stride_row, rns_params.stride_col};
   h.rows = rows;
-  h.wide_apart = small_rows == 0 ? 1 : 0;
+  h.wide_apart = wide_rows_apart(small_rows, limbs * (n / (2 * kTile)) * batch) ? 1 : 0;
   h.fwd_w = forward_twiddles;
   h.fwd_wp = forward_twiddles_shoup;
   h.inv_w = inverse_twiddles;
