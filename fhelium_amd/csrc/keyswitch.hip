@@ -2495,6 +2495,13 @@ __global__ __launch_bounds__(kMacBlock) __attribute__((amdgpu_waves_per_eu(4))) 
 // does both of its tiles' digits there and the integer rows' register count
 // halves the binary64 rows' occupancy).
 constexpr int64_t kSmallCallPairs = 2816;
+// Without rows below 2^42 the other path is one ModUp and one tile pass on one
+// stream at these sizes, and two or three digits give the waves little to
+// share.  Key switches of 50-bit chains on the device, split against together,
+// two digits: 51 / 56 us at 960 pairs, 63 / 66 at 1344, 70 / 68 at 1632, 75 / 70
+// at 1920, 95 / 92 at 2784; three digits: 62 / 65 at 1280, 72 / 71 at 1536, 78 /
+// 74 at 1920; four digits: 83 / 78 at 1920, but 92 / 94 at 2240.
+constexpr int64_t kSmallCallPairsFewDigits = 1500;
 // F64Wide rows take tile-pass launches of their own, the integer rows' launch
 // running beside theirs on the side stream, in chains without rows below 2^42
 // and above the same size.  Otherwise they share the integer rows' launch: for
@@ -2756,7 +2763,9 @@ int keyswitch_fused_impl(fh_view3 component, int64_t batch, int64_t lq, int64_t 
   };
   // Few tiles: the digits are dealt over several waves and both arithmetic
   // paths share their launches (no side stream, two launches fewer).
-  const bool small_call = mode == 1 && !hoist && digit_count >= 2 && tile_pairs <= kSmallCallPairs;
+  const bool few_digits = small_rows == 0 && digit_count <= 3;
+  const bool small_call = mode == 1 && !hoist && digit_count >= 2 &&
+                          tile_pairs <= (few_digits ? kSmallCallPairsFewDigits : kSmallCallPairs);
   if (small_call) {
     const int64_t modup_blocks = (kTile / C) * lqp * digit_count * batch;
 #define FH_MODUP_SMALL_CASE(S) \

@@ -107,27 +107,29 @@ def test_fast_transforms_match_exact_on_extreme_residues(log_n, chain):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("preset,batch", [("slots32768-scale40-levels34-int64", 10),
-                                          ("slots32768-scale50-levels27-int64", 12),
-                                          ("slots8192-scale30-levels9-int64", 36)])
-def test_small_calls_match_large_ones(preset, batch):
+@pytest.mark.parametrize("preset,level,batch,limit", [("slots32768-scale40-levels34-int64", 0, 10, 2816),
+                                                      ("slots32768-scale50-levels27-int64", 0, 12, 2816),
+                                                      ("slots8192-scale30-levels9-int64", 0, 36, 2816),
+                                                      # three digits of 50-bit rows, all rows in one tile pass
+                                                      ("slots8192-scale50-levels5-int64", 3, 48, 1500)])
+def test_small_calls_match_large_ones(preset, level, batch, limit):
     """A batch large enough for the launch per arithmetic path, entry by
     entry against single-entry calls, whose digits are dealt over the waves
     of a block (shared and per-entry keys, bases, seeds, fused rescale)."""
 
     eng = CkksEngine(CkksConfig.from_preset(preset).with_ring_log(12), rng_seed=23)
     eng.generate_relinearization_key()
-    rows = eng.config.total_num_primes
-    assert rows * 8 * batch > 2816 >= rows * 8
-    q = torch.tensor(eng.config.moduli[: eng.config.num_q_primes], dtype=torch.int64, device=eng.device)
+    rows = eng.config.total_num_primes - level
+    assert rows * 8 * batch > limit >= rows * 8
+    q = torch.tensor(eng.config.moduli[level: eng.config.num_q_primes], dtype=torch.int64, device=eng.device)
     data = Csprng(5, eng.device).uniform_mod(q, (4, batch), eng.config.N)
-    a = Ciphertext(data[:2].contiguous(), 0, eng.config.default_scale)
-    b = Ciphertext(data[2:].contiguous(), 0, eng.config.default_scale)
+    a = Ciphertext(data[:2].contiguous(), level, eng.config.default_scale)
+    b = Ciphertext(data[2:].contiguous(), level, eng.config.default_scale)
     steps = [1 + e % 3 for e in range(batch)]
     product, rotated = eng.hmult(a, b).data, eng.rotate_by_steps(a, steps).data
     for e in (0, 1, batch - 1):
-        one_a = Ciphertext(data[:2, e: e + 1].contiguous(), 0, a.scale)
-        one_b = Ciphertext(data[2:, e: e + 1].contiguous(), 0, a.scale)
+        one_a = Ciphertext(data[:2, e: e + 1].contiguous(), level, a.scale)
+        one_b = Ciphertext(data[2:, e: e + 1].contiguous(), level, a.scale)
         assert torch.equal(eng.hmult(one_a, one_b).data[:, 0], product[:, e])
         assert torch.equal(eng.rotate_by_steps(one_a, [steps[e]]).data[:, 0], rotated[:, e])
 
