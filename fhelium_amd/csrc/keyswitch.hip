@@ -111,7 +111,7 @@ struct KsArgs {
   // the accumulators' scaling, added to the Q rows times seed_scale[row].
   const int64_t* seed0;
   const int64_t* seed1;
-  const int64_t* seed_scale;  // [Q0] P mod q (binary64 rows), P R mod q (integer rows)
+  const int64_t* seed_scale;  // [Q0] P mod q (binary64 rows, F64Wide's among them), P R mod q (integer rows)
   // Hoisted rotations (null otherwise): [B, 2] (g, g^{-1} mod 2N) per entry.
   // The decompose and ModUp launches then see one input entry, and every MAC
   // entry reads that entry's intermediate through the NTT-domain Galois map
@@ -612,7 +612,11 @@ __device__ __forceinline__ void modup_columns_x2(const KsArgs& a, const KsDigit&
       // Digits of 3 and 4 rows: one reduction per sum (F64Sum).  Digits are
       // below 2^45, so the sum is below 2^47 q; its reduced value stays
       // within q (0.54 + rows^2 / 64) < 0.8q.  Four coefficients at a time
-      // keep both parts of the sums in registers.
+      // keep both parts of the sums in registers.  4 operations a product in
+      // place of 7, but this kernel waits on loads, LDS and stores as much as
+      // on arithmetic: whole calls gain 0.4 to 0.7% (logN = 16, against a
+      // reduction per product: one product 471 / 473 us, rotations by 7 keys
+      // 1590 / 1601, 16 products 4363 / 4392), nothing where few digits run.
       constexpr int kGroup = 4;
       const double start0 = f64_sum_start(0x1.0p45 * kRows * q0), start1 = f64_sum_start(0x1.0p45 * kRows * q1);
 #pragma unroll
@@ -692,7 +696,12 @@ __device__ __forceinline__ void modup_integer_block(const KsArgs& a, const NttRo
   }
 }
 
-// One launch per arithmetic path, as for the tile pass below.
+// One launch per arithmetic path, as for the tile pass below.  Four waves per
+// SIMD (128 VGPRs): the fast binary64 rows spill one register there, the
+// integer rows' kernel, which holds the bodies of three kinds of primes, 23 to
+// 40 (60 to 88 bytes per thread).  That kernel still takes 301 us for the five
+// 60-bit rows of a 16-entry product at logN = 16, where U64Fast alone took 339
+// us at three waves without a spill.
 template <int S1, int MODE, bool kSmall>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSmall && MODE == 0 ? 2 : 4))) void k_ks_modup_columns(KsArgs a, int64_t j_begin, int64_t j_count) {
   // (+1 column of padding: the packed store's transpose pitch)
@@ -740,7 +749,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSmall &
 }
 
 // Calls too small to fill the GPU (small_call): both arithmetic paths in one
-// launch, one destination row per block, the longer integer rows first.
+// launch, one destination row per block, the longer integer rows first.  Its
+// integer bodies spill as those of k_ks_modup_columns do: 11 us of a 55 us
+// rotation at logN = 14, 43 us of 283 busy ones in a product chain at logN = 16.
 template <int S1>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_ks_modup_small(KsArgs a) {
   __shared__ int64_t lds[(1 << S1) * (kBlock / ((1 << S1) / 16) + 1)];
@@ -1285,8 +1296,10 @@ constexpr int kMacTilesPerBlock = kMacTiles;
 
 // One launch per arithmetic path (binary64 rows, then the integer rows) so
 // each kernel is register-allocated for its own path only.
-// Register budgets: 3 waves per SIMD for the binary64 rows (no spills at 156
-// VGPRs), 2+ for the integer rows.
+// Register budgets: 3 waves per SIMD (168 VGPRs) for the binary64 rows, which
+// fits the fast path below 2^42; F64Wide's body spills 5 registers there (24
+// bytes per thread) and exact arithmetic's 11 (48 bytes).  2 waves for the
+// integer rows.
 // kRowsKind: which rows a tile-pass launch serves.  Rows of F64Wide primes run
 // in the integer rows' launch or, with wide_apart, in one of their own over
 // every row (blocks of other rows end at once).

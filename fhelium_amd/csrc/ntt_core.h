@@ -195,8 +195,8 @@ struct F64Fast {
 // stay within 4 and products within 2.  Against the integer path (at least 10
 // 32-bit multiplies per product) a butterfly is 9.5 or 11 binary64
 // operations: the 24 50-bit rows of a 3-entry key switch at logN = 16 take 174
-// us in the tile pass and MAC and 190 us in ModUp, where with the integer path
-// the 29 rows took 313 and 264 us.
+// us in the tile pass and MAC, and ModUp of all its 29 rows 177 to 192 us, where
+// with the integer path the 29 rows took 313 and 264 us.
 struct F64Wide {
   static constexpr bool kCompanion = false;
   static constexpr bool kWide = true;
@@ -371,7 +371,7 @@ struct U64Fast {
 // forward sums are folded once in four stages instead of once per butterfly.
 // On the five 60-bit rows of a 16-entry key switch at 33 Q rows (logN = 16):
 // tile pass and MAC 329 -> 282 us, ModUp (whose digit products sum exactly
-// before one fold) 339 -> 297 us, both bound by the multiply rate.
+// before one fold) 339 -> 301 us.
 // In units of 2^60: products are below 2.32, forward values below 13.1 (1.1
 // after a fold, a stage adds at most 3), inverse values below 2.32 (sums
 // folded each stage).

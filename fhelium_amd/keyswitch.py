@@ -45,9 +45,9 @@ class AccumulatorSeeds:
     """d0, d1 of an HMult front left in the NTT domain for the key switch.
 
     ``data`` is [2, *batch, Q_level, N] int64 words in a private working
-    format, not residues: rows whose prime is below 2^42 hold the binary64
-    bit patterns of a b R^2 (signed, not reduced), the other rows a b R below
-    2q; within each 256-coefficient tile, coefficient 8t + k sits at position
+    format, not residues: rows whose prime is below 2^50 + 2^30 hold the
+    binary64 bit patterns of a b R^2 (signed, not reduced), the other rows
+    a b R below 2q; within each 256-coefficient tile, coefficient 8t + k sits at position
     t + 32k.  Only ``HybridKeySwitcher.key_switch_fused(seeds=...)`` reads
     it."""
 

@@ -219,14 +219,16 @@ int fh_ckks_keyswitch_accumulate_multi_key(fh_view3 acc0, fh_view3 acc1, fh_view
 /* A whole hybrid key switch of a batched component in eight launches
  * (decompose, ModUp fused into the forward NTT column pass, tile pass fused
  * with the key MAC over every digit, inverse NTT, ModDown fused with the
- * engine's final canonical addition; a rotation adds one gather of base0).  Replaces the per-digit loop of
+ * engine's final canonical addition; a rotation adds one gather of base0; a
+ * call of few tiles takes two launches fewer).  Replaces the per-digit loop of
  * fhelium/engine/hybrid_keyswitch.py:321-371 plus :530-568 and
  * ckks_engine.py:1664-1667 / :3342, bit for bit; with Galois tables it also
  * replaces the coefficient automorphism of a rotation (ckks_engine.py:3822-3897).
  * The integer rows' MAC runs on a library-owned side stream (one per device)
  * forked from `stream` by an event and joined back to it before the inverse
  * transform, so the call is ordered like launches on `stream` alone (and is
- * captured with it).
+ * captured with it).  Calls of few tiles use no side stream in fast
+ * arithmetic, or when no row is below 2^42.
  *   component        [batch, lq, N] canonical standard Q rows at `level`
  *   small_rows       number of leading QP rows at `level` whose prime is
  *                    below 2^42 (binary64 arithmetic, 6-byte intermediates;
