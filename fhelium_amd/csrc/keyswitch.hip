@@ -153,7 +153,7 @@ __device__ __forceinline__ int64_t read_maybe_galois(const View3& v, const int64
   if (gal_idx == nullptr) return v.at(b, row, i);
   Global<int32_t>* idx = global(reinterpret_cast<const int32_t*>(gal_idx[b]));
   Global<int8_t>* sgn = global(reinterpret_cast<const int8_t*>(gal_sign[b]));
-  int64_t x = v.at(b, row, idx[i]);
+  int64_t x = canonicalize(v.at(b, row, idx[i]), twice_q);  // a word below 2q would turn negative
   if (sgn[i] == -1) x = -x;
   return canonicalize(shift_positive(x, twice_q), twice_q);
 }

@@ -76,6 +76,22 @@ def test_product_and_hoisted_rotation_match_composition(eng, offset):
         eng.fused_keyswitch = True
 
 
+@pytest.mark.parametrize("offset", [0, -2])
+def test_rotations_take_residues_below_twice_the_prime(eng, offset):
+    """Words in [q, 2q) stand for their residues, also where a rotation negates them."""
+
+    level = offset if offset >= 0 else eng.config.public_level_count + offset
+    q = torch.tensor(eng.config.moduli[level: eng.config.num_q_primes], dtype=torch.int64, device=eng.device)
+    x = components(eng, level)
+    a = Ciphertext(torch.stack([x, x.flip(0)]), level, eng.config.default_scale)
+    above = torch.arange(eng.config.N, device=eng.device) % 3 > 0
+    lazy = Ciphertext(a.data + q.unsqueeze(1) * above, level, a.scale)
+    assert torch.equal(eng.rotate_by_step(lazy, 1).data, eng.rotate_by_step(a, 1).data)
+    assert torch.equal(eng.rotate_by_steps(lazy, [1, 5, 1]).data, eng.rotate_by_steps(a, [1, 5, 1]).data)
+    one, lazy_one = (Ciphertext(c.data[:, 0].contiguous(), level, c.scale) for c in (a, lazy))
+    assert torch.equal(eng.rotate_hoisted(lazy_one, [1, 5]).data, eng.rotate_hoisted(one, [1, 5]).data)
+
+
 @pytest.mark.parametrize("log_n,chain", [(12, "slots8192-scale50-levels5-int64"),
                                          (13, "slots8192-scale30-levels9-int64"),
                                          (14, "slots8192-scale50-levels5-int64"),
