@@ -7,6 +7,7 @@ range, where the sums of products are largest."""
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
@@ -90,6 +91,16 @@ def test_rotations_take_residues_below_twice_the_prime(eng, offset):
     assert torch.equal(eng.rotate_by_steps(lazy, [1, 5, 1]).data, eng.rotate_by_steps(a, [1, 5, 1]).data)
     one, lazy_one = (Ciphertext(c.data[:, 0].contiguous(), level, c.scale) for c in (a, lazy))
     assert torch.equal(eng.rotate_hoisted(lazy_one, [1, 5]).data, eng.rotate_hoisted(one, [1, 5]).data)
+
+
+@pytest.mark.parametrize("offset", [0, -2])
+def test_device_decryption_matches_the_host_codec(eng, offset):
+    """On the two rows it decodes: a 60-bit one and the last scale prime's, of every kind."""
+
+    level = offset if offset >= 0 else eng.config.public_level_count + offset
+    ct = eng.encrypt(np.random.default_rng(level).uniform(-1, 1, (2, eng.config.slots)), level=level)
+    got, want = eng.decrypt_on_device(ct).cpu().numpy(), eng.decrypt(ct, crt_primes=2)
+    assert np.abs(got - want).max() < 1e-9 * 2.0 ** max(0, 40 - eng.config.scale_bits)
 
 
 @pytest.mark.parametrize("log_n,chain", [(12, "slots8192-scale50-levels5-int64"),
